@@ -137,6 +137,7 @@ struct rd_disk {
     int32_t *id = nullptr, *type = nullptr;
     double* m_ex = nullptr;
     float* m32 = nullptr;
+    uint32_t* mass_odd = nullptr;  // nonzero: a source mass outside the FP64 kernels' short sequences
     uint32_t* disk_of = nullptr;
     DiskInfo* info = nullptr;
     DiskCtl* ctl = nullptr;
@@ -167,8 +168,7 @@ struct rd_disk {
     uint32_t coll_table = 0;
     WorkItem* items_feat = nullptr;
     uint32_t n_items_feat = 0;
-    bool exact_lane = false;       // FP64 pair kernel: one sink per lane (see build_lists)
-    bool exact_small = false;      // FP64 pair kernel: 4-sink items (small disks, see build_lists)
+    uint32_t exact_sinks = 18;     // FP64 pair kernel: sinks per item, 1 for one per lane (see build_lists)
     bool lists_valid = false;
     double pairs_per_eval = 0.0;
 
@@ -285,6 +285,7 @@ void free_buffers(rd_disk* d)
     dev_free(d->id);
     dev_free(d->type);
     dev_free(d->m32);
+    dev_free(d->mass_odd);
     dev_free(d->disk_of);
     dev_free(d->errw);
     dev_free(d->info);
@@ -335,6 +336,7 @@ int alloc_buffers(rd_disk* d)
     if (int rc = dev_alloc(&d->id, n)) return rc;
     if (int rc = dev_alloc(&d->type, n)) return rc;
     if (int rc = dev_alloc(&d->m32, n)) return rc;
+    if (int rc = dev_alloc(&d->mass_odd, 1)) return rc;
     if (int rc = dev_alloc(&d->disk_of, n)) return rc;
     if (int rc = dev_alloc(&d->info, d->n_disk)) return rc;
     if (int rc = dev_alloc(&d->ctl, d->n_disk)) return rc;
@@ -490,24 +492,36 @@ int build_lists(rd_disk* d)
     double pairs = 0.0;
     const uint32_t S = d->tuning.sinks_per_lane;
     const uint32_t C = std::max<uint32_t>(kTile, d->tuning.chunk / kTile * kTile);
-    // FP64: one sink per lane when 256-sink items give >= 4 blocks per CU,
-    // else the term-parallel kernel on 16-sink items, or on 4-sink items when
-    // 16-sink items would be fewer than the CUs (same bits in every case)
+    // FP64: one sink per lane when 256-sink items give >= 4 blocks per CU, else
+    // the term-parallel kernel on items of kExactSinks (same bits in every case)
     if (d->precision == RD_PREC_FP64) {
-        size_t groups = 0, groups16 = 0;
-        for (auto& o : order)
-            for (int cls = 0; cls < 3; ++cls) {
-                uint32_t b[4];
-                class_bounds(d->hd[o.second], cls, b);
-                if (b[1] > b[0]) {
-                    groups += (b[1] - b[0] + kBlock - 1) / kBlock;
-                    groups16 += (b[1] - b[0] + kExactSinks - 1) / kExactSinks;
+        auto n_groups = [&](uint32_t group) {
+            size_t n = 0;
+            for (auto& o : order)
+                for (int cls = 0; cls < 3; ++cls) {
+                    uint32_t b[4];
+                    class_bounds(d->hd[o.second], cls, b);
+                    if (b[1] > b[0]) n += (b[1] - b[0] + group - 1) / group;
+                }
+            return n;
+        };
+        if (n_groups((uint32_t)kBlock) >= 4 * (size_t)d->n_cu) {
+            d->exact_sinks = 1;
+        } else {
+            size_t best = ~(size_t)0;   // sinks of the fullest CU
+            for (uint32_t q : kExactSinks) {
+                const size_t n = n_groups(q), per_cu = (n + d->n_cu - 1) / d->n_cu;
+                // more blocks than serve a CU well: one of 4 or 8 sinks, six of 12 (all
+                // it holds at once)
+                if (per_cu > (q < 12 ? 1u : (q == 12 ? 6u : ~0u))) continue;
+                if (per_cu * q < best || (per_cu * q == best && per_cu > 2)) {
+                    best = per_cu * q;
+                    d->exact_sinks = q;
                 }
             }
-        d->exact_lane = groups >= 4 * (size_t)d->n_cu;
-        d->exact_small = !d->exact_lane && groups16 < (size_t)d->n_cu;
+        }
     }
-    const uint32_t exact_group = d->exact_lane ? (uint32_t)kBlock : (d->exact_small ? kExactSinksSmall : kExactSinks);
+    const uint32_t exact_group = d->exact_sinks == 1 ? (uint32_t)kBlock : d->exact_sinks;
     const bool sym = d->precision == RD_PREC_MIXED && d->tuning.pair_mode == RD_PAIRS_SYMMETRIC;
     std::vector<std::pair<uint32_t, WorkItem>> sym_items;   // (tiles, item)
     d->sym_R = 1;
@@ -615,8 +629,8 @@ int build_lists(rd_disk* d)
     if (!items.empty())
         HIP_TRY(hipMemcpy(d->items_force, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
     const uint32_t maxgrid = std::max<uint32_t>(1, d->tuning.blocks_per_cu) * (uint32_t)d->n_cu;
-    // the exact kernel's blocks use 26 KB of LDS: 6 fit on a CU
-    const uint32_t grid_cap = d->precision == RD_PREC_FP64 && !d->exact_lane ? 6u * (uint32_t)d->n_cu : maxgrid;
+    // the term-parallel FP64 kernel's items are single-pass: a block each, up to 8 per CU
+    const uint32_t grid_cap = d->precision == RD_PREC_FP64 && d->exact_sinks != 1 ? 8u * (uint32_t)d->n_cu : maxgrid;
     d->grid_force = std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_force, grid_cap));
     d->grid_sym = std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_sym, maxgrid));
     const size_t need = max_chunks * 3 * (size_t)d->n_all;
@@ -628,7 +642,8 @@ int build_lists(rd_disk* d)
         HIP_TRY(hipMemsetAsync(d->part, 0, need * sizeof(double), d->stream));
     }
     HIP_TRY(hipMemcpy(d->info, d->h_info.data(), d->n_disk * sizeof(DiskInfo), hipMemcpyHostToDevice));
-    HIP_TRY(launch_set_sources(d->stream, d->n_all, d->mass, d->id, d->disk_of, d->info, d->m_ex, d->m32));
+    HIP_TRY(launch_set_sources(d->stream, d->n_all, d->mass, d->id, d->disk_of, d->info, d->m_ex, d->m32,
+                               d->mass_odd));
     HIP_TRY(hipStreamSynchronize(d->stream));
     d->lists_valid = true;
     d->generation++;
@@ -684,9 +699,8 @@ StageArgs make_args(rd_disk* d, int r, int adaptive, int err_all)
 hipError_t enqueue_force(rd_disk* d, const double* fx, const double* fy, const double* fz, uint32_t need)
 {
     if (d->precision == RD_PREC_FP64)
-        return launch_force_exact(d->stream, d->exact_lane ? 1 : (d->exact_small ? 2 : 0), d->items_force,
-                                  d->n_items_force, d->grid_force,
-                                  fx, fy, fz, d->m_ex, d->ctl, need, d->part, d->n_all);
+        return launch_force_exact(d->stream, d->exact_sinks, d->items_force, d->n_items_force, d->grid_force, fx, fy,
+                                  fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all);
     // mixed precision: FP32 slot totals, in float units of the same buffer
     float* part32 = reinterpret_cast<float*>(d->part);
     if (hipError_t e = launch_force_sym(d->stream, d->sym_R, d->sym_self, d->items_sym, d->n_items_sym, d->grid_sym,
@@ -715,12 +729,12 @@ hipError_t enqueue_attempt(rd_integrator* it, int commit_advance)
 {
     rd_disk* d = it->d;
     hipError_t e;
-    // FP64, one small gas-free disk (4-sink items: launches, not pairs, set
+    // FP64, one small gas-free disk (4- or 8-sink items: launches, not pairs, set
     // the time), fixed-step RK4: each stage is done by the summing lanes of
     // its FP64 pair pass (launch_force_exact_rk4), which hold every body's
     // complete sum; the same operations in the same order as pair pass + stage
     // kernel, one launch per stage instead of two
-    if (d->precision == RD_PREC_FP64 && !d->exact_lane && d->exact_small && d->n_disk == 1 &&
+    if (d->precision == RD_PREC_FP64 && (d->exact_sinks == 4 || d->exact_sinks == 8) && d->n_disk == 1 &&
         d->gas.on == kGasNone && it->method == RD_RK4 && !it->adaptive) {
         // the last stage also commits (k_commit's copy and time advance): its
         // summing lanes cover every body, and no pair term of that launch reads y_n
@@ -728,9 +742,9 @@ hipError_t enqueue_attempt(rd_integrator* it, int commit_advance)
             StageArgs a = make_args(d, r, it->adaptive, it->err_all);
             a.fuse_comb1 = r == 0;   // stage 0 forms stage 1 itself, as in the separate kernel
             if (r == last_stage(it)) a.commit = commit_advance;
-            if ((e = launch_force_exact_rk4(d->stream, r, d->items_force, d->n_items_force, d->grid_force,
-                                            a.fpos[0], a.fpos[1], a.fpos[2], d->m_ex, d->ctl,
-                                            r == 0 ? F_K0_FORCE : F_ACTIVE, a)) != hipSuccess)
+            if ((e = launch_force_exact_rk4(d->stream, d->exact_sinks, r, d->items_force, d->n_items_force,
+                                            d->grid_force, a.fpos[0], a.fpos[1], a.fpos[2], d->m_ex, d->mass_odd,
+                                            d->ctl, r == 0 ? F_K0_FORCE : F_ACTIVE, a)) != hipSuccess)
                 return e;
         }
         return hipSuccess;
@@ -1916,7 +1930,8 @@ int push_records(rd_disk* d, uint32_t k, const SparseView& sv)
     HIP_TRY(hipMemcpyAsync(d->ev_sids, ids.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, d->stream));
     HIP_TRY(hipMemcpyAsync(d->ev_srec, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice, d->stream));
     HIP_TRY(launch_scatter_bodies(d->stream, n, d->ev_sidx, d->ev_srec, d->ev_sids, body_arrays(d), d->id));
-    HIP_TRY(launch_set_sources(d->stream, d->n_all, d->mass, d->id, d->disk_of, d->info, d->m_ex, d->m32));
+    HIP_TRY(launch_set_sources(d->stream, d->n_all, d->mass, d->id, d->disk_of, d->info, d->m_ex, d->m32,
+                               d->mass_odd));
     HIP_TRY(hipStreamSynchronize(d->stream));
     return RD_OK;
 }

@@ -8,7 +8,7 @@
 //                    ka[r][3] (= acceleration at stage r)            r < 13
 //   pair partials  : part[(c*3 + comp) * n_all + i]: FP64 from the FP64 pair
 //                    kernel (one slot), FP32 chunk totals in mixed precision
-//   sources        : m_ex (FP64 mass, -1 if inactive), m32 (FP32 mass, 0 if
+//   sources        : m_ex (FP64 mass, -0 if inactive), m32 (FP32 mass, 0 if
 //                    inactive or summed in FP64)
 //   gas grid       : FARGO cells as 32-byte records (density, v_rad, v_theta, 0),
 //                    ring-major, then the n_rad + 1 ring radii
@@ -23,10 +23,20 @@ constexpr int kMaxStage = 13;
 constexpr int kBlock = 256;          // threads per block of the pair kernels
 constexpr int kBodyBlock = 64;       // per-body kernels: one wave per block, so small N still spreads over all CUs
 constexpr int kTile = 256;           // sources staged in LDS per tile
-// sinks per work item of the exact (FP64, reference-order) pair kernel
-constexpr uint32_t kExactSinks = 16;
-// ... and 4 for disks whose 16-sink items would leave CUs idle
-constexpr uint32_t kExactSinksSmall = 4;
+// Sinks per work item of the exact (FP64, reference-order) pair kernel.  While
+// the items are no more than the CUs: the smallest that keeps them so.  One
+// block per CU is bound by its serial sums, which a second block on the CU
+// slows down and more sinks per block do not (2047 bodies: 25.0 us with two
+// blocks of 4 sinks per CU, 20.4 with one of 8).  Beyond that, 12 or 18, whichever
+// gives the fullest CU fewer sinks, since it ends last (6000 bodies: 103 us with
+// two blocks of 12 on a CU, 117 with two of 18); when equal, 18 from three
+// blocks a CU on (16384 bodies: 470 us, 545 with 12), and past six blocks of 12,
+// all that a CU holds at once (20000 bodies: 725 us, 799 with 12).
+constexpr uint32_t kExactSinks[] = {4, 8, 12, 18};
+// high words of the r^2 the FP64 kernels' short root and division sequences
+// take: from 2^-200, up to 2^200
+constexpr uint32_t kExactR2Lo = (1023u - 200u) << 20;
+constexpr uint32_t kExactR2Span = 400u << 20;
 // bodies per block of the symmetric pair kernel (64 lanes x 4 sinks)
 constexpr uint32_t kSymBlockBodies = 256;
 // largest chunk (in blocks) of a symmetric-kernel work item; its reaction
@@ -145,16 +155,19 @@ struct BodyArrays {
 };
 
 // Launchers (kernels.hip).
-// lane: 0 term-parallel 16-sink items, 1 one sink per lane, 2 term-parallel 4-sink items
-hipError_t launch_force_exact(hipStream_t s, int lane, const WorkItem* items, uint32_t n_items, uint32_t grid,
+// sinks: sinks per item, 4, 8, 12 or 18 (term-parallel), or 1 for one sink per lane
+// (256-sink items)
+hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
-                              const DiskCtl* ctl, uint32_t need, double* part, uint32_t n_all);
-// The FP64 pair pass (4-sink items) of single-disk, gas-free, fixed-step RK4
-// stage r (0-3) with the stage combination done by the kernel's summing lanes
-// (no stage kernel, no partial-sum slot).
-hipError_t launch_force_exact_rk4(hipStream_t s, int r, const WorkItem* items, uint32_t n_items, uint32_t grid,
-                                  const double* x, const double* y, const double* z, const double* m_ex,
-                                  const DiskCtl* ctl, uint32_t need, const StageArgs& a);
+                              const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
+                              uint32_t n_all);
+// The FP64 pair pass (4- or 8-sink items) of single-disk, gas-free, fixed-step
+// RK4 stage r (0-3) with the stage combination done by the kernel's summing
+// lanes (no stage kernel, no partial-sum slot).
+hipError_t launch_force_exact_rk4(hipStream_t s, uint32_t sinks, int r, const WorkItem* items, uint32_t n_items,
+                                  uint32_t grid, const double* x, const double* y, const double* z,
+                                  const double* m_ex, const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need,
+                                  const StageArgs& a);
 hipError_t launch_force_mixed(hipStream_t s, int sinks_per_lane, const WorkItem* items, uint32_t n_items,
                               uint32_t grid, const double* x, const double* y, const double* z,
                               const float* m32, const DiskCtl* ctl, uint32_t need_mask, float* part,
@@ -211,6 +224,7 @@ hipError_t launch_gather_bodies(hipStream_t s, uint32_t n, const uint32_t* idx, 
 hipError_t launch_scatter_bodies(hipStream_t s, uint32_t n, const uint32_t* idx, const double* rec,
                                  const int32_t* ids, const BodyArrays& b, int32_t* id);
 hipError_t launch_set_sources(hipStream_t s, uint32_t n_all, const double* mass, const int32_t* id,
-                              const uint32_t* disk_of, const DiskInfo* info, double* m_ex, float* m32);
+                              const uint32_t* disk_of, const DiskInfo* info, double* m_ex, float* m32,
+                              uint32_t* mass_odd);
 
 }  // namespace rdamd

@@ -78,58 +78,132 @@ __host__ __device__ constexpr double rk4_c(int r) { return (r == 1 || r == 2) ? 
 // rounded separately (the reference builds -fmad=false).
 //
 // The sum per (sink, component) is a chain of FP64 adds in j order, so it
-// cannot be split; the pair terms feeding it can.  A block takes kS sinks
-// (16, or 4 for disks whose 16-sink items would not reach every CU) and has
-// five waves.  Waves 0-3 compute, for each LDS tile of kTile sources, the
-// kS x kTile terms (m_j / (d * d^2)) * dx (sqrt and divide are the costly
-// part) into LDS; 3 kS lanes of wave 4 -- one per (sink, component) -- add a
-// tile's terms in j order to their running sums.  Terms and sources are
-// double-buffered: wave 4 adds tile t - 1 while waves 0-3 compute tile t, one
-// barrier per tile, so a tile costs the longer of the two, not their sum.
-// Same terms, same order: the result is bit-identical to one lane summing
-// alone, for either kS, while the term work spreads over N / kS blocks instead
-// of N lanes.  Threads of sinks past the item's end (a disk's last item)
-// compute nothing.
-constexpr int kExactBlock = kBlock + 64;   // 4 term waves + 1 summing wave
+// cannot be split; the pair terms feeding it can.  A block takes kS sinks (4, 8
+// or 18, build_lists).  Its term waves compute, for each tile of kTile sources, the
+// kS x kTile terms (m_j / (d * d^2)) * dx (sqrt and divide are the costly part)
+// into LDS; the summing waves add a tile's terms in j order to their running
+// sums.  The term buffer is doubled: tile t - 1 is added while tile t is
+// computed, one barrier per tile, so a tile costs the longer of the two, not
+// their sum.  Same terms, same order: the result is bit-identical to one lane
+// summing alone, for every kS, while the term work spreads over N / kS blocks
+// instead of N lanes.
+//
+// The chain bounds the small shapes (cycle counters in the kernel: the summing
+// wave worked 80-90% of the time), so it decides how the terms are read.  A
+// wave issues an LDS read about every 15-22 cycles whatever its width, and a
+// dependent FP64 add takes 8: 8-byte reads, one per term and lane, ran the
+// chain at 25 cycles a term.
+//   4 or 8 sinks (latency-bound, idle VALU): 3 kS / 4 summing waves, one per
+//     component and 4 sinks.  A row of 16 lanes belongs to one sink and reads
+//     16 consecutive terms at once; each is broadcast to the row and added by
+//     v_fmac_f64 with row_newbcast (term * 1 + sum: the add's rounding), every
+//     lane of the row holding the same sum.  One LDS read per 16 terms.
+//   18 sinks (throughput-bound: a broadcast add per term would cost more
+//     than the term's share of a wave): one summing wave, a lane per (sink,
+//     component), reading two terms at a time.  Three term waves: a block of
+//     four waves puts one on each SIMD, and since consecutive blocks of a CU
+//     start on consecutive SIMDs, four blocks leave each SIMD with three term
+//     waves and a summing one.
+// Term rows are kRow doubles apart, 2 more than the tile: lanes of consecutive
+// rows then touch consecutive 16-byte banks in the two-term reads.
+//
+// A term thread takes one source of the tile against kT sinks.  Its source
+// comes from memory straight into registers, kAhead tiles early (every wave reads
+// the same few KB: L1 hits), so no source passes through LDS, whose traffic the
+// 18-sink shape would run into next.  The kT terms are
+// computed phase by phase (their chains of dependent FP64 operations, ~450
+// cycles each, interleave) with a single branch at the end for the rare pair
+// outside the short sequences' range.
+constexpr uint32_t exact_tile(uint32_t kS) { return kS >= 12 ? 32u : 128u; }
+constexpr uint32_t exact_term_waves(uint32_t kS) { return kS >= 12 ? 3u : 4u; }
+constexpr uint32_t exact_sum_waves(uint32_t kS) { return kS >= 12 ? 1u : 3u * kS / 4u; }
+constexpr int exact_block(uint32_t kS) { return 64 * (int)(exact_term_waves(kS) + exact_sum_waves(kS)); }
 
-// m / (sqrt(r2) * r2) for r2 and m in the range exact_scale_in_range accepts,
-// bit for bit what the IEEE square root and division give: the instruction
-// sequences the compiler emits for them (v_rsq_f64 and two Goldschmidt steps
-// for the root; v_rcp_f64, two Newton steps and a residual step for the
-// quotient) without their range handling, which does nothing in that range (no
-// operand is scaled by v_ldexp or v_div_scale, and v_div_fixup and the
-// zero/infinity test of the root return the computed value).  About a fifth of
-// a pair term's instructions.
-__device__ __forceinline__ bool exact_scale_in_range(double r2, double m)
+// sum += the row's 8 terms v of lanes 8 H .. 8 H + 7, in order (row: 16 lanes).
+// The leading s_nop keeps a register copy of v, should there be one, clear of
+// its DPP reads.
+template <int H>
+__device__ __forceinline__ void row_add8(double& sum, double v)
 {
-    return r2 >= 0x1p-200 && r2 <= 0x1p200 && m >= 0x1p-300 && m <= 0x1p300;
-}
-__device__ __forceinline__ double exact_scale_fast(double r2, double m)
-{
-    const double y = __builtin_amdgcn_rsq(r2);
-    double g = r2 * y, h = y * 0.5;
-    const double r = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, r, g);
-    double e = __builtin_fma(-g, g, r2);
-    h = __builtin_fma(h, r, h);
-    g = __builtin_fma(e, h, g);
-    e = __builtin_fma(-g, g, r2);
-    g = __builtin_fma(e, h, g);   // sqrt(r2)
-    const double den = g * r2;
-    double q = __builtin_amdgcn_rcp(den);
-    double t = __builtin_fma(-den, q, 1.0);
-    q = __builtin_fma(q, t, q);
-    t = __builtin_fma(-den, q, 1.0);
-    q = __builtin_fma(q, t, q);   // 1 / den
-    const double a = m * q;
-    const double rem = __builtin_fma(-den, a, m);
-    return __builtin_fma(rem, q, a);
+    const double one = 1.0;
+#define ROW_ADD(K) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"
+    if constexpr (H == 0)
+        asm volatile("s_nop 1\n\t" ROW_ADD(0) ROW_ADD(1) ROW_ADD(2) ROW_ADD(3) ROW_ADD(4) ROW_ADD(5) ROW_ADD(6)
+                         ROW_ADD(7)
+                     : "+v"(sum)
+                     : "v"(v), "v"(one));
+    else
+        asm volatile("s_nop 1\n\t" ROW_ADD(8) ROW_ADD(9) ROW_ADD(10) ROW_ADD(11) ROW_ADD(12) ROW_ADD(13) ROW_ADD(14)
+                         ROW_ADD(15)
+                     : "+v"(sum)
+                     : "v"(v), "v"(one));
+#undef ROW_ADD
 }
 
-// Single-disk classical RK4 stage R for body i, component q (defined with the
-// stage kernels below).
-template <int R, bool kFused>
-__device__ void stage_rk4_body(const StageArgs& a, uint32_t i, int q, bool in, double ps_fused);
+// m / (sqrt(r2) * r2) for r2 in [2^-200, 2^200) and m = 0 or |m| in [2^-300,
+// 2^300], bit for bit what the IEEE square root and division give: the
+// instruction sequences the compiler emits for them (v_rsq_f64 and two
+// Goldschmidt steps for the root; v_rcp_f64, two Newton steps and a residual
+// step for the quotient) without their range handling, which does nothing in
+// that range (no operand is scaled by v_ldexp or v_div_scale, and v_div_fixup
+// and the zero/infinity test of the root return the computed value).  About a
+// third of a pair term's instructions.  The range of r2 is tested on its high
+// word (one subtract, one compare); the masses' when they are set
+// (k_set_sources): *mass_odd is nonzero if some source is outside, and every
+// pair then takes the library's root and division.
+__device__ __forceinline__ bool exact_r2_in_range(double r2, uint32_t span)
+{
+    return (uint32_t)__double2hiint(r2) - kExactR2Lo < span;
+}
+template <uint32_t kT>
+__device__ __forceinline__ void exact_scale_fast(const double (&r2)[kT], double m, double (&sc)[kT])
+{
+    double g[kT], h[kT], e[kT], den[kT];
+#define EXACT_EACH _Pragma("unroll") for (uint32_t q = 0; q < kT; ++q)
+    EXACT_EACH h[q] = __builtin_amdgcn_rsq(r2[q]);
+    EXACT_EACH g[q] = r2[q] * h[q];
+    EXACT_EACH h[q] = h[q] * 0.5;
+    EXACT_EACH e[q] = __builtin_fma(-h[q], g[q], 0.5);
+    EXACT_EACH g[q] = __builtin_fma(g[q], e[q], g[q]);
+    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);
+    EXACT_EACH e[q] = __builtin_fma(-g[q], g[q], r2[q]);
+    EXACT_EACH g[q] = __builtin_fma(e[q], h[q], g[q]);
+    EXACT_EACH e[q] = __builtin_fma(-g[q], g[q], r2[q]);
+    EXACT_EACH g[q] = __builtin_fma(e[q], h[q], g[q]);   // sqrt(r2)
+    EXACT_EACH den[q] = g[q] * r2[q];
+    EXACT_EACH g[q] = __builtin_amdgcn_rcp(den[q]);
+    EXACT_EACH e[q] = __builtin_fma(-den[q], g[q], 1.0);
+    EXACT_EACH g[q] = __builtin_fma(g[q], e[q], g[q]);
+    EXACT_EACH e[q] = __builtin_fma(-den[q], g[q], 1.0);
+    EXACT_EACH g[q] = __builtin_fma(g[q], e[q], g[q]);   // 1 / den
+    EXACT_EACH h[q] = m * g[q];
+    EXACT_EACH e[q] = __builtin_fma(-den[q], h[q], m);
+    EXACT_EACH sc[q] = __builtin_fma(e[q], g[q], h[q]);
+#undef EXACT_EACH
+}
+// An inactive source's mass is -0 (k_set_sources; an active one's never is), and
+// so is padding's.  Its terms are then zeros of either sign, which leave the
+// running sum unchanged: it starts at +0 and round-to-nearest never makes it -0.
+// The scale of a pair outside the short sequences' range: 0 for the sink itself
+// and for an inactive or padding source.
+__device__ __forceinline__ double exact_scale_any(double r2, double m, bool self)
+{
+    if (self || (m == 0.0 && signbit(m))) return 0.0;
+    return m / (sqrt(r2) * r2);
+}
+
+// What the summing lane of (body i, component q) needs for RK4 stage R of a
+// single gas-free disk, loaded before the pair sums so that the loads overlap
+// them, and the stage itself (defined with the stage kernels below).
+struct Rk4Lane {
+    DiskCtl c;
+    double yy, vv, kk, k0v, k1v, k2v, k0a, k1a, k2a;
+    int id;
+};
+template <int R>
+__device__ void rk4_lane_load(const StageArgs& a, uint32_t i, int q, Rk4Lane& s);
+template <int R>
+__device__ void rk4_lane_finish(const StageArgs& a, uint32_t i, int q, const Rk4Lane& s, double ps);
 struct NoStage {};
 
 // FR < 0: each summing lane stores its sum in the partial-sum slot.  FR >= 0
@@ -142,123 +216,240 @@ template <uint32_t kS, int FR, typename SA>
 __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ items, uint32_t n_items,
                                                  const double* __restrict__ x, const double* __restrict__ y,
                                                  const double* __restrict__ z, const double* __restrict__ m_ex,
+                                                 const uint32_t* __restrict__ mass_odd,
                                                  const DiskCtl* __restrict__ ctl, uint32_t need,
                                                  double* __restrict__ part, uint32_t n_all, const SA& sa)
 {
-    constexpr uint32_t kLanesPerSink = kBlock / kS;              // term threads sharing one sink
-    // sources per tile: 32 for 16-sink items (two term buffers in 26 KB of
-    // LDS), one per term thread of a sink otherwise
-    constexpr uint32_t kTile = kS >= 16 ? 32u : kLanesPerSink;
-    constexpr uint32_t kT = kTile / kLanesPerSink;               // terms per thread per tile
-    static_assert(kS * kTile == kT * kBlock && kT >= 1 && 3 * kS <= 64 && kTile <= kBlock, "tile shape");
-    __shared__ double4 src[2][kTile];
-    __shared__ double term[2][3][kS][kTile + 1];   // +1: summing lanes read with an odd stride
-    const uint32_t tid = threadIdx.x;
-    const bool termer = tid < (uint32_t)kBlock;   // waves 0-3
-    const uint32_t g = tid / kLanesPerSink;   // term threads: sink of this thread's terms
-    const uint32_t k_lo = tid % kLanesPerSink;    //            its sources: k_lo + kLanesPerSink q, q < kT
-    const uint32_t sl = tid - (uint32_t)kBlock;   // wave 4: summing lane (sl < 3 kS)
-    const uint32_t sc_c = sl / kS % 3u;      //         component
-    const uint32_t sc_g = sl % kS;           //         sink
+    constexpr uint32_t kTile = exact_tile(kS);
+    constexpr uint32_t kTermers = 64 * exact_term_waves(kS);
+    constexpr uint32_t kGroups = kTermers / kTile;    // term threads per source of a tile
+    constexpr uint32_t kT = kS / kGroups;             // sinks per term thread
+    constexpr uint32_t kRow = kTile + 2;
+    constexpr bool kRowSum = exact_sum_waves(kS) >= 3;
+    // a 12-sink tile alone on its CU is shorter than a load's latency; two tiles
+    // ahead needs the loop twice in the code, which the 18-sink items' registers
+    // (5 blocks a CU) and the smallest disks' instruction fetch do not afford
+    constexpr uint32_t kAhead = kS == 12 ? 2 : 1;
+    static_assert(kGroups * kTile == kTermers && kT * kGroups == kS && kT >= 1, "tile shape");
+    static_assert(kRowSum ? kS % 4 == 0 && kTile % 16 == 0 : 3 * kS <= 64 && kTile == 32, "summing lanes");
+    __shared__ __align__(16) double term[2][3][kS][kRow];
+    // Roles: kTermers term threads, then the summing lanes.  With one summing
+    // wave to three term waves the blocks of a CU should sum on different SIMDs:
+    // the n-th block of the CU (its first wave's slot on its SIMD) takes the
+    // wave on SIMD n.  The hardware's own order mostly gives that, but one CU
+    // with two summing waves on a SIMD made the launch 548 instead of 482 us.
+    uint32_t tid = threadIdx.x;
+    uint32_t my_turn = 0;
+    if constexpr (!kRowSum) {
+        constexpr uint32_t kWaves = (uint32_t)exact_block(kS) / 64u;
+        __shared__ uint32_t place[kWaves];
+        const uint32_t wv = __builtin_amdgcn_readfirstlane(tid / 64u);
+        // HW_ID: wave slot in bits 0-3, SIMD in bits 4-5
+        if (tid % 64u == 0) place[wv] = __builtin_amdgcn_s_getreg((5 << 11) | (0 << 6) | 4);
+        __syncthreads();
+        my_turn = __builtin_amdgcn_readfirstlane(place[0]) & 15u;
+        uint32_t sum_wave = kWaves - 1;
+        for (uint32_t q = 0; q < kWaves; ++q)
+            if ((__builtin_amdgcn_readfirstlane(place[q]) >> 4) == (my_turn & 3u)) sum_wave = q;
+        const uint32_t role = wv == sum_wave ? kWaves - 1 : wv - (wv > sum_wave ? 1u : 0u);
+        tid = role * 64u + tid % 64u;
+    }
+    const bool termer = __builtin_amdgcn_readfirstlane(tid) < kTermers;
+    const uint32_t k = tid % kTile;           // term threads: their source of each tile
+    const uint32_t g0 = tid / kTile;          //               their sinks: g0 + kGroups q, q < kT
+    const uint32_t sl = tid - kTermers;       // summing lane
+    const uint32_t sc_c = kRowSum ? sl / (16u * kS) : sl / kS % 3u;      // its component
+    const uint32_t sc_g = kRowSum ? sl / 16u % kS : sl % kS;             // its sink
+    const uint32_t sc_k = kRowSum ? sl % 16u : 0u;                       // its term among 16
+    // The adds are the block's serial chain: they go first on their SIMD (not
+    // those of 8-sink items, whose six summing waves would keep the term waves
+    // waiting: 16.2 instead of 15.0 us at 1501 bodies).  The term waves of the
+    // blocks that share a CU take turns there, by tile: the oldest block would
+    // otherwise run at full speed, end first and leave the CU to ever fewer
+    // (16385 bodies: blocks ended between 259 and 538 us).
+    // Only while all blocks of the launch are resident: beyond, those that end
+    // early make room for the next.
+    const bool shared_cu = gridDim.x > 256u && gridDim.x <= (kS == 18 ? 1280u : 1536u);
+    if (!termer && kS != 8) __builtin_amdgcn_s_setprio(3);
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
         const WorkItem w = items[it];
-        if (!(ctl[w.disk].flags & need)) continue;
-        const uint32_t i = w.sink_lo + g;
-        const bool valid = termer && i < w.sink_hi;
-        const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
         const uint32_t si = w.sink_lo + sc_g;  // sink of a summing lane
-        const bool summer = !termer && sl < 3 * kS && si < w.sink_hi;
-        const uint32_t n_tiles = (w.src_hi - w.src_lo + kTile - 1) / kTile;
-        auto load_src = [&](uint32_t j) {
-            return j < w.src_hi ? make_double4(x[j], y[j], z[j], m_ex[j]) : make_double4(0.0, 0.0, 0.0, -1.0);
+        // the lane that stores the sum
+        const bool owner = !termer && (kRowSum ? sc_k == 0 : sl < 3 * kS) && si < w.sink_hi;
+        auto finish = [&](double sum) {
+            if constexpr (FR >= 0) {
+                Rk4Lane lane;
+                rk4_lane_load<FR>(sa, si, (int)sc_c, lane);
+                rk4_lane_finish<FR>(sa, si, (int)sc_c, lane, sum);
+            } else {
+                part[(size_t)(w.slot * 3 + sc_c) * n_all + si] = sum;
+            }
         };
-        double acc = 0.0;
-        // tile 0 into LDS, tile 1 into registers; the loop stages tile t + 1
-        // and loads tile t + 2 while tile t's terms are computed
-        double4 nxt = make_double4(0.0, 0.0, 0.0, -1.0);
-        if (tid < kTile) {
-            src[0][tid] = load_src(w.src_lo + tid);
-            nxt = load_src(w.src_lo + kTile + tid);
+        if (w.src_hi <= w.src_lo) {   // no sources: the sums are zero
+            if ((ctl[w.disk].flags & need) && owner) finish(0.0);
+            continue;
         }
-        __syncthreads();
-        for (uint32_t t = 0; t <= n_tiles; ++t) {
-            const uint32_t b = t & 1u;
-            if (termer) {
-                if (t < n_tiles) {
-                    const uint32_t t0 = w.src_lo + t * kTile;
-                    if (valid) {
+        // the item's first loads go out together with the control's.  Source
+        // loads are unconditional (the index is clamped, the mass of what lies
+        // past the end is -0): a guarded load is waited for where its branch ends
+        double xi[kT], yi[kT], zi[kT];
 #pragma unroll
-                        for (uint32_t q = 0; q < kT; ++q) {
-                            const uint32_t k = k_lo + kLanesPerSink * q;
-                            const double4 sj = src[b][k];
-                            const double dx = sj.x - xi;
-                            const double dy = sj.y - yi;
-                            const double dz = sj.z - zi;
-                            const double r2 = SQR(dx) + SQR(dy) + SQR(dz);
-                            const bool skip = sj.w < 0.0 || t0 + k == i;
-                            double sc;
-                            if constexpr (kS >= 16) {
-                                // throughput-bound (large disks): the short sequence, with
-                                // the library's for the rare pair outside its range
-                                sc = exact_scale_fast(r2, sj.w);
-                                if (!skip && !exact_scale_in_range(r2, sj.w)) sc = sj.w / (sqrt(r2) * r2);
-                            } else {
-                                // latency-bound (small disks): the branch would cost more
-                                // than the shorter sequence saves
-                                sc = sj.w / (sqrt(r2) * r2);
-                            }
-                            // a skipped pair (self, inactive or padding source) adds 0 * d,
-                            // a zero of either sign: the running sum starts at +0 and
-                            // round-to-nearest never makes it -0, so the sum is unchanged
-                            sc = skip ? 0.0 : sc;
-                            term[b][0][g][k] = sc * dx;
-                            term[b][1][g][k] = sc * dy;
-                            term[b][2][g][k] = sc * dz;
-                        }
+        for (uint32_t q = 0; q < kT; ++q) {
+            // sinks past the item's end repeat its last (their sums are not stored)
+            const uint32_t i = min(w.sink_lo + g0 + kGroups * q, w.sink_hi - 1u);
+            xi[q] = x[i];
+            yi[q] = y[i];
+            zi[q] = z[i];
+        }
+        auto load_src = [&](uint32_t j) {
+            const uint32_t jc = min(j, w.src_hi - 1u);
+            return make_double4(x[jc], y[jc], z[jc], m_ex[jc]);
+        };
+        double4 sj_even = load_src(w.src_lo + k), sj_odd = sj_even;
+        if constexpr (kAhead == 2) sj_odd = load_src(w.src_lo + k + kTile);
+        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
+        if (!(ctl[w.disk].flags & need)) continue;
+        const uint32_t n_src = w.src_hi - w.src_lo;
+        const uint32_t n_tiles = (n_src + kTile - 1) / kTile;
+        Rk4Lane lane;
+        if constexpr (FR >= 0)
+            if (owner) rk4_lane_load<FR>(sa, si, (int)sc_c, lane);
+        double acc = 0.0;
+        // the first cnt terms of the tile's row tr in order, rounded up to 32 or
+        // 8 (padding adds zeros)
+        auto chain = [&](const double* tr, uint32_t cnt) {
+            if constexpr (kRowSum) {
+                double v[kTile / 16];
+#pragma unroll
+                for (uint32_t q = 0; q < kTile / 16; ++q) v[q] = tr[16 * q + sc_k];
+                // 32 at a time: finer steps cost a branch each, coarser ones up to
+                // that many adds of padding
+#pragma unroll
+                for (uint32_t q = 0; q < kTile / 16; q += 2) {
+                    if (16 * q >= cnt) break;
+                    row_add8<0>(acc, v[q]);
+                    row_add8<1>(acc, v[q]);
+                    row_add8<0>(acc, v[q + 1]);
+                    row_add8<1>(acc, v[q + 1]);
+                }
+            } else {
+                // two sets of 8 terms, one being read while the other is added
+                double2 u[4], v[4];
+                auto read = [&](uint32_t k0, double2 (&r)[4]) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) r[k] = reinterpret_cast<const double2*>(tr + k0)[k];
+                };
+                auto add = [&](const double2 (&r)[4]) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        acc += r[k].x;
+                        acc += r[k].y;
                     }
-                    if (tid < kTile) {
-                        src[b ^ 1u][tid] = nxt;
-                        nxt = load_src(w.src_lo + (t + 2) * kTile + tid);
+                };
+                read(0, u);
+                read(8, v);
+                add(u);
+                if (cnt <= 8) return;
+                read(16, u);
+                add(v);
+                if (cnt <= 16) return;
+                read(24, v);
+                add(u);
+                if (cnt <= 24) return;
+                add(v);
+            }
+        };
+        // one tile: its terms into term[b] from the thread's source sj, which is
+        // reloaded for kAhead tiles later as soon as the offsets are formed; and
+        // the sums of the tile before, from term[b ^ 1]
+        auto tile = [&](uint32_t t, uint32_t b, double4& sj) {
+            if (termer) {
+                if (!kRowSum && shared_cu) switch ((t + my_turn) & 3u) {
+                    case 0: __builtin_amdgcn_s_setprio(0); break;
+                    case 1: __builtin_amdgcn_s_setprio(1); break;
+                    default: __builtin_amdgcn_s_setprio(2);
+                    }
+                if (t < n_tiles) {
+                    const uint32_t j = w.src_lo + t * kTile + k;
+                    const double m = j < w.src_hi ? sj.w : -0.0;
+                    double dx[kT], dy[kT], dz[kT], r2[kT], sc[kT];
+                    bool out = false;
+#pragma unroll
+                    for (uint32_t q = 0; q < kT; ++q) {
+                        dx[q] = sj.x - xi[q];
+                        dy[q] = sj.y - yi[q];
+                        dz[q] = sj.z - zi[q];
+                    }
+                    sj = load_src(j + kAhead * kTile);
+#pragma unroll
+                    for (uint32_t q = 0; q < kT; ++q) {
+                        r2[q] = SQR(dx[q]) + SQR(dy[q]) + SQR(dz[q]);
+                        out |= !exact_r2_in_range(r2[q], r2_span);
+                    }
+                    exact_scale_fast<kT>(r2, m, sc);
+                    if (out) {
+#pragma unroll
+                        for (uint32_t q = 0; q < kT; ++q)
+                            if (!exact_r2_in_range(r2[q], r2_span))
+                                sc[q] = exact_scale_any(r2[q], m, j == w.sink_lo + g0 + kGroups * q);
+                    }
+#pragma unroll
+                    for (uint32_t q = 0; q < kT; ++q) {
+                        const uint32_t g = g0 + kGroups * q;
+                        term[b][0][g][k] = sc[q] * dx[q];
+                        term[b][1][g][k] = sc[q] * dy[q];
+                        term[b][2][g][k] = sc[q] * dz[q];
                     }
                 }
-            } else if (t > 0 && summer) {
-                const double* tr = &term[b ^ 1u][sc_c][sc_g][0];
-#pragma unroll
-                for (uint32_t k = 0; k < kTile; ++k) acc += tr[k];
+            } else if (t > 0 && (kRowSum || sl < 3 * kS)) {
+                chain(&term[b ^ 1u][sc_c][sc_g][0], min(kTile, n_src - (t - 1) * kTile));
             }
             __syncthreads();
-        }
-        if constexpr (FR >= 0) {
-            if (summer) stage_rk4_body<FR, true>(sa, si, (int)sc_c, true, acc);
+        };
+        if constexpr (kAhead == 1) {
+            for (uint32_t t = 0; t <= n_tiles; ++t) tile(t, t & 1u, sj_even);
         } else {
-            if (summer) part[(size_t)(w.slot * 3 + sc_c) * n_all + si] = acc;
+            for (uint32_t t = 0; t <= n_tiles; t += 2) {
+                tile(t, 0u, sj_even);
+                if (t < n_tiles) tile(t + 1, 1u, sj_odd);
+            }
+        }
+        if (owner) {
+            if constexpr (FR >= 0) rk4_lane_finish<FR>(sa, si, (int)sc_c, lane, acc);
+            else finish(acc);
         }
     }
 }
 
+// Registers for 6 blocks of 12 and 5 of 18 sinks on a CU: with one less each, more
+// launches leave a few items for a second round (18432 bodies, 1025 items of 18:
+// 740 us, 664 with 5 a CU)
 template <uint32_t kS>
-__global__ __launch_bounds__(kExactBlock) void k_force_exact(const WorkItem* __restrict__ items, uint32_t n_items,
+__global__ __launch_bounds__(exact_block(kS)) __attribute__((amdgpu_waves_per_eu(kS == 12 ? 6 : (kS == 18 ? 5 : 1))))
+void k_force_exact(const WorkItem* __restrict__ items, uint32_t n_items,
                                                              const double* __restrict__ x,
                                                              const double* __restrict__ y,
                                                              const double* __restrict__ z,
                                                              const double* __restrict__ m_ex,
+                                                             const uint32_t* __restrict__ mass_odd,
                                                              const DiskCtl* __restrict__ ctl, uint32_t need,
                                                              double* __restrict__ part, uint32_t n_all)
 {
-    force_exact_body<kS, -1>(items, n_items, x, y, z, m_ex, ctl, need, part, n_all, NoStage{});
+    force_exact_body<kS, -1>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, part, n_all, NoStage{});
 }
 
 // The FP64 pair pass of RK4 stage R with the stage itself done by the summing lanes.
 template <uint32_t kS, int R>
-__global__ __launch_bounds__(kExactBlock) void k_force_exact_rk4(const WorkItem* __restrict__ items,
+__global__ __launch_bounds__(exact_block(kS)) void k_force_exact_rk4(const WorkItem* __restrict__ items,
                                                                  uint32_t n_items, const double* __restrict__ x,
                                                                  const double* __restrict__ y,
                                                                  const double* __restrict__ z,
                                                                  const double* __restrict__ m_ex,
+                                                                 const uint32_t* __restrict__ mass_odd,
                                                                  const DiskCtl* __restrict__ ctl, uint32_t need,
                                                                  StageArgs sa)
 {
-    force_exact_body<kS, R>(items, n_items, x, y, z, m_ex, ctl, need, nullptr, sa.n_all, sa);
+    force_exact_body<kS, R>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, nullptr, sa.n_all, sa);
 }
 
 // The same sum with one sink per lane, each lane adding its terms in j order
@@ -270,6 +461,7 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
                                                              const double* __restrict__ y,
                                                              const double* __restrict__ z,
                                                              const double* __restrict__ m_ex,
+                                                             const uint32_t* __restrict__ mass_odd,
                                                              const DiskCtl* __restrict__ ctl, uint32_t need,
                                                              double* __restrict__ part, uint32_t n_all)
 {
@@ -278,6 +470,7 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
         const WorkItem w = items[it];
         if (!(ctl[w.disk].flags & need)) continue;
+        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
         const uint32_t i = w.sink_lo + tid;
         const bool valid = i < w.sink_hi;
         const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
@@ -290,13 +483,14 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
             const uint32_t nt = min((uint32_t)kTile, w.src_hi - t0);
             for (uint32_t k = 0; k < nt; ++k) {
                 const double4 sj = tile[k];
-                if (sj.w < 0.0 || t0 + k == i) continue;
                 const double dx = sj.x - xi;
                 const double dy = sj.y - yi;
                 const double dz = sj.z - zi;
                 const double r2 = SQR(dx) + SQR(dy) + SQR(dz);
-                double sc = exact_scale_fast(r2, sj.w);
-                if (!exact_scale_in_range(r2, sj.w)) sc = sj.w / (sqrt(r2) * r2);
+                double one_sc[1];
+                exact_scale_fast<1>({r2}, sj.w, one_sc);
+                double sc = one_sc[0];
+                if (!exact_r2_in_range(r2, r2_span)) sc = exact_scale_any(r2, sj.w, t0 + k == i);
                 ax += sc * dx;
                 ay += sc * dy;
                 az += sc * dz;
@@ -866,39 +1060,43 @@ hipError_t launch_force_sym(hipStream_t st, uint32_t R, bool self, const WorkIte
 
 size_t force_sym_lds_bytes(uint32_t R) { return sym_lds_bytes(R); }
 
-hipError_t launch_force_exact(hipStream_t st, int lane, const WorkItem* items, uint32_t n_items, uint32_t grid,
+hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
-                              const DiskCtl* ctl, uint32_t need, double* part, uint32_t n_all)
+                              const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
+                              uint32_t n_all)
 {
     if (n_items == 0) return hipSuccess;
-    if (lane == 1)
-        hipLaunchKernelGGL(k_force_exact_lane, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m_ex, ctl,
-                           need, part, n_all);
-    else if (lane == 2)
-        hipLaunchKernelGGL(k_force_exact<kExactSinksSmall>, dim3(grid), dim3(kExactBlock), 0, st, items, n_items, x,
-                           y, z, m_ex, ctl, need, part, n_all);
-    else
-        hipLaunchKernelGGL(k_force_exact<kExactSinks>, dim3(grid), dim3(kExactBlock), 0, st, items, n_items, x, y,
-                           z, m_ex, ctl, need, part, n_all);
+#define EXACT_LAUNCH(KERNEL, BLOCK, ...)                                                                        \
+    hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(BLOCK), 0, st, items, n_items, x, y, z, m_ex, mass_odd, ctl, need, \
+                       __VA_ARGS__)
+    switch (sinks) {
+    case 1: EXACT_LAUNCH(k_force_exact_lane, kBlock, part, n_all); break;
+    case 4: EXACT_LAUNCH(k_force_exact<4>, exact_block(4), part, n_all); break;
+    case 8: EXACT_LAUNCH(k_force_exact<8>, exact_block(8), part, n_all); break;
+    case 12: EXACT_LAUNCH(k_force_exact<12>, exact_block(12), part, n_all); break;
+    case 18: EXACT_LAUNCH(k_force_exact<18>, exact_block(18), part, n_all); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_force_exact_rk4(hipStream_t st, int r, const WorkItem* items, uint32_t n_items, uint32_t grid,
-                                  const double* x, const double* y, const double* z, const double* m_ex,
-                                  const DiskCtl* ctl, uint32_t need, const StageArgs& a)
+hipError_t launch_force_exact_rk4(hipStream_t st, uint32_t sinks, int r, const WorkItem* items, uint32_t n_items,
+                                  uint32_t grid, const double* x, const double* y, const double* z,
+                                  const double* m_ex, const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need,
+                                  const StageArgs& a)
 {
     if (n_items == 0) return hipSuccess;
-#define EXACT_RK4(R)                                                                                            \
-    hipLaunchKernelGGL((k_force_exact_rk4<kExactSinksSmall, R>), dim3(grid), dim3(kExactBlock), 0, st, items,   \
-                       n_items, x, y, z, m_ex, ctl, need, a)
+    if (r < 0 || r > 3 || (sinks != 4 && sinks != 8)) return hipErrorInvalidValue;
+#define EXACT_RK4(R)                                                                            \
+    case R:                                                                                     \
+        if (sinks == 4) EXACT_LAUNCH((k_force_exact_rk4<4, R>), exact_block(4), a);             \
+        else EXACT_LAUNCH((k_force_exact_rk4<8, R>), exact_block(8), a);                        \
+        break;
     switch (r) {
-    case 0: EXACT_RK4(0); break;
-    case 1: EXACT_RK4(1); break;
-    case 2: EXACT_RK4(2); break;
-    case 3: EXACT_RK4(3); break;
-    default: return hipErrorInvalidValue;
+        EXACT_RK4(0) EXACT_RK4(1) EXACT_RK4(2) EXACT_RK4(3)
     }
 #undef EXACT_RK4
+#undef EXACT_LAUNCH
     return hipGetLastError();
 }
 
@@ -1459,17 +1657,73 @@ __global__ __launch_bounds__(kBodyBlock) void k_stage_rk8(StageArgs a)
     if constexpr (R == 12) error_reduce(a, valid, d, e);
 }
 
-// Classical RK4 stage R over a single disk, for body i and component q.
-// kFused: called by the FP64 pair kernel's summing lane with the body's
-// complete FP64 sum, for a body of a gas-free disk (fixed step: no stage 4),
-// and returns early where the stage does not apply; stores go to the arrays.
-// Otherwise a stage-kernel thread: the sums come from the partial-sum slots,
-// and a thread past the end or outside the attempt stores into its discard
-// slot, so no branch sits between the loads and the stores.
-template <int R, bool kFused>
-__device__ __forceinline__ void stage_rk4_body(const StageArgs& a, uint32_t i, int q, bool in, double ps_fused)
+// Classical RK4 stage R of a fixed-step run on a single gas-free disk, done by
+// the FP64 pair kernel's summing lane of (body i, component q): the loads, and
+// the stage from them and the body's complete sum ps.  The same operations as
+// the stage kernel's (stage_rk4_one); returns early where the stage does not
+// apply.  With gas the drag code would take the registers the pair pass needs.
+template <int R>
+__device__ __forceinline__ void rk4_lane_load(const StageArgs& a, uint32_t i, int q, Rk4Lane& s)
 {
-    static_assert(!kFused || R <= 3, "fused stages are the fixed-step ones");
+    static_assert(R >= 0 && R <= 3, "fused stages are the fixed-step ones");
+    s.c = a.ctl[0];
+    s.id = a.id[i];
+    s.yy = a.pos[q][i];
+    s.vv = a.vel[q][i];
+    s.kk = kv_of(a, R, q)[i];
+    if constexpr (R == 3) {
+        s.k0v = kv_of(a, 0, q)[i]; s.k1v = kv_of(a, 1, q)[i]; s.k2v = kv_of(a, 2, q)[i];
+        s.k0a = ka_of(a, 0, q)[i]; s.k1a = ka_of(a, 1, q)[i]; s.k2a = ka_of(a, 2, q)[i];
+    }
+}
+template <int R>
+__device__ __forceinline__ void rk4_lane_finish(const StageArgs& a, uint32_t i, int q, const Rk4Lane& s, double ps)
+{
+    const DiskCtl& c = s.c;
+    if (!(c.flags & (R == 0 ? F_NEED_K0 : F_ACTIVE))) return;
+    const double h = c.h;
+    // stage_accel without the drag: the reference's sum, zero for an inactive sink
+    const double kRa = s.id > 0 ? ps : 0.0;
+    ka_w(a, R, q)[i] = kRa;
+    if constexpr (R == 0) {
+        if (a.fuse_comb1) {   // k_comb1's stage-1 combination, same operands
+            const double fac = rk4_a(1) * h;
+            a.npos[q][i] = s.yy + fac * s.vv;
+            kv_w(a, 1, q)[i] = s.vv + fac * kRa;
+        }
+    } else if constexpr (R == 1 || R == 2) {
+        const double fac = rk4_a(R + 1) * h;
+        a.npos[q][i] = s.yy + fac * s.kk;
+        kv_w(a, R + 1, q)[i] = s.vv + fac * kRa;
+    } else {
+        // y + b0 (f1 + f4) + b1 (f2 + f3), b pre-multiplied by h (int_rungekutta4.cu:50-60, 150-171)
+        const double b0 = (1.0 / 6.0) * h, b1 = (1.0 / 3.0) * h;
+        const double yo = s.yy + b0 * (s.k0v + s.kk) + b1 * (s.k1v + s.k2v);
+        const double vo = s.vv + b0 * (s.k0a + kRa) + b1 * (s.k1a + s.k2a);
+        // k_commit's work for a committed attempt: y_n <- y_{n+1} in place (this
+        // lane alone reads body i's y_n, and no pair term of the launch does)
+        // and t += h (no stage of a gas-free fused step reads t)
+        if (a.commit >= 0 && (c.flags & F_COMMIT)) {
+            const_cast<double*>(a.pos[q])[i] = yo;
+            const_cast<double*>(a.vel[q])[i] = vo;
+            if (a.commit == 1 && q == 0 && i == a.info0.off) const_cast<DiskCtl*>(a.ctl)[0].t = c.t + c.h;
+            return;
+        }
+        a.out[q][i] = yo;
+        a.out[3 + q][i] = vo;
+    }
+}
+
+// Classical RK4 stage R over a single disk.  The sums come from the
+// partial-sum slots, and a thread past the end or outside the attempt stores
+// into its discard slot, so no branch sits between the loads and the stores.
+template <int R>
+__device__ __forceinline__ void stage_rk4_one(const StageArgs& a)
+{
+    const uint32_t i0 = blockIdx.x * kBodyBlock + threadIdx.x;
+    const bool in = i0 < a.n_all;
+    const uint32_t i = in ? i0 : a.n_all - 1;
+    const int q = blockIdx.y;
     const DiskInfo& di = a.info0;
     const DiskCtl c = a.ctl[0];
     if constexpr (R == 0)
@@ -1486,33 +1740,14 @@ __device__ __forceinline__ void stage_rk4_body(const StageArgs& a, uint32_t i, i
         k3a = ka_of(a, 3, q)[i];
     }
     double ps, b;
-    if constexpr (kFused) {
-        ps = ps_fused;   // the FP64 kernel's one slot: no prefix in FP64 mode
-        b = 0.0;
-    } else {
-        one_disk_sums(a, i, q, ps, b);
-    }
+    one_disk_sums(a, i, q, ps, b);
     const bool valid = in && (c.flags & (R == 0 ? F_NEED_K0 : F_ACTIVE)) != 0;
-    if constexpr (kFused)
-        if (!valid) return;
     const double h = c.h;
     const double t = c.t + rk4_c(R) * h;
     const double* vR[3] = {kv_of(a, R, 0), kv_of(a, R, 1), kv_of(a, R, 2)};
-    // the fused form runs only without gas (its drag code would take the
-    // registers the pair pass needs): the reference's sum, zero for an
-    // inactive sink (stage_accel without the drag)
-    double kRa;
-    if constexpr (kFused) {
-        (void)vR;
-        (void)t;
-        kRa = a.id[i] > 0 ? ps : 0.0;
-    } else {
-        kRa = stage_accel(a, i, q, di, t, b, ps, a.fpos, vR);
-    }
-    auto at = [&](double* p) -> double* {
-        if constexpr (kFused) return p + i;
-        else return valid ? p + i : a.trash + (size_t)q * kBodyBlock + threadIdx.x;
-    };
+    const double kRa = stage_accel(a, i, q, di, t, b, ps, a.fpos, vR);
+    double* const trash = a.trash + (size_t)q * kBodyBlock + threadIdx.x;
+    auto at = [&](double* p) { return valid ? p + i : trash; };
     *at(ka_w(a, R, q)) = kRa;
     if constexpr (R == 0) {
         if (a.fuse_comb1) {   // k_comb1's stage-1 combination, same operands
@@ -1529,17 +1764,6 @@ __device__ __forceinline__ void stage_rk4_body(const StageArgs& a, uint32_t i, i
         const double b0 = (1.0 / 6.0) * h, b1 = (1.0 / 3.0) * h;
         const double yo = yy + b0 * (k0v + kk) + b1 * (k1v + k2v);
         const double vo = vv + b0 * (k0a + kRa) + b1 * (k1a + k2a);
-        if constexpr (kFused) {
-            // k_commit's work for a committed attempt: y_n <- y_{n+1} in place (this
-            // lane alone reads body i's y_n, and no pair term of the launch does)
-            // and t += h (no stage of a gas-free fused step reads t)
-            if (a.commit >= 0 && (c.flags & F_COMMIT)) {
-                const_cast<double*>(a.pos[q])[i] = yo;
-                const_cast<double*>(a.vel[q])[i] = vo;
-                if (a.commit == 1 && q == 0 && i == di.off) const_cast<DiskCtl*>(a.ctl)[0].t = c.t + c.h;
-                return;
-            }
-        }
         *at(a.out[q]) = yo;
         *at(a.out[3 + q]) = vo;
         if (a.adaptive) {
@@ -1552,14 +1776,6 @@ __device__ __forceinline__ void stage_rk4_body(const StageArgs& a, uint32_t i, i
         if (valid && (a.err_all || li < di.err_hi)) e = fmax(fabs(k3v - kk), fabs(k3a - kRa));   // |f4 - f5|
         error_store_wave(a, valid, e);
     }
-}
-
-template <int R>
-__device__ __forceinline__ void stage_rk4_one(const StageArgs& a)
-{
-    const uint32_t i0 = blockIdx.x * kBodyBlock + threadIdx.x;
-    const bool in = i0 < a.n_all;
-    stage_rk4_body<R, false>(a, in ? i0 : a.n_all - 1, (int)blockIdx.y, in, 0.0);
 }
 
 // Classical RK4 stage kernel (int_rungekutta4.cu:37-73, 130-247).
@@ -1911,27 +2127,35 @@ hipError_t launch_var4_join(hipStream_t st, uint32_t n, const double* const a[3]
 }
 
 // ---------------------------------------------------------------------------
-// Sources: FP64 mass with -1 for inactive bodies, FP32 mass with 0 for
-// inactive bodies and for the FP64 prefix.
+// Sources: FP64 mass with -0 for inactive bodies, FP32 mass with 0 for
+// inactive bodies and for the FP64 prefix.  *mass_odd (cleared by the caller)
+// becomes 1 if a source that pulls has a mass the FP64 pair kernels' short
+// sequences do not take.  + 0.0: a mass of -0 becomes +0 (-0 marks a source that
+// is skipped).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_set_sources(uint32_t n_all, const double* mass, const int32_t* id,
                                                         const uint32_t* disk_of, const DiskInfo* info, double* m_ex,
-                                                        float* m32)
+                                                        float* m32, uint32_t* mass_odd)
 {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n_all) return;
     const DiskInfo di = info[disk_of[i]];
     const bool act = id[i] > 0;
-    m_ex[i] = act ? mass[i] : -1.0;
+    const double m = mass[i] + 0.0;
+    m_ex[i] = act ? m : -0.0;
+    if (act && !(m == 0.0 || (fabs(m) >= 0x1p-300 && fabs(m) <= 0x1p300))) *mass_odd = 1u;   // NaN too
     m32[i] = (act && (i - di.off) >= di.n_fp64) ? (float)mass[i] : 0.0f;
 }
 
 hipError_t launch_set_sources(hipStream_t st, uint32_t n_all, const double* mass, const int32_t* id,
-                              const uint32_t* disk_of, const DiskInfo* info, double* m_ex, float* m32)
+                              const uint32_t* disk_of, const DiskInfo* info, double* m_ex, float* m32,
+                              uint32_t* mass_odd)
 {
     const uint32_t grid = (n_all + kBlock - 1) / kBlock;
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_set_sources, dim3(grid), dim3(kBlock), 0, st, n_all, mass, id, disk_of, info, m_ex, m32);
+    if (hipError_t e = hipMemsetAsync(mass_odd, 0, sizeof(uint32_t), st)) return e;
+    hipLaunchKernelGGL(k_set_sources, dim3(grid), dim3(kBlock), 0, st, n_all, mass, id, disk_of, info, m_ex, m32,
+                       mass_odd);
     return hipGetLastError();
 }
 
