@@ -299,7 +299,7 @@ int rd_calc_integral(rd_disk* d, uint32_t k, rd_integral* out);
  * allocate device memory (code that must not call hipMalloc, such as tight
  * serving or monitoring loops and harnesses that forbid it).  Same kernels and
  * results, bit for bit; the partial sums live in a file-scope device array of
- * 2^21 doubles (16 MiB per GPU, held until the process ends) instead of a
+ * 2^19 doubles (4 MiB per GPU, held until the process ends) instead of a
  * buffer the disk allocates on first use, so it takes disks of at most 65536
  * bodies (RD_EINVAL above that).  Calls that overlap on one GPU share that
  * array and race. */

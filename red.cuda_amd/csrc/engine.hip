@@ -2341,8 +2341,10 @@ namespace {
 int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, double* red, rd_integral* out)
 {
     const HostDisk& h = d->hd[k];
+    // the masses' range flag belongs to the work lists' sources
+    if (int rc = ensure_lists(d)) return rc;
     HIP_TRY(launch_integral(d->stream, h.off, h.off + h.n, d->x, d->y, d->z, d->vx, d->vy, d->vz, d->mass, d->id,
-                            scr, len, red, red + 11));
+                            d->mass_odd, scr, len, red, red + 11));
     double o[12];
     HIP_TRY(hipMemcpyAsync(o, red, sizeof(o), hipMemcpyDeviceToHost, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
@@ -2350,23 +2352,17 @@ int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, double* red, 
     out->R = rd_var4{o[1] / M0, o[2] / M0, o[3] / M0, 0.0};
     out->V = rd_var4{o[4] / M0, o[5] / M0, o[6] / M0, 0.0};
     out->C = rd_var4{o[7], o[8], o[9], 0.0};
-    out->E = o[10] / 2.0 - o[11] / 2.0;
+    out->E = o[10] / 2.0 - o[11];
     return RD_OK;
 }
 
-// doubles of partial sums launch_integral needs for n bodies
-size_t integral_scratch(uint32_t n)
-{
-    const size_t nch = (n + 2047) / 2048;
-    return std::max<size_t>(11 * (size_t)n, nch * n);
-}
-
 // Scratch of rd_calc_integral_noalloc: a file-scope device array, so the call
-// allocates nothing.  Every GPU the library runs on holds its own copy (16 MiB
+// allocates nothing.  Every GPU the library runs on holds its own copy (4 MiB
 // of partial sums plus 16 doubles of results) until the process ends; calls on
 // one GPU share it, so calls that overlap on one GPU race.  Every value a call
 // reads was written by the same call: nothing needs clearing.
-constexpr size_t kNoAllocScratch = (size_t)1 << 21;
+constexpr uint32_t kNoAllocBodies = 65536;
+constexpr size_t kNoAllocScratch = (size_t)1 << 19;
 static __device__ __align__(256) double scratch[kNoAllocScratch + 16];
 
 constexpr int kMaxDevices = 64;
@@ -2413,10 +2409,10 @@ int rd_calc_integral_noalloc(rd_disk* d, uint32_t k, rd_integral* out)
     DeviceScope dev_scope(d ? d->device : -1);
     if (!d || !out || k >= d->n_disk) return fail(RD_EINVAL, "bad argument");
     const size_t need = integral_scratch(d->hd[k].n);
-    if (need > kNoAllocScratch)
+    if (d->hd[k].n > kNoAllocBodies || need > kNoAllocScratch)
         return fail(RD_EINVAL, "rd_calc_integral_noalloc: disk of " + std::to_string(d->hd[k].n) +
-                                   " bodies needs " + std::to_string(need) + " doubles of scratch, more than the " +
-                                   std::to_string(kNoAllocScratch) + " it holds (at most 65536 bodies)");
+                                   " bodies, more than its scratch is sized for (at most " +
+                                   std::to_string(kNoAllocBodies) + " bodies)");
     double* scr = nullptr;
     if (int rc = scratch_on(d->device, &scr)) return rc;
     return integral_with(d, k, scr, kNoAllocScratch, scr + kNoAllocScratch, out);

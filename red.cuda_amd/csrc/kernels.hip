@@ -181,6 +181,34 @@ __device__ __forceinline__ void exact_scale_fast(const double (&r2)[kT], double 
     EXACT_EACH sc[q] = __builtin_fma(e[q], g[q], h[q]);
 #undef EXACT_EACH
 }
+// m / sqrt(r2), the same sequences and range (r2 as above; |m| in [2^-600, 2^600]
+// or 0).
+template <uint32_t kT>
+__device__ __forceinline__ void exact_ratio_fast(const double (&r2)[kT], const double (&m)[kT], double (&v)[kT])
+{
+    double g[kT], h[kT], e[kT];
+#define EXACT_EACH _Pragma("unroll") for (uint32_t q = 0; q < kT; ++q)
+    EXACT_EACH h[q] = __builtin_amdgcn_rsq(r2[q]);
+    EXACT_EACH g[q] = r2[q] * h[q];
+    EXACT_EACH h[q] = h[q] * 0.5;
+    EXACT_EACH e[q] = __builtin_fma(-h[q], g[q], 0.5);
+    EXACT_EACH g[q] = __builtin_fma(g[q], e[q], g[q]);
+    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);
+    EXACT_EACH e[q] = __builtin_fma(-g[q], g[q], r2[q]);
+    EXACT_EACH g[q] = __builtin_fma(e[q], h[q], g[q]);
+    EXACT_EACH e[q] = __builtin_fma(-g[q], g[q], r2[q]);
+    EXACT_EACH g[q] = __builtin_fma(e[q], h[q], g[q]);   // sqrt(r2)
+    EXACT_EACH h[q] = __builtin_amdgcn_rcp(g[q]);
+    EXACT_EACH e[q] = __builtin_fma(-g[q], h[q], 1.0);
+    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);
+    EXACT_EACH e[q] = __builtin_fma(-g[q], h[q], 1.0);
+    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);   // 1 / sqrt(r2)
+    EXACT_EACH v[q] = m[q] * h[q];
+    EXACT_EACH e[q] = __builtin_fma(-g[q], v[q], m[q]);
+    EXACT_EACH v[q] = __builtin_fma(e[q], h[q], v[q]);
+#undef EXACT_EACH
+}
+
 // An inactive source's mass is -0 (k_set_sources; an active one's never is), and
 // so is padding's.  Its terms are then zeros of either sign, which leave the
 // running sum unchanged: it starts at +0 and round-to-nearest never makes it -0.
@@ -2371,109 +2399,159 @@ hipError_t launch_ejection(hipStream_t st, uint32_t n_all, const double* x, cons
 }
 
 // ---------------------------------------------------------------------------
-// Integrals (tools.cpp:367-410, 545-700) in FP64 with Neumaier summation.
+// Integrals (tools.cpp:367-410, 545-700) in FP64 with compensated sums: every
+// addition's rounding error is kept (two-sum) and added at the end.
 // ---------------------------------------------------------------------------
 struct KSum {
     double s, c;
     __device__ void add(double v)
     {
         const double t = s + v;
-        if (fabs(s) >= fabs(v)) c += (s - t) + v;
-        else c += (v - t) + s;
+        const double u = t - s;
+        c += (s - (t - u)) + (v - u);
         s = t;
     }
-    __device__ double value() const { return s + c; }
+    __device__ void add(const KSum& o)
+    {
+        add(o.s);
+        c += o.c;
+    }
 };
 
-constexpr int kIntChunk = 2048;
+// Sum of the block's kBlock values, in thread 0, in a fixed order (a tree over
+// the lanes, then the waves in turn).
+__device__ KSum block_sum(KSum v)
+{
+    __shared__ KSum wave_sum[kBlock / 64];
+    for (int off = 32; off > 0; off >>= 1) {
+        const KSum o{__shfl_down(v.s, off, 64), __shfl_down(v.c, off, 64)};
+        v.add(o);
+    }
+    __syncthreads();   // wave_sum may still be read from the call before
+    if ((threadIdx.x & 63u) == 0) wave_sum[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < kBlock / 64; ++w) v.add(wave_sum[w]);
+    return v;
+}
 
-// Potential partials: one value per (sink, source chunk).
+constexpr uint32_t kIntSrc = 128;   // sources per block of the potential pass
+
+// Potential: sum of m_i m_j / r_ij over the pairs i < j of active bodies (the
+// reference sums the ordered pairs and halves them; both orders of a pair give
+// the same value).  A block takes 256 sinks, one per thread, against kIntSrc
+// sources on or above the diagonal and leaves one partial sum.  VALU-bound:
+// about 33 FP64 instructions per pair with the short root and division
+// sequences (exact_ratio_fast; the library's outside their range).  16385
+// bodies, under the profiler: 226 us, where every ordered pair with the
+// library's root and division took 827.
 __global__ __launch_bounds__(kBlock) void k_potential(uint32_t lo, uint32_t hi, const double* __restrict__ x,
                                                       const double* __restrict__ y, const double* __restrict__ z,
                                                       const double* __restrict__ mass,
-                                                      const int32_t* __restrict__ id, double* __restrict__ out)
+                                                      const int32_t* __restrict__ id,
+                                                      const uint32_t* __restrict__ mass_odd, KSum* __restrict__ out)
 {
-    __shared__ double4 tile[kTile];
-    const uint32_t n = hi - lo;
-    const uint32_t li = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t c = blockIdx.y;
-    const uint32_t j0 = lo + c * kIntChunk, j1 = min(hi, j0 + kIntChunk);
-    const uint32_t i = lo + li;
-    const bool valid = li < n && id[i] > 0;
-    const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
-    const double mi = valid ? mass[i] : 0.0;
+    __shared__ double4 tile[kIntSrc];
+    const uint32_t i0 = lo + blockIdx.x * kBlock, j0 = lo + blockIdx.y * kIntSrc;
+    const uint32_t j1 = min(hi, j0 + kIntSrc);
     KSum s{0.0, 0.0};
-    for (uint32_t t0 = j0; t0 < j1; t0 += kTile) {
+    if (j1 > i0 + 1) {   // else no pair i < j
+        const uint32_t i = i0 + threadIdx.x;
+        const bool valid = i < hi && id[i] > 0;
+        const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
+        const double mi = valid ? mass[i] : 0.0;
+        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
+        if (threadIdx.x < kIntSrc) {
+            const uint32_t j = j0 + threadIdx.x;
+            // w: the mass, -0 for an inactive body
+            if (j < j1) tile[threadIdx.x] = make_double4(x[j], y[j], z[j], id[j] > 0 ? mass[j] + 0.0 : -0.0);
+        }
         __syncthreads();
-        const uint32_t j = t0 + threadIdx.x;
-        if (j < j1) tile[threadIdx.x] = make_double4(x[j], y[j], z[j], id[j] > 0 ? mass[j] : -1.0);
-        __syncthreads();
-        const uint32_t nt = min((uint32_t)kTile, j1 - t0);
-        if (valid) {
-            for (uint32_t k = 0; k < nt; ++k) {
-                const double4 q = tile[k];
-                if (q.w < 0.0 || t0 + k == i) continue;
-                const double r = sqrt(SQR(q.x - xi) + SQR(q.y - yi) + SQR(q.z - zi));
-                s.add(mi * q.w / r);
+        // the sources past the sink, two at a time
+        const uint32_t k0 = i + 1 > j0 ? min(i + 1 - j0, j1 - j0) : 0u;
+        const uint32_t k_first = __builtin_amdgcn_readfirstlane(k0);   // the wave's smallest
+        for (uint32_t k = k_first & ~1u; k < j1 - j0; k += 2) {
+            double r2[2], m[2], d[2];
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                const double4 q = tile[min(k + u, j1 - j0 - 1)];
+                r2[u] = SQR(q.x - xi) + SQR(q.y - yi) + SQR(q.z - zi);
+                m[u] = mi * q.w;
+                const bool on = valid && k + u >= k0 && k + u < j1 - j0 && !(q.w == 0.0 && signbit(q.w));
+                d[u] = on ? 1.0 : 0.0;
+            }
+            double v[2];
+            exact_ratio_fast<2>(r2, m, v);
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                if (!exact_r2_in_range(r2[u], r2_span)) v[u] = d[u] != 0.0 ? m[u] / sqrt(r2[u]) : 0.0;
+                s.add(d[u] != 0.0 ? v[u] : 0.0);
             }
         }
     }
-    if (li < n) out[(size_t)c * n + li] = s.value();
+    s = block_sum(s);
+    if (threadIdx.x == 0) out[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
-// Per-body terms of M, R, V, C and T.
+// Per-body terms of M, R, V, C and T: a partial sum of each per block of kBlock
+// bodies, out[k * gridDim.x + block].
 __global__ __launch_bounds__(kBlock) void k_body_terms(uint32_t lo, uint32_t hi, const double* x, const double* y,
                                                        const double* z, const double* vx, const double* vy,
                                                        const double* vz, const double* mass, const int32_t* id,
-                                                       double* out)
+                                                       KSum* out)
 {
-    const uint32_t n = hi - lo;
-    const uint32_t li = blockIdx.x * kBlock + threadIdx.x;
-    if (li >= n) return;
-    const uint32_t i = lo + li;
-    const bool act = id[i] > 0;
-    const double m = act ? mass[i] : 0.0;
-    const double cx = y[i] * vz[i] - z[i] * vy[i];
-    const double cy = z[i] * vx[i] - x[i] * vz[i];
-    const double cz = x[i] * vy[i] - y[i] * vx[i];
-    const double t[11] = {m, m * x[i], m * y[i], m * z[i], m * vx[i], m * vy[i], m * vz[i],
-                          cx * m, cy * m, cz * m, m * (SQR(vx[i]) + SQR(vy[i]) + SQR(vz[i]))};
+    const uint32_t i = lo + blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t ic = min(i, hi - 1);
+    const bool act = i < hi && id[ic] > 0;
+    const double m = mass[ic];
+    const double px = x[ic], py = y[ic], pz = z[ic], ux = vx[ic], uy = vy[ic], uz = vz[ic];
+    const double cx = py * uz - pz * uy;
+    const double cy = pz * ux - px * uz;
+    const double cz = px * uy - py * ux;
+    const double t[11] = {m, m * px, m * py, m * pz, m * ux, m * uy, m * uz,
+                          cx * m, cy * m, cz * m, m * (SQR(ux) + SQR(uy) + SQR(uz))};
 #pragma unroll
-    for (int k = 0; k < 11; ++k) out[(size_t)k * n + li] = act ? t[k] : 0.0;
+    for (int k = 0; k < 11; ++k) {
+        const KSum s = block_sum(KSum{act ? t[k] : 0.0, 0.0});
+        if (threadIdx.x == 0) out[(size_t)k * gridDim.x + blockIdx.x] = s;
+    }
 }
 
-// Sums rows of a [rows][len] array, one block per row, fixed order.
-__global__ __launch_bounds__(kBlock) void k_row_sum(const double* in, size_t len, double* out)
+// The totals: block k < 11 sums the n_body partials of body term k, block 11
+// the n_pair partials of the potential, in a fixed order.
+__global__ __launch_bounds__(kBlock) void k_integral_total(const KSum* __restrict__ body, uint32_t n_body,
+                                                           const KSum* __restrict__ pair, uint32_t n_pair,
+                                                           double* __restrict__ out, double* __restrict__ out_u)
 {
-    __shared__ double ss[kBlock], cs[kBlock];
-    const double* row = in + (size_t)blockIdx.x * len;
+    const uint32_t k = blockIdx.x;
+    const KSum* row = k < 11 ? body + (size_t)k * n_body : pair;
+    const uint32_t len = k < 11 ? n_body : n_pair;
     KSum s{0.0, 0.0};
-    for (size_t k = threadIdx.x; k < len; k += kBlock) s.add(row[k]);
-    ss[threadIdx.x] = s.s;
-    cs[threadIdx.x] = s.c;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        KSum t{0.0, 0.0};
-        for (int k = 0; k < kBlock; ++k) t.add(ss[k]);
-        for (int k = 0; k < kBlock; ++k) t.add(cs[k]);
-        out[blockIdx.x] = t.value();
-    }
+    for (uint32_t q = threadIdx.x; q < len; q += kBlock) s.add(row[q]);
+    s = block_sum(s);
+    if (threadIdx.x == 0) *(k < 11 ? out + k : out_u) = s.s + s.c;
+}
+
+size_t integral_scratch(uint32_t n)
+{
+    const size_t nb = (n + kBlock - 1) / kBlock, nc = (n + kIntSrc - 1) / kIntSrc;
+    return (11 * nb + nb * nc) * (sizeof(KSum) / sizeof(double));
 }
 
 hipError_t launch_integral(hipStream_t st, uint32_t lo, uint32_t hi, const double* x, const double* y,
                            const double* z, const double* vx, const double* vy, const double* vz,
-                           const double* mass, const int32_t* id, double* scratch, size_t scratch_len, double* out,
-                           double* out_u)
+                           const double* mass, const int32_t* id, const uint32_t* mass_odd, double* scratch,
+                           size_t scratch_len, double* out, double* out_u)
 {
     const uint32_t n = hi - lo;
     if (n == 0) return hipSuccess;
-    const uint32_t nchunk = (n + kIntChunk - 1) / kIntChunk;
-    if (scratch_len < (size_t)11 * n || scratch_len < (size_t)nchunk * n) return hipErrorInvalidValue;
-    const uint32_t gb = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_body_terms, dim3(gb), dim3(kBlock), 0, st, lo, hi, x, y, z, vx, vy, vz, mass, id, scratch);
-    hipLaunchKernelGGL(k_row_sum, dim3(11), dim3(kBlock), 0, st, scratch, (size_t)n, out);
-    hipLaunchKernelGGL(k_potential, dim3(gb, nchunk), dim3(kBlock), 0, st, lo, hi, x, y, z, mass, id, scratch);
-    hipLaunchKernelGGL(k_row_sum, dim3(1), dim3(kBlock), 0, st, scratch, (size_t)nchunk * n, out_u);
+    if (scratch_len < integral_scratch(n)) return hipErrorInvalidValue;
+    const uint32_t nb = (n + kBlock - 1) / kBlock, nc = (n + kIntSrc - 1) / kIntSrc;
+    KSum* body = reinterpret_cast<KSum*>(scratch);
+    KSum* pair = body + (size_t)11 * nb;
+    hipLaunchKernelGGL(k_body_terms, dim3(nb), dim3(kBlock), 0, st, lo, hi, x, y, z, vx, vy, vz, mass, id, body);
+    hipLaunchKernelGGL(k_potential, dim3(nb, nc), dim3(kBlock), 0, st, lo, hi, x, y, z, mass, id, mass_odd, pair);
+    hipLaunchKernelGGL(k_integral_total, dim3(12), dim3(kBlock), 0, st, body, nb, pair, nb * nc, out, out_u);
     return hipGetLastError();
 }
 
