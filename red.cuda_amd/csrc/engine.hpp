@@ -220,6 +220,9 @@ hipError_t launch_features(hipStream_t s, const WorkItem* items, uint32_t n_item
                            const double* vy, const double* vz, const double* mass, const int32_t* id,
                            const uint32_t* disk_of, const DiskInfo* info, const DiskCtl* ctl, uint32_t* feat,
                            double* eterm, double* esum);
+// records of n bodies from `first` on into pinned host arrays (NULL: not wanted)
+hipError_t launch_export_bodies(hipStream_t s, uint32_t first, uint32_t n, const BodyArrays& b, double* r, double* v,
+                                double* p);
 // rec[kBodyRecord q + f] = b.a[f][idx[q]] for q < n
 hipError_t launch_gather_bodies(hipStream_t s, uint32_t n, const uint32_t* idx, const BodyArrays& b, double* rec);
 // the inverse, plus id[idx[q]] = ids[q]

@@ -2213,6 +2213,31 @@ __global__ __launch_bounds__(kBlock) void k_scatter_bodies(uint32_t n, const uin
     else id[idx[q]] = ids[q];
 }
 
+// Records of n consecutive bodies from `first` on, as the caller's structs:
+// r and v as (x, y, z, 0), p as (mass, radius, density, cd), each array skipped
+// if NULL.  The destination is pinned host memory, written over PCIe in whole
+// 16-byte pieces of consecutive lanes; blockIdx.y picks the array.
+__global__ __launch_bounds__(kBlock) void k_export_bodies(uint32_t first, uint32_t n, BodyArrays b, double2* r,
+                                                          double2* v, double2* p)
+{
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= 2 * n) return;
+    const uint32_t i = first + t / 2, half = t & 1u, which = blockIdx.y;
+    double2* dst = which == 0 ? r : (which == 1 ? v : p);
+    if (!dst) return;
+    const uint32_t f = 3 * which + 2 * half;   // first field of this piece
+    dst[t] = make_double2(b.a[f][i], which < 2 && half ? 0.0 : b.a[f + 1][i]);
+}
+
+hipError_t launch_export_bodies(hipStream_t st, uint32_t first, uint32_t n, const BodyArrays& b, double* r, double* v,
+                                double* p)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_export_bodies, dim3((2 * n + kBlock - 1) / kBlock, 3), dim3(kBlock), 0, st, first, n, b,
+                       (double2*)r, (double2*)v, (double2*)p);
+    return hipGetLastError();
+}
+
 hipError_t launch_gather_bodies(hipStream_t st, uint32_t n, const uint32_t* idx, const BodyArrays& b, double* rec)
 {
     const uint32_t grid = (n * kBodyRecord + kBlock - 1) / kBlock;
