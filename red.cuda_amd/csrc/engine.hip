@@ -507,7 +507,7 @@ int build_lists(rd_disk* d)
     size_t max_chunks = 1;
     double pairs = 0.0;
     const uint32_t S = d->tuning.sinks_per_lane;
-    const uint32_t C = std::max<uint32_t>(kTile, d->tuning.chunk / kTile * kTile);
+    const uint32_t C_max = std::max<uint32_t>(kTile, d->tuning.chunk / kTile * kTile);
     // FP64: one sink per lane when 256-sink items give >= 4 blocks per CU, else
     // the term-parallel kernel on items of kExactSinks (same bits in every case)
     if (d->precision == RD_PREC_FP64) {
@@ -545,6 +545,27 @@ int build_lists(rd_disk* d)
         const uint32_t k = o.second;
         const HostDisk& h = d->hd[k];
         DiskInfo& di = d->h_info[k];
+        // one-sided pairs: chunk and sinks per item of this disk (kOneSidedItems)
+        auto one_sided_src = [&](int cls, const uint32_t b[4]) {   // first one-sided source
+            const uint32_t lo = std::max(b[2], di.n_fp64);
+            return sym && cls == 0 ? std::max(lo, b[1]) : lo;
+        };
+        uint32_t C = C_max, S_one = S;
+        if (d->precision == RD_PREC_MIXED) {
+            auto n_one = [&](uint32_t chunk, uint32_t s) {
+                size_t n = 0;
+                for (int cls = 0; cls < 3; ++cls) {
+                    uint32_t b[4];
+                    class_bounds(h, cls, b);
+                    const uint32_t lo = one_sided_src(cls, b);
+                    if (b[1] > b[0] && b[3] > lo)
+                        n += (size_t)((b[1] - b[0] + 64 * s - 1) / (64 * s)) * ((b[3] - lo + chunk - 1) / chunk);
+                }
+                return n;
+            };
+            while (C > (uint32_t)kTile && n_one(C, S) < kOneSidedItems) C = (C / 2 + kTile - 1) / kTile * kTile;
+            if (n_one(C, S) < kOneSidedItems) S_one = 1;
+        }
         for (int cls = 0; cls < 3; ++cls) {
             uint32_t b[4];
             class_bounds(h, cls, b);
@@ -561,7 +582,8 @@ int build_lists(rd_disk* d)
                 // symmetric: SI x SI pairs once each (the FP64 prefix takes part
                 // with FP32 mass 0: its own sink sums are kept, it pulls no one);
                 // the SI sinks' NSI sources stay one-sided, in slots after them
-                uint32_t base = 0, lo = std::max(b[2], di.n_fp64);
+                uint32_t base = 0;
+                const uint32_t lo = one_sided_src(cls, b);
                 if (sym && cls == 0) {
                     const uint32_t nblk = (b[1] + kSymBlockBodies - 1) / kSymBlockBodies;
                     // kSymChunks..2 kSymChunks - 1 chunks once the disk is that large:
@@ -582,19 +604,19 @@ int build_lists(rd_disk* d)
                                                                  c, a, a == c ? self : 0u}});
                         }
                     base = nc;
-                    lo = std::max(lo, b[1]);
                 }
                 const uint32_t hi = b[3];
                 const uint32_t nsrc = hi > lo ? hi - lo : 0;
                 const uint32_t nch = (nsrc + C - 1) / C;
                 di.nchunk[cls] = base + nch;
                 max_chunks = std::max<size_t>(max_chunks, base + nch);
-                const uint32_t G = 64u * S;
+                const uint32_t G = 64u * S_one;
+                const uint32_t narrow = S_one == 1 ? kItemNarrow : 0u;
                 for (uint32_t s = b[0]; s < b[1]; s += G)
                     for (uint32_t c = 0; c < nch; ++c)
                         items.push_back(WorkItem{k, h.off + s, h.off + std::min(b[1], s + G),
                                                  h.off + lo + c * C, h.off + std::min(hi, lo + (c + 1) * C), base + c,
-                                                 0, 0});
+                                                 0, narrow});
             }
         }
     }
@@ -719,11 +741,9 @@ hipError_t enqueue_force(rd_disk* d, const double* fx, const double* fy, const d
                                   fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all);
     // mixed precision: FP32 slot totals, in float units of the same buffer
     float* part32 = reinterpret_cast<float*>(d->part);
-    if (hipError_t e = launch_force_sym(d->stream, d->sym_R, d->sym_self, d->items_sym, d->n_items_sym, d->grid_sym,
-                                        fx, fy, fz, d->m32, d->ctl, need, part32, d->n_all))
-        return e;
-    return launch_force_mixed(d->stream, (int)d->tuning.sinks_per_lane, d->items_force, d->n_items_force,
-                              d->grid_force, fx, fy, fz, d->m32, d->ctl, need, part32, d->n_all);
+    const MixedLists l{d->items_sym,   d->n_items_sym,   d->grid_sym,   d->sym_R,                    d->sym_self,
+                       d->items_force, d->n_items_force, d->grid_force, (int)d->tuning.sinks_per_lane};
+    return launch_force_mixed(d->stream, l, fx, fy, fz, d->m32, d->ctl, need, part32, d->n_all);
 }
 
 int last_stage(const rd_integrator* it) { return it->n_stage - 1; }

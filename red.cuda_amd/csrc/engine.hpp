@@ -93,11 +93,17 @@ struct WorkItem {
     uint32_t src_lo, src_hi;
     uint32_t slot;       // partial-sum slot of the sinks
     uint32_t src_slot;   // symmetric kernel: partial-sum slot of the sources
-    uint32_t flags;      // symmetric kernel: kItemSelf
+    uint32_t flags;      // kItemSelf, kItemNarrow
 };
 // diagonal item whose full-block diagonal tiles take each pair once with its
 // reaction (a disk of at most kSymSelfMaxBlocks blocks)
 constexpr uint32_t kItemSelf = 1u;
+// one-sided item of 64 sinks, one per lane, whatever the launch's sinks per lane
+constexpr uint32_t kItemNarrow = 2u;
+// One-sided items of a disk: chunks are halved (down to one 256-source tile),
+// then the sinks taken one per lane, until the disk has this many items -- two
+// per CU.  A decision of the disk alone: results never depend on the batch.
+constexpr uint32_t kOneSidedItems = 512;
 
 // Gas disk, device copy: the analytic model (analytic_gas_disk_params_t
 // red_type.h:464-485) or frame 0 of a FARGO grid (fargo_gas_disk.h:8-60).
@@ -168,19 +174,22 @@ hipError_t launch_force_exact_rk4(hipStream_t s, uint32_t sinks, int r, const Wo
                                   uint32_t grid, const double* x, const double* y, const double* z,
                                   const double* m_ex, const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need,
                                   const StageArgs& a);
-hipError_t launch_force_mixed(hipStream_t s, int sinks_per_lane, const WorkItem* items, uint32_t n_items,
-                              uint32_t grid, const double* x, const double* y, const double* z,
+// Mixed precision: the symmetric kernel's (chunk a, chunk c) items -- sink_lo/hi =
+// chunk a, src_lo/hi = chunk c (256-body blocks, R per chunk), slot = c (sink
+// side), src_slot = a (source side); self: some item carries kItemSelf (the
+// kernel instance with the diagonal reaction sweep) -- and the one-sided
+// kernel's, of 64 S sinks (64 where flagged kItemNarrow), in one launch.
+struct MixedLists {
+    const WorkItem* sym;
+    uint32_t n_sym, grid_sym, R;
+    bool self;
+    const WorkItem* one;
+    uint32_t n_one, grid_one;
+    int S;
+};
+hipError_t launch_force_mixed(hipStream_t s, const MixedLists& l, const double* x, const double* y, const double* z,
                               const float* m32, const DiskCtl* ctl, uint32_t need_mask, float* part,
                               uint32_t n_all);
-// Symmetric pair kernel over (chunk a, chunk c) items: sink_lo/hi = chunk a,
-// src_lo/hi = chunk c (256-body blocks, R per chunk), slot = c (sink side),
-// src_slot = a (source side).
-// self: some item carries kItemSelf (the kernel instance with the diagonal
-// reaction sweep).
-hipError_t launch_force_sym(hipStream_t s, uint32_t R, bool self, const WorkItem* items, uint32_t n_items,
-                            uint32_t grid, const double* x, const double* y, const double* z, const float* m32,
-                            const DiskCtl* ctl, uint32_t need_mask, float* part, uint32_t n_all);
-size_t force_sym_lds_bytes(uint32_t R);
 hipError_t launch_stage(hipStream_t s, int method, int r, const StageArgs& a);
 hipError_t launch_comb1(hipStream_t s, int method, const StageArgs& a);
 hipError_t launch_commit(hipStream_t s, const StageArgs& a, int advance_time, DiskCtl* ctl_rw);

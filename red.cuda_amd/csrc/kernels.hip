@@ -550,6 +550,122 @@ constexpr float kEps2 = 1.0e-24f;
 // v_rsq_f32, FP32 partial sums per 64-source quarter tile folded into FP64.
 // The quarter sums of the four waves are combined in fixed order, so the
 // result is deterministic.
+// LDS of the one-sided kernel: the source tile and three waves' sums.
+constexpr size_t mixed_lds_bytes(int S) { return kTile * sizeof(SrcF) + (size_t)3 * S * 3 * 64 * sizeof(double); }
+
+// One item of 64 S sinks.
+template <int S>
+__device__ __forceinline__ void force_mixed_item(const WorkItem& w, unsigned char* lds, const double* __restrict__ x,
+                                                 const double* __restrict__ y, const double* __restrict__ z,
+                                                 const float* __restrict__ m32, float* __restrict__ part,
+                                                 uint32_t n_all)
+{
+    SrcF* tile = reinterpret_cast<SrcF*>(lds);
+    double(*red)[3][64] = reinterpret_cast<double(*)[3][64]>(tile + kTile);   // [3 S][3][64]
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    double xi[S], yi[S], zi[S], ax[S], ay[S], az[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const uint32_t i = w.sink_lo + lane + 64u * s;
+        const bool valid = i < w.sink_hi;
+        xi[s] = valid ? x[i] : 0.0;
+        yi[s] = valid ? y[i] : 0.0;
+        zi[s] = valid ? z[i] : 0.0;
+        ax[s] = ay[s] = az[s] = 0.0;
+    }
+    for (uint32_t t0 = w.src_lo; t0 < w.src_hi; t0 += kTile) {
+        __syncthreads();
+        {
+            const uint32_t j = t0 + tid;
+            SrcF r;
+            if (j < w.src_hi) {
+                r.x = x[j]; r.y = y[j]; r.z = z[j]; r.m = m32[j];
+            } else {
+                r.x = 0.0; r.y = 0.0; r.z = 0.0; r.m = 0.0f;
+            }
+            r.pad = 0.0f;
+            tile[tid] = r;
+        }
+        __syncthreads();
+        const uint32_t nt = min((uint32_t)kTile, w.src_hi - t0);
+        const uint32_t k0 = wave * 64u;
+        const uint32_t k1 = min(k0 + 64u, (nt + 3u) & ~3u);
+        float fx[S], fy[S], fz[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) fx[s] = fy[s] = fz[s] = 0.0f;
+        for (uint32_t k = k0; k < k1; k += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const SrcF r = tile[k + u];
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    const float dx = (float)(r.x - xi[s]);
+                    const float dy = (float)(r.y - yi[s]);
+                    const float dz = (float)(r.z - zi[s]);
+                    float r2 = __builtin_fmaf(dz, dz, kEps2);
+                    r2 = __builtin_fmaf(dy, dy, r2);
+                    r2 = __builtin_fmaf(dx, dx, r2);
+                    const float ri = __builtin_amdgcn_rsqf(r2);
+                    const float ri2 = ri * ri;
+                    const float sc = (r.m * ri) * ri2;
+                    fx[s] = __builtin_fmaf(sc, dx, fx[s]);
+                    fy[s] = __builtin_fmaf(sc, dy, fy[s]);
+                    fz[s] = __builtin_fmaf(sc, dz, fz[s]);
+                }
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            ax[s] += (double)fx[s];
+            ay[s] += (double)fy[s];
+            az[s] += (double)fz[s];
+        }
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            red[(wave - 1) * S + s][0][lane] = ax[s];
+            red[(wave - 1) * S + s][1][lane] = ay[s];
+            red[(wave - 1) * S + s][2][lane] = az[s];
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const uint32_t i = w.sink_lo + lane + 64u * s;
+            if (i < w.sink_hi) {
+                const double sx = ((ax[s] + red[s][0][lane]) + red[S + s][0][lane]) + red[2 * S + s][0][lane];
+                const double sy = ((ay[s] + red[s][1][lane]) + red[S + s][1][lane]) + red[2 * S + s][1][lane];
+                const double sz = ((az[s] + red[s][2][lane]) + red[S + s][2][lane]) + red[2 * S + s][2][lane];
+                part[(size_t)(w.slot * 3 + 0) * n_all + i] = (float)sx;
+                part[(size_t)(w.slot * 3 + 1) * n_all + i] = (float)sy;
+                part[(size_t)(w.slot * 3 + 2) * n_all + i] = (float)sz;
+            }
+        }
+    }
+}
+
+// Items first, first + stride, ...: 64 S sinks each, or 64 where flagged
+// kItemNarrow.
+template <int S>
+__device__ __forceinline__ void force_mixed_body(uint32_t first, uint32_t stride, unsigned char* lds,
+                                                 const WorkItem* __restrict__ items, uint32_t n_items,
+                                                 const double* __restrict__ x, const double* __restrict__ y,
+                                                 const double* __restrict__ z, const float* __restrict__ m32,
+                                                 const DiskCtl* __restrict__ ctl, uint32_t need,
+                                                 float* __restrict__ part, uint32_t n_all)
+{
+    for (uint32_t it = first; it < n_items; it += stride) {
+        const WorkItem w = items[it];
+        if (!(ctl[w.disk].flags & need)) continue;
+        if (S > 1 && (w.flags & kItemNarrow)) force_mixed_item<1>(w, lds, x, y, z, m32, part, n_all);
+        else force_mixed_item<S>(w, lds, x, y, z, m32, part, n_all);
+        __syncthreads();
+    }
+}
+
 template <int S>
 __global__ __launch_bounds__(kBlock) void k_force_mixed(const WorkItem* __restrict__ items, uint32_t n_items,
                                                         const double* __restrict__ x, const double* __restrict__ y,
@@ -558,96 +674,8 @@ __global__ __launch_bounds__(kBlock) void k_force_mixed(const WorkItem* __restri
                                                         const DiskCtl* __restrict__ ctl, uint32_t need,
                                                         float* __restrict__ part, uint32_t n_all)
 {
-    __shared__ SrcF tile[kTile];
-    __shared__ double red[3][S][3][64];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
-        const WorkItem w = items[it];
-        if (!(ctl[w.disk].flags & need)) continue;
-        double xi[S], yi[S], zi[S], ax[S], ay[S], az[S];
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const uint32_t i = w.sink_lo + lane + 64u * s;
-            const bool valid = i < w.sink_hi;
-            xi[s] = valid ? x[i] : 0.0;
-            yi[s] = valid ? y[i] : 0.0;
-            zi[s] = valid ? z[i] : 0.0;
-            ax[s] = ay[s] = az[s] = 0.0;
-        }
-        for (uint32_t t0 = w.src_lo; t0 < w.src_hi; t0 += kTile) {
-            __syncthreads();
-            {
-                const uint32_t j = t0 + tid;
-                SrcF r;
-                if (j < w.src_hi) {
-                    r.x = x[j]; r.y = y[j]; r.z = z[j]; r.m = m32[j];
-                } else {
-                    r.x = 0.0; r.y = 0.0; r.z = 0.0; r.m = 0.0f;
-                }
-                r.pad = 0.0f;
-                tile[tid] = r;
-            }
-            __syncthreads();
-            const uint32_t nt = min((uint32_t)kTile, w.src_hi - t0);
-            const uint32_t k0 = wave * 64u;
-            const uint32_t k1 = min(k0 + 64u, (nt + 3u) & ~3u);
-            float fx[S], fy[S], fz[S];
-#pragma unroll
-            for (int s = 0; s < S; ++s) fx[s] = fy[s] = fz[s] = 0.0f;
-            for (uint32_t k = k0; k < k1; k += 4) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const SrcF r = tile[k + u];
-#pragma unroll
-                    for (int s = 0; s < S; ++s) {
-                        const float dx = (float)(r.x - xi[s]);
-                        const float dy = (float)(r.y - yi[s]);
-                        const float dz = (float)(r.z - zi[s]);
-                        float r2 = __builtin_fmaf(dz, dz, kEps2);
-                        r2 = __builtin_fmaf(dy, dy, r2);
-                        r2 = __builtin_fmaf(dx, dx, r2);
-                        const float ri = __builtin_amdgcn_rsqf(r2);
-                        const float ri2 = ri * ri;
-                        const float sc = (r.m * ri) * ri2;
-                        fx[s] = __builtin_fmaf(sc, dx, fx[s]);
-                        fy[s] = __builtin_fmaf(sc, dy, fy[s]);
-                        fz[s] = __builtin_fmaf(sc, dz, fz[s]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                ax[s] += (double)fx[s];
-                ay[s] += (double)fy[s];
-                az[s] += (double)fz[s];
-            }
-        }
-        if (wave > 0) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                red[wave - 1][s][0][lane] = ax[s];
-                red[wave - 1][s][1][lane] = ay[s];
-                red[wave - 1][s][2][lane] = az[s];
-            }
-        }
-        __syncthreads();
-        if (wave == 0) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const uint32_t i = w.sink_lo + lane + 64u * s;
-                if (i < w.sink_hi) {
-                    const double sx = ((ax[s] + red[0][s][0][lane]) + red[1][s][0][lane]) + red[2][s][0][lane];
-                    const double sy = ((ay[s] + red[0][s][1][lane]) + red[1][s][1][lane]) + red[2][s][1][lane];
-                    const double sz = ((az[s] + red[0][s][2][lane]) + red[1][s][2][lane]) + red[2][s][2][lane];
-                    part[(size_t)(w.slot * 3 + 0) * n_all + i] = (float)sx;
-                    part[(size_t)(w.slot * 3 + 1) * n_all + i] = (float)sy;
-                    part[(size_t)(w.slot * 3 + 2) * n_all + i] = (float)sz;
-                }
-            }
-        }
-        __syncthreads();
-    }
+    __shared__ __align__(16) unsigned char lds[mixed_lds_bytes(S)];
+    force_mixed_body<S>(blockIdx.x, gridDim.x, lds, items, n_items, x, y, z, m32, ctl, need, part, n_all);
 }
 
 // ---------------------------------------------------------------------------
@@ -912,13 +940,13 @@ static_assert(kSymS * 3 * 64 * sizeof(double) <= kSymTile * (sizeof(double2) + s
 // one only when an item is flagged (the compiler schedules the main loop of
 // the instance with the extra sweep less well).
 template <bool kSelf>
-__global__ __launch_bounds__(kBlock) void k_force_sym(const WorkItem* __restrict__ items, uint32_t n_items,
-                                                      const double* __restrict__ x, const double* __restrict__ y,
-                                                      const double* __restrict__ z, const float* __restrict__ m32,
-                                                      const DiskCtl* __restrict__ ctl, uint32_t need,
-                                                      float* __restrict__ part, uint32_t n_all)
+__device__ __forceinline__ void force_sym_body(uint32_t first, uint32_t stride, unsigned char* sym_lds,
+                                               const WorkItem* __restrict__ items, uint32_t n_items,
+                                               const double* __restrict__ x, const double* __restrict__ y,
+                                               const double* __restrict__ z, const float* __restrict__ m32,
+                                               const DiskCtl* __restrict__ ctl, uint32_t need,
+                                               float* __restrict__ part, uint32_t n_all)
 {
-    extern __shared__ __align__(16) unsigned char sym_lds[];
     double2* txy = reinterpret_cast<double2*>(sym_lds);
     SrcZM* tzm = reinterpret_cast<SrcZM*>(txy + kSymTile);
     double* red = reinterpret_cast<double*>(sym_lds);          // [S][3][64], aliases the tile
@@ -926,7 +954,7 @@ __global__ __launch_bounds__(kBlock) void k_force_sym(const WorkItem* __restrict
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t kb = wave * 128u + 64u + lane;   // this lane's tile entry at step 0 (kSymTile)
-    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
+    for (uint32_t it = first; it < n_items; it += stride) {
         const WorkItem w = items[it];
         if (!(ctl[w.disk].flags & need)) continue;
         const bool diag = w.sink_lo == w.src_lo;
@@ -1071,22 +1099,38 @@ __global__ __launch_bounds__(kBlock) void k_force_sym(const WorkItem* __restrict
     }
 }
 
-hipError_t launch_force_sym(hipStream_t st, uint32_t R, bool self, const WorkItem* items, uint32_t n_items,
-                            uint32_t grid, const double* x, const double* y, const double* z, const float* m32,
-                            const DiskCtl* ctl, uint32_t need, float* part, uint32_t n_all)
+template <bool kSelf>
+__global__ __launch_bounds__(kBlock) void k_force_sym(const WorkItem* __restrict__ items, uint32_t n_items,
+                                                      const double* __restrict__ x, const double* __restrict__ y,
+                                                      const double* __restrict__ z, const float* __restrict__ m32,
+                                                      const DiskCtl* __restrict__ ctl, uint32_t need,
+                                                      float* __restrict__ part, uint32_t n_all)
 {
-    if (n_items == 0) return hipSuccess;
-    if (R < 1 || R > kSymMaxR) return hipErrorInvalidValue;
-    if (self)
-        hipLaunchKernelGGL(k_force_sym<true>, dim3(grid), dim3(kBlock), sym_lds_bytes(R), st, items, n_items, x, y, z,
-                           m32, ctl, need, part, n_all);
-    else
-        hipLaunchKernelGGL(k_force_sym<false>, dim3(grid), dim3(kBlock), sym_lds_bytes(R), st, items, n_items, x, y,
-                           z, m32, ctl, need, part, n_all);
-    return hipGetLastError();
+    extern __shared__ __align__(16) unsigned char sym_lds[];
+    force_sym_body<kSelf>(blockIdx.x, gridDim.x, sym_lds, items, n_items, x, y, z, m32, ctl, need, part, n_all);
 }
 
-size_t force_sym_lds_bytes(uint32_t R) { return sym_lds_bytes(R); }
+// Both kinds of pairs in one launch (disks with NSI or NI bodies): blocks
+// [0, grid_sym) take the symmetric items, the others the one-sided ones.  The
+// two write different partial-sum slots and wait for nothing of each other; as two
+// launches a small disk paid for both in turn (star + 3000 bodies of all
+// classes: 17 + 23 us, each on a few blocks).
+template <bool kSelf, int S>
+__global__ __launch_bounds__(kBlock) void k_force_both(const WorkItem* __restrict__ items_sym, uint32_t n_sym,
+                                                       uint32_t grid_sym, const WorkItem* __restrict__ items,
+                                                       uint32_t n_items, const double* __restrict__ x,
+                                                       const double* __restrict__ y, const double* __restrict__ z,
+                                                       const float* __restrict__ m32,
+                                                       const DiskCtl* __restrict__ ctl, uint32_t need,
+                                                       float* __restrict__ part, uint32_t n_all)
+{
+    extern __shared__ __align__(16) unsigned char sym_lds[];
+    if (blockIdx.x < grid_sym)
+        force_sym_body<kSelf>(blockIdx.x, grid_sym, sym_lds, items_sym, n_sym, x, y, z, m32, ctl, need, part, n_all);
+    else
+        force_mixed_body<S>(blockIdx.x - grid_sym, gridDim.x - grid_sym, sym_lds, items, n_items, x, y, z, m32, ctl,
+                            need, part, n_all);
+}
 
 hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
@@ -1128,16 +1172,41 @@ hipError_t launch_force_exact_rk4(hipStream_t st, uint32_t sinks, int r, const W
     return hipGetLastError();
 }
 
-hipError_t launch_force_mixed(hipStream_t st, int S, const WorkItem* items, uint32_t n_items, uint32_t grid,
-                              const double* x, const double* y, const double* z, const float* m32,
-                              const DiskCtl* ctl, uint32_t need, float* part, uint32_t n_all)
+hipError_t launch_force_mixed(hipStream_t st, const MixedLists& l, const double* x, const double* y, const double* z,
+                              const float* m32, const DiskCtl* ctl, uint32_t need, float* part, uint32_t n_all)
 {
-    if (n_items == 0) return hipSuccess;
-    switch (S) {
-    case 1: hipLaunchKernelGGL(k_force_mixed<1>, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m32, ctl, need, part, n_all); break;
-    case 2: hipLaunchKernelGGL(k_force_mixed<2>, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m32, ctl, need, part, n_all); break;
-    case 4: hipLaunchKernelGGL(k_force_mixed<4>, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m32, ctl, need, part, n_all); break;
-    default: return hipErrorInvalidValue;
+    if (l.n_sym && (l.R < 1 || l.R > kSymMaxR)) return hipErrorInvalidValue;
+    if (l.S != 1 && l.S != 2 && l.S != 4) return hipErrorInvalidValue;
+    if (l.n_sym && l.n_one) {
+        const size_t lds = std::max(sym_lds_bytes(l.R), mixed_lds_bytes(l.S));
+#define FORCE_BOTH(SELF, S)                                                                                         \
+    hipLaunchKernelGGL((k_force_both<SELF, S>), dim3(l.grid_sym + l.grid_one), dim3(kBlock), lds, st, l.sym, l.n_sym, \
+                       l.grid_sym, l.one, l.n_one, x, y, z, m32, ctl, need, part, n_all)
+        if (l.self) {
+            if (l.S == 1) FORCE_BOTH(true, 1);
+            else if (l.S == 2) FORCE_BOTH(true, 2);
+            else FORCE_BOTH(true, 4);
+        } else {
+            if (l.S == 1) FORCE_BOTH(false, 1);
+            else if (l.S == 2) FORCE_BOTH(false, 2);
+            else FORCE_BOTH(false, 4);
+        }
+#undef FORCE_BOTH
+    } else if (l.n_sym) {
+#define FORCE_SYM(SELF)                                                                                              \
+    hipLaunchKernelGGL(k_force_sym<SELF>, dim3(l.grid_sym), dim3(kBlock), sym_lds_bytes(l.R), st, l.sym, l.n_sym, x, \
+                       y, z, m32, ctl, need, part, n_all)
+        if (l.self) FORCE_SYM(true);
+        else FORCE_SYM(false);
+#undef FORCE_SYM
+    } else if (l.n_one) {
+#define FORCE_ONE(S)                                                                                              \
+    hipLaunchKernelGGL(k_force_mixed<S>, dim3(l.grid_one), dim3(kBlock), 0, st, l.one, l.n_one, x, y, z, m32, ctl, \
+                       need, part, n_all)
+        if (l.S == 1) FORCE_ONE(1);
+        else if (l.S == 2) FORCE_ONE(2);
+        else FORCE_ONE(4);
+#undef FORCE_ONE
     }
     return hipGetLastError();
 }
