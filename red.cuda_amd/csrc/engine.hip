@@ -322,7 +322,12 @@ void free_buffers(rd_disk* d)
 }
 
 // Waves of a per-body launch (3 components): the single-disk error slots.
-size_t n_errw(const rd_disk* d) { return 3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock) + 1; }
+// error words: one per wave of the last stage kernel, or per summing wave of the
+// fused one (at most 6 in a block, a block per CU)
+size_t n_errw(const rd_disk* d)
+{
+    return std::max(3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock) + 1, 6 * (size_t)d->n_cu);
+}
 
 int alloc_buffers(rd_disk* d)
 {
@@ -759,29 +764,93 @@ int flag_check_only(rd_disk* d, const std::vector<char>& on)
     return RD_OK;
 }
 
+ExactLists exact_lists(const rd_disk* d)
+{
+    return {d->items_force, d->n_items_force, d->grid_force, d->exact_sinks, d->m_ex, d->mass_odd};
+}
+
+// FP64 items of 4 or 8 sinks are at most one block per CU: launches, not pairs,
+// set the time, and the summing lanes, which hold every body's complete sum, can
+// do what follows it.  One gas-free disk's RKF7(8) or fixed-step RK4 runs each stage
+// so (launch_force_exact_stage): the same operations in the same order as pair
+// pass + stage kernel, one launch per stage instead of two (RKF7(8), 1501
+// bodies: 267 -> 253 us a step; 701 bodies: 163 -> 134)
+bool fused_stages(const rd_integrator* it)
+{
+    const rd_disk* d = it->d;
+    return d->precision == RD_PREC_FP64 && (d->exact_sinks == 4 || d->exact_sinks == 8) && d->n_disk == 1 &&
+           d->gas.on == kGasNone && (it->method == RD_RKF78 || (it->method == RD_RK4 && !it->adaptive));
+}
+
+// The operator too, and with gas on 4-sink items (drag takes more registers than the
+// ten waves of an 8-sink block have).  701 bodies in gas: 35.5 -> 23.9 us.
+bool fused_operator(const rd_disk* d)
+{
+    return d->precision == RD_PREC_FP64 &&
+           (d->exact_sinks == 4 || (d->exact_sinks == 8 && d->gas.on == kGasNone));
+}
+
+// error words that the last stage of an adaptive attempt writes for a single disk
+size_t error_words(const rd_integrator* it)
+{
+    const rd_disk* d = it->d;
+    if (fused_stages(it)) return (size_t)d->grid_force * (3 * d->exact_sinks / 4);
+    return 3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock);
+}
+
+// The next attempt's stage-0 pair pass of the disks flagged F_SPEC_K0.
+hipError_t enqueue_k0_ahead(rd_integrator* it)
+{
+    rd_disk* d = it->d;
+    if (!fused_stages(it)) return enqueue_force(d, d->x, d->y, d->z, F_SPEC_K0);
+    StageArgs a = make_args(d, 0, it->adaptive, it->err_all);
+    return launch_force_exact_stage(d->stream, exact_lists(d), it->method, 0, F_SPEC_K0, a);
+}
+
+// calc_dydx of disk k on the disk's device: r, v and dy are rd_var4 records
+// there.  Positions into P[0], velocities into the stage-1 velocity slot.
+int enqueue_operator(rd_disk* d, uint32_t k, double t, const double* r, const double* v, double* dy)
+{
+    const HostDisk& h = d->hd[k];
+    double* const p[3] = {d->P[0][0] + h.off, d->P[0][1] + h.off, d->P[0][2] + h.off};
+    double* const vel[3] = {kv_ptr(d, 1, 0) + h.off, kv_ptr(d, 1, 1) + h.off, kv_ptr(d, 1, 2) + h.off};
+    HIP_TRY(launch_operator_begin(d->stream, h.n, r, v, p, vel, d->ctl, d->n_disk, k));
+    StageArgs a = make_args(d, 2, 0, 0);   // fpos = P[0]
+    a.info0 = d->h_info[k];
+    const double* const va[3] = {kv_ptr(d, 1, 0), kv_ptr(d, 1, 1), kv_ptr(d, 1, 2)};
+    if (fused_operator(d)) {
+        HIP_TRY(launch_force_exact_operator(d->stream, exact_lists(d), F_NEED_K0, a, t, va, dy));
+        return RD_OK;
+    }
+    HIP_TRY(enqueue_force(d, d->P[0][0], d->P[0][1], d->P[0][2], F_NEED_K0));
+    HIP_TRY(launch_operator(d->stream, a, t, va, dy));
+    return RD_OK;
+}
+
 // One attempt for every disk whose ctl flags say so; with commit_advance >= 0
 // (fixed-step chains) the commit follows in the same sequence.
 hipError_t enqueue_attempt(rd_integrator* it, int commit_advance)
 {
     rd_disk* d = it->d;
     hipError_t e;
-    // FP64, one small gas-free disk (4- or 8-sink items: launches, not pairs, set
-    // the time), fixed-step RK4: each stage is done by the summing lanes of
-    // its FP64 pair pass (launch_force_exact_rk4), which hold every body's
-    // complete sum; the same operations in the same order as pair pass + stage
-    // kernel, one launch per stage instead of two
-    if (d->precision == RD_PREC_FP64 && (d->exact_sinks == 4 || d->exact_sinks == 8) && d->n_disk == 1 &&
-        d->gas.on == kGasNone && it->method == RD_RK4 && !it->adaptive) {
-        // the last stage also commits (k_commit's copy and time advance): its
-        // summing lanes cover every body, and no pair term of that launch reads y_n
+    if (fused_stages(it)) {
         for (int r = 0; r <= last_stage(it); ++r) {
             StageArgs a = make_args(d, r, it->adaptive, it->err_all);
-            a.fuse_comb1 = r == 0;   // stage 0 forms stage 1 itself, as in the separate kernel
-            if (r == last_stage(it)) a.commit = commit_advance;
-            if ((e = launch_force_exact_rk4(d->stream, d->exact_sinks, r, d->items_force, d->n_items_force,
-                                            d->grid_force, a.fpos[0], a.fpos[1], a.fpos[2], d->m_ex, d->mass_odd,
-                                            d->ctl, r == 0 ? F_K0_FORCE : F_ACTIVE, a)) != hipSuccess)
+            if (it->method == RD_RK4) {
+                a.fuse_comb1 = r == 0;   // stage 0 forms stage 1 itself, as in the separate kernel
+                // the last stage also commits (k_commit's copy and time advance): its
+                // summing lanes cover every body, and no pair term of that launch reads y_n
+                if (r == last_stage(it)) a.commit = commit_advance;
+            }
+            if ((e = launch_force_exact_stage(d->stream, exact_lists(d), it->method, r,
+                                              r == 0 ? F_K0_FORCE : F_ACTIVE, a)) != hipSuccess)
                 return e;
+            if (r == 0 && it->method == RD_RKF78 && (e = launch_comb1(d->stream, it->method, a)) != hipSuccess)
+                return e;
+        }
+        if (it->method == RD_RKF78 && commit_advance >= 0) {
+            StageArgs a = make_args(d, 0, it->adaptive, it->err_all);
+            return launch_commit(d->stream, a, commit_advance, d->ctl);
         }
         return hipSuccess;
     }
@@ -1131,27 +1200,15 @@ int rd_calc_dydx(rd_disk* d, uint32_t k, uint32_t i, uint32_t rr, double t, cons
     }
     if (i != 1) return fail(RD_EINVAL, "Parameter 'i' is out of range.");
     if (int rc = ensure_lists(d)) return rc;
-    // positions into P[0], velocities into the stage-1 velocity slot
-    std::vector<double> buf(h.n);
-    double* dst[6] = {d->P[0][0], d->P[0][1], d->P[0][2], kv_ptr(d, 1, 0), kv_ptr(d, 1, 1), kv_ptr(d, 1, 2)};
-    for (int c = 0; c < 6; ++c) {
-        const rd_var4* src = c < 3 ? r : v;
-        for (uint32_t q = 0; q < h.n; ++q) buf[q] = c % 3 == 0 ? src[q].x : (c % 3 == 1 ? src[q].y : src[q].z);
-        HIP_TRY(hipMemcpyAsync(dst[c] + h.off, buf.data(), h.n * sizeof(double), hipMemcpyHostToDevice, d->stream));
-        HIP_TRY(hipStreamSynchronize(d->stream));
-    }
-    for (uint32_t q = 0; q < d->n_disk; ++q) d->h_ctl[q] = DiskCtl{d->hd[q].t, 0.0, q == k ? F_NEED_K0 : 0u, 0};
-    HIP_TRY(hipMemcpyAsync(d->ctl, d->h_ctl, d->n_disk * sizeof(DiskCtl), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(enqueue_force(d, d->P[0][0], d->P[0][1], d->P[0][2], F_NEED_K0));
-    StageArgs a = make_args(d, 2, 0, 0);   // fx = P[0]
-    HIP_TRY(launch_operator(d->stream, a, t, k, ka_ptr(d, 0, 0), ka_ptr(d, 0, 1), ka_ptr(d, 0, 2), kv_ptr(d, 1, 0),
-                            kv_ptr(d, 1, 1), kv_ptr(d, 1, 2)));
-    std::vector<double> ax(h.n), ay(h.n), az(h.n);
-    HIP_TRY(hipMemcpyAsync(ax.data(), ka_ptr(d, 0, 0) + h.off, h.n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipMemcpyAsync(ay.data(), ka_ptr(d, 0, 1) + h.off, h.n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipMemcpyAsync(az.data(), ka_ptr(d, 0, 2) + h.off, h.n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
+    // records staged in k rows, which hold nothing between attempts (6 components
+    // a body each, where a record takes 4)
+    double *const dr = kv_ptr(d, 2, 0), *const dv = kv_ptr(d, 3, 0), *const dd = kv_ptr(d, 4, 0);
+    const size_t bytes = h.n * sizeof(rd_var4);
+    HIP_TRY(hipMemcpyAsync(dr, r, bytes, hipMemcpyHostToDevice, d->stream));
+    HIP_TRY(hipMemcpyAsync(dv, v, bytes, hipMemcpyHostToDevice, d->stream));
+    if (int rc = enqueue_operator(d, k, t, dr, dv, dd)) return rc;
+    HIP_TRY(hipMemcpyAsync(dy, dd, bytes, hipMemcpyDeviceToHost, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
-    for (uint32_t q = 0; q < h.n; ++q) dy[q] = rd_var4{ax[q], ay[q], az[q], 0.0};
     return RD_OK;
 }
 
@@ -1193,19 +1250,9 @@ int rd_calc_dydx_device(rd_disk* d, uint32_t k, uint32_t i, uint32_t rr, double 
     }
     if (int rc = check_device_var4(d, r, h.n, "r")) return rc;
     if (int rc = ensure_lists(d)) return rc;
-    // positions into P[0], velocities into the stage-1 velocity slot, as rd_calc_dydx
-    double* const p[3] = {d->P[0][0] + h.off, d->P[0][1] + h.off, d->P[0][2] + h.off};
-    double* const vel[3] = {kv_ptr(d, 1, 0) + h.off, kv_ptr(d, 1, 1) + h.off, kv_ptr(d, 1, 2) + h.off};
-    HIP_TRY(launch_var4_split(d->stream, h.n, reinterpret_cast<const double*>(r), reinterpret_cast<const double*>(v),
-                              p, vel));
-    for (uint32_t q = 0; q < d->n_disk; ++q) d->h_ctl[q] = DiskCtl{d->hd[q].t, 0.0, q == k ? F_NEED_K0 : 0u, 0};
-    HIP_TRY(hipMemcpyAsync(d->ctl, d->h_ctl, d->n_disk * sizeof(DiskCtl), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(enqueue_force(d, d->P[0][0], d->P[0][1], d->P[0][2], F_NEED_K0));
-    StageArgs a = make_args(d, 2, 0, 0);   // fx = P[0]
-    HIP_TRY(launch_operator(d->stream, a, t, k, ka_ptr(d, 0, 0), ka_ptr(d, 0, 1), ka_ptr(d, 0, 2), kv_ptr(d, 1, 0),
-                            kv_ptr(d, 1, 1), kv_ptr(d, 1, 2)));
-    const double* const acc[3] = {ka_ptr(d, 0, 0) + h.off, ka_ptr(d, 0, 1) + h.off, ka_ptr(d, 0, 2) + h.off};
-    HIP_TRY(launch_var4_join(d->stream, h.n, acc, reinterpret_cast<double*>(dy)));
+    if (int rc = enqueue_operator(d, k, t, reinterpret_cast<const double*>(r), reinterpret_cast<const double*>(v),
+                                  reinterpret_cast<double*>(dy)))
+        return rc;
     HIP_TRY(hipStreamSynchronize(d->stream));
     return RD_OK;
 }
@@ -1597,7 +1644,7 @@ static int step_disks(rd_integrator* it, const std::vector<uint32_t>& want, bool
             n_new += need_k0[k];
         }
         it->force_evals += (uint64_t)(last_stage(it)) + (n_new ? 1 : 0);
-        const size_t nw = 3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock);
+        const size_t nw = error_words(it);
         if (it->adaptive && nd == 1)   // single disk: one error slot per wave of the last stage
             HIP_TRY(hipMemcpyAsync(d->h_errw, d->errw, nw * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                                    d->stream));
@@ -1610,7 +1657,7 @@ static int step_disks(rd_integrator* it, const std::vector<uint32_t>& want, bool
                                   it->tol, it->reject_nonfinite ? 1 : 0));
             StageArgs ca = make_args(d, 0, it->adaptive, it->err_all);
             HIP_TRY(launch_commit(d->stream, ca, 0, d->ctl));
-            HIP_TRY(enqueue_force(d, d->x, d->y, d->z, F_SPEC_K0));
+            HIP_TRY(enqueue_k0_ahead(it));
             HIP_TRY(hipEventSynchronize(d->ev_err));
         } else {
             HIP_TRY(hipStreamSynchronize(d->stream));

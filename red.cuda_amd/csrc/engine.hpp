@@ -167,13 +167,20 @@ hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, const WorkItem* ite
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
                               uint32_t n_all);
-// The FP64 pair pass (4- or 8-sink items) of single-disk, gas-free, fixed-step
-// RK4 stage r (0-3) with the stage combination done by the kernel's summing
-// lanes (no stage kernel, no partial-sum slot).
-hipError_t launch_force_exact_rk4(hipStream_t s, uint32_t sinks, int r, const WorkItem* items, uint32_t n_items,
-                                  uint32_t grid, const double* x, const double* y, const double* z,
-                                  const double* m_ex, const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need,
-                                  const StageArgs& a);
+// The FP64 pair pass on 4- or 8-sink items with what follows the sums done by the
+// kernel's summing lanes (no stage kernel, no partial-sum slot): stage r of a single
+// gas-free disk's RKF7(8) (method 4, 0-12) or fixed-step RK4 (0-3), or the operator on
+// disk a.info0 (launch_operator's work; with gas, 4-sink items only).
+struct ExactLists {
+    const WorkItem* items;
+    uint32_t n_items, grid, sinks;
+    const double* m_ex;
+    const uint32_t* mass_odd;
+};
+hipError_t launch_force_exact_stage(hipStream_t s, const ExactLists& l, int method, int r, uint32_t need,
+                                    const StageArgs& a);
+hipError_t launch_force_exact_operator(hipStream_t s, const ExactLists& l, uint32_t need, const StageArgs& a,
+                                       double t, const double* const vel[3], double* dy);
 // Mixed precision: the symmetric kernel's (chunk a, chunk c) items -- sink_lo/hi =
 // chunk a, src_lo/hi = chunk c (256-body blocks, R per chunk), slot = c (sink
 // side), src_slot = a (source side); self: some item carries kItemSelf (the
@@ -198,12 +205,12 @@ hipError_t launch_commit(hipStream_t s, const StageArgs& a, int advance_time, Di
 // F_MORE was set, on accepted disks; clears every other flag.
 hipError_t launch_decide(hipStream_t s, const unsigned long long* errw, uint32_t nw, const unsigned long long* err,
                          uint32_t n_disk, DiskCtl* ctl, double lambda, double tol, int nonfinite_guard);
-hipError_t launch_operator(hipStream_t s, const StageArgs& a, double t, uint32_t disk, double* ax, double* ay,
-                           double* az, const double* vx, const double* vy, const double* vz);
-// var4 records (x, y, z, w) <-> component arrays, for calc_dydx on device arrays
-hipError_t launch_var4_split(hipStream_t s, uint32_t n, const double* r, const double* v, double* const p[3],
-                             double* const vel[3]);
-hipError_t launch_var4_join(hipStream_t s, uint32_t n, const double* const a[3], double* dy);
+// calc_dydx on device arrays: var4 records (x, y, z, w) into component arrays,
+// and the control flags of a pass over `disk` alone; then, after the pair pass,
+// the accelerations of disk a.info0 as var4 records
+hipError_t launch_operator_begin(hipStream_t s, uint32_t n, const double* r, const double* v, double* const p[3],
+                                 double* const vel[3], DiskCtl* ctl, uint32_t n_disk, uint32_t disk);
+hipError_t launch_operator(hipStream_t s, const StageArgs& a, double t, const double* const vel[3], double* dy);
 hipError_t launch_collision_grid(hipStream_t s, uint32_t n_all, const double* x, const double* y, const double* z,
                                  const double* radius, const int32_t* id, const uint32_t* disk_of,
                                  const DiskCtl* ctl, double f, uint32_t table, uint32_t* head, uint32_t* next,

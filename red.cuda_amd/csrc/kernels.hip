@@ -117,6 +117,8 @@ __host__ __device__ constexpr double rk4_c(int r) { return (r == 1 || r == 2) ? 
 constexpr uint32_t exact_tile(uint32_t kS) { return kS >= 12 ? 32u : 128u; }
 constexpr uint32_t exact_term_waves(uint32_t kS) { return kS >= 12 ? 3u : 4u; }
 constexpr uint32_t exact_sum_waves(uint32_t kS) { return kS >= 12 ? 1u : 3u * kS / 4u; }
+constexpr uint32_t kRowSumTermWaves = exact_term_waves(4);   // items of 4 and 8 sinks
+static_assert(exact_term_waves(8) == kRowSumTermWaves, "one count for the fused stages");
 constexpr int exact_block(uint32_t kS) { return 64 * (int)(exact_term_waves(kS) + exact_sum_waves(kS)); }
 
 // sum += the row's 8 terms v of lanes 8 H .. 8 H + 7, in order (row: 16 lanes).
@@ -220,33 +222,34 @@ __device__ __forceinline__ double exact_scale_any(double r2, double m, bool self
     return m / (sqrt(r2) * r2);
 }
 
-// What the summing lane of (body i, component q) needs for RK4 stage R of a
-// single gas-free disk, loaded before the pair sums so that the loads overlap
-// them, and the stage itself (defined with the stage kernels below).
-struct Rk4Lane {
-    DiskCtl c;
-    double yy, vv, kk, k0v, k1v, k2v, k0a, k1a, k2a;
-    int id;
+// What becomes of a body's complete sum, in the summing lane that holds component
+// q of body i.  load() is called by the lane that owns the sum, before the
+// pair sums, so that its loads overlap them, finish() after them by that lane, or
+// with kWave by every lane of the summing waves.  Stored in the partial-sum slot here; the fused stages are
+// defined with the stage kernels below.
+struct StoreSum {
+    double* part;
+    uint32_t n_all;
+    static constexpr bool kWave = false;
+    struct Lane {};
+    __device__ __forceinline__ void load(uint32_t, int, Lane&) const {}
+    __device__ __forceinline__ void finish(bool, uint32_t i, int q, uint32_t slot, const Lane&, double sum) const
+    {
+        part[(size_t)(slot * 3 + q) * n_all + i] = sum;
+    }
 };
-template <int R>
-__device__ void rk4_lane_load(const StageArgs& a, uint32_t i, int q, Rk4Lane& s);
-template <int R>
-__device__ void rk4_lane_finish(const StageArgs& a, uint32_t i, int q, const Rk4Lane& s, double ps);
-struct NoStage {};
 
-// FR < 0: each summing lane stores its sum in the partial-sum slot.  FR >= 0
-// (a single gas-free disk, fixed-step RK4, FP64): the lane holds body si's complete
-// component-sc_c sum -- the value the stage kernel would read back from that
-// slot -- and runs stage FR for the body itself: it reads only that body's
-// state and k rows and writes the other position buffer, which no pair term
-// of this launch reads.
-template <uint32_t kS, int FR, typename SA>
+// Fin: what follows the sum.  The fused ones (single disk, 4- or 8-sink items) run
+// the stage for the body in the lane that holds its sum, the value the stage
+// kernel would read back from the slot: it reads only that body's state and k
+// rows and writes the other position buffer, which no pair term of this launch
+// reads.
+template <uint32_t kS, typename Fin>
 __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ items, uint32_t n_items,
                                                  const double* __restrict__ x, const double* __restrict__ y,
                                                  const double* __restrict__ z, const double* __restrict__ m_ex,
                                                  const uint32_t* __restrict__ mass_odd,
-                                                 const DiskCtl* __restrict__ ctl, uint32_t need,
-                                                 double* __restrict__ part, uint32_t n_all, const SA& sa)
+                                                 const DiskCtl* __restrict__ ctl, uint32_t need, const Fin& fin)
 {
     constexpr uint32_t kTile = exact_tile(kS);
     constexpr uint32_t kTermers = 64 * exact_term_waves(kS);
@@ -302,19 +305,21 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
         const WorkItem w = items[it];
         const uint32_t si = w.sink_lo + sc_g;  // sink of a summing lane
-        // the lane that stores the sum
+        // the lane that owns the sum
         const bool owner = !termer && (kRowSum ? sc_k == 0 : sl < 3 * kS) && si < w.sink_hi;
+        typename Fin::Lane lane;
         auto finish = [&](double sum) {
-            if constexpr (FR >= 0) {
-                Rk4Lane lane;
-                rk4_lane_load<FR>(sa, si, (int)sc_c, lane);
-                rk4_lane_finish<FR>(sa, si, (int)sc_c, lane, sum);
+            if constexpr (Fin::kWave) {
+                if (!termer) fin.finish(owner, si, (int)sc_c, w.slot, lane, sum);
             } else {
-                part[(size_t)(w.slot * 3 + sc_c) * n_all + si] = sum;
+                if (owner) fin.finish(true, si, (int)sc_c, w.slot, lane, sum);
             }
         };
         if (w.src_hi <= w.src_lo) {   // no sources: the sums are zero
-            if ((ctl[w.disk].flags & need) && owner) finish(0.0);
+            if (ctl[w.disk].flags & need) {
+                if (owner) fin.load(si, (int)sc_c, lane);
+                finish(0.0);
+            }
             continue;
         }
         // the item's first loads go out together with the control's.  Source
@@ -339,9 +344,7 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
         if (!(ctl[w.disk].flags & need)) continue;
         const uint32_t n_src = w.src_hi - w.src_lo;
         const uint32_t n_tiles = (n_src + kTile - 1) / kTile;
-        Rk4Lane lane;
-        if constexpr (FR >= 0)
-            if (owner) rk4_lane_load<FR>(sa, si, (int)sc_c, lane);
+        if (owner) fin.load(si, (int)sc_c, lane);
         double acc = 0.0;
         // the first cnt terms of the tile's row tr in order, rounded up to 32 or
         // 8 (padding adds zeros)
@@ -442,10 +445,7 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
                 if (t < n_tiles) tile(t + 1, 1u, sj_odd);
             }
         }
-        if (owner) {
-            if constexpr (FR >= 0) rk4_lane_finish<FR>(sa, si, (int)sc_c, lane, acc);
-            else finish(acc);
-        }
+        finish(acc);
     }
 }
 
@@ -463,21 +463,7 @@ void k_force_exact(const WorkItem* __restrict__ items, uint32_t n_items,
                                                              const DiskCtl* __restrict__ ctl, uint32_t need,
                                                              double* __restrict__ part, uint32_t n_all)
 {
-    force_exact_body<kS, -1>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, part, n_all, NoStage{});
-}
-
-// The FP64 pair pass of RK4 stage R with the stage itself done by the summing lanes.
-template <uint32_t kS, int R>
-__global__ __launch_bounds__(exact_block(kS)) void k_force_exact_rk4(const WorkItem* __restrict__ items,
-                                                                 uint32_t n_items, const double* __restrict__ x,
-                                                                 const double* __restrict__ y,
-                                                                 const double* __restrict__ z,
-                                                                 const double* __restrict__ m_ex,
-                                                                 const uint32_t* __restrict__ mass_odd,
-                                                                 const DiskCtl* __restrict__ ctl, uint32_t need,
-                                                                 StageArgs sa)
-{
-    force_exact_body<kS, R>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, nullptr, sa.n_all, sa);
+    force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, StoreSum{part, n_all});
 }
 
 // The same sum with one sink per lane, each lane adding its terms in j order
@@ -1149,25 +1135,6 @@ hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* it
     case 18: EXACT_LAUNCH(k_force_exact<18>, exact_block(18), part, n_all); break;
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
-}
-
-hipError_t launch_force_exact_rk4(hipStream_t st, uint32_t sinks, int r, const WorkItem* items, uint32_t n_items,
-                                  uint32_t grid, const double* x, const double* y, const double* z,
-                                  const double* m_ex, const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need,
-                                  const StageArgs& a)
-{
-    if (n_items == 0) return hipSuccess;
-    if (r < 0 || r > 3 || (sinks != 4 && sinks != 8)) return hipErrorInvalidValue;
-#define EXACT_RK4(R)                                                                            \
-    case R:                                                                                     \
-        if (sinks == 4) EXACT_LAUNCH((k_force_exact_rk4<4, R>), exact_block(4), a);             \
-        else EXACT_LAUNCH((k_force_exact_rk4<8, R>), exact_block(8), a);                        \
-        break;
-    switch (r) {
-        EXACT_RK4(0) EXACT_RK4(1) EXACT_RK4(2) EXACT_RK4(3)
-    }
-#undef EXACT_RK4
 #undef EXACT_LAUNCH
     return hipGetLastError();
 }
@@ -1438,6 +1405,26 @@ __device__ double prefix_accel(const StageArgs& a, uint32_t i, int q, const Disk
     return b;
 }
 
+// Component q of the drag on body i at time t; false if the gas does not act on
+// it.  pos: force-input positions; vel: velocities of this stage.
+__device__ __forceinline__ bool drag_on(const StageArgs& a, uint32_t i, int q, const DiskInfo& di, double t,
+                                        const double* __restrict__ const* pos, const double* __restrict__ const* vel,
+                                        double& f)
+{
+    const uint32_t li = i - di.off;
+    if (a.gas.on == kGasNone || li < di.drag_lo || li >= di.drag_hi) return false;
+    if (a.gas.on == kGasAnalytic) {
+        const double decr = reduction_factor(a.gas, t);
+        if (1.0e-6 > decr) return false;
+        f = drag_component(a.gas, decr, a.mass[di.off], pos[0][i], pos[1][i], pos[2][i], vel[0][i], vel[1][i],
+                           vel[2][i], a.cd[i], a.radius[i], a.density[i], q);
+    } else {
+        f = grid_drag_component(a.gas, a.mass[di.off], pos[0][i], pos[1][i], vel[0][i], vel[1][i], vel[2][i],
+                                a.cd[i], a.radius[i], a.density[i], q);
+    }
+    return true;
+}
+
 // Component q of the acceleration of body i at this stage from the FP64
 // prefix part b and the summed partials s: b + s in mixed mode, zero for
 // inactive sinks, plus drag.  pos: force-input positions; vel: velocities of
@@ -1445,18 +1432,10 @@ __device__ double prefix_accel(const StageArgs& a, uint32_t i, int q, const Disk
 __device__ double stage_accel(const StageArgs& a, uint32_t i, int q, const DiskInfo& di, double t, double b, double s,
                               const double* __restrict__ const* pos, const double* __restrict__ const* vel)
 {
-    const uint32_t li = i - di.off;
     if (a.mixed) s = b + s;
     if (!(a.id[i] > 0)) s = 0.0;
-    if (a.gas.on == kGasAnalytic && li >= di.drag_lo && li < di.drag_hi) {
-        const double decr = reduction_factor(a.gas, t);
-        if (!(1.0e-6 > decr))
-            s += drag_component(a.gas, decr, a.mass[di.off], pos[0][i], pos[1][i], pos[2][i], vel[0][i], vel[1][i],
-                                vel[2][i], a.cd[i], a.radius[i], a.density[i], q);
-    } else if (a.gas.on == kGasGrid && li >= di.drag_lo && li < di.drag_hi) {
-        s += grid_drag_component(a.gas, a.mass[di.off], pos[0][i], pos[1][i], vel[0][i], vel[1][i], vel[2][i],
-                                 a.cd[i], a.radius[i], a.density[i], q);
-    }
+    double f;
+    if (drag_on(a, i, q, di, t, pos, vel, f)) s += f;
     return s;
 }
 
@@ -1535,11 +1514,11 @@ __device__ void error_reduce(const StageArgs& a, bool valid, uint32_t d, double 
 }
 
 // Single-disk form of error_reduce: the wave's max goes to its own slot,
-// a.errw[blockIdx.y * gridDim.x + blockIdx.x] (one wave per block), with the
+// a.errw[slot], with the
 // non-finite flag in bit 63 (free: a non-negative double's bits are below it),
 // and the host takes the max of the slots.  One same-address atomic per wave
 // would serialise hundreds of waves on one word.
-__device__ void error_store_wave(const StageArgs& a, bool valid, double e)
+__device__ void error_store_wave(const StageArgs& a, bool valid, double e, uint32_t slot)
 {
     unsigned long long bits = (valid && e == e) ? (unsigned long long)__double_as_longlong(e) : 0ull;
     const bool bad = valid && !(e <= DBL_MAX);
@@ -1548,7 +1527,7 @@ __device__ void error_store_wave(const StageArgs& a, bool valid, double e)
         bits = o > bits ? o : bits;
     }
     if (__any(bad)) bits |= kErrNonFinite;
-    if ((threadIdx.x & 63u) == 0) a.errw[blockIdx.y * gridDim.x + blockIdx.x] = bits;
+    if ((threadIdx.x & 63u) == 0) a.errw[slot] = bits;
 }
 
 // Stage kernels over a single disk (ONE = true).  The disk's info comes in
@@ -1579,6 +1558,72 @@ __device__ __forceinline__ void one_disk_sums(const StageArgs& a, uint32_t i, in
     b = prefix_accel(a, i, q, di, a.fpos, &s0);
 }
 
+// Body i's values that RKF7(8) stage R combines, component q, and the stage from
+// them: at(p) is where the result for array p goes.  Returns the body's error
+// term (stage 12).
+template <int R>
+struct Rk8Rows {
+    static constexpr int NR = (R >= 1 && R <= 9) ? R + 1 : (R == 10 ? 11 : (R == 11 ? 12 : 1));
+    double yy, vv, kk;
+    double kv[9], ka[9];
+    double y10v[6], y10a[6];
+    double e0v, e10v, e11v, e0a, e10a, e11a;
+
+    __device__ __forceinline__ void load(const StageArgs& a, uint32_t i, int q)
+    {
+        yy = a.pos[q][i];
+        vv = a.vel[q][i];
+        kk = kv_of(a, R, q)[i];
+        if constexpr (R >= 1 && R <= 11) rk8_load_row<NR, R>(a, i, q, kv, ka);
+        if constexpr (R == 10) {
+            const int cols[6] = {0, 5, 6, 7, 8, 9};
+#pragma unroll
+            for (int u = 0; u < 6; ++u) {
+                y10v[u] = kv_of(a, cols[u], q)[i];
+                y10a[u] = ka_of(a, cols[u], q)[i];
+            }
+        }
+        if constexpr (R == 12) {
+            e0v = kv_of(a, 0, q)[i]; e10v = kv_of(a, 10, q)[i]; e11v = kv_of(a, 11, q)[i];
+            e0a = ka_of(a, 0, q)[i]; e10a = ka_of(a, 10, q)[i]; e11a = ka_of(a, 11, q)[i];
+        }
+    }
+    template <typename At>
+    __device__ __forceinline__ double finish(const StageArgs& a, int q, double h, double kRa, At at)
+    {
+        *at(ka_w(a, R, q)) = kRa;
+        if constexpr (R >= 1 && R <= 9) {
+            double p, w;
+            rk8_comb_q<NR, R>(yy, vv, h, kv, ka, kk, kRa, p, w);
+            *at(a.npos[q]) = p;
+            *at(kv_w(a, NR, q)) = w;
+        } else if constexpr (R == 10) {
+            // y_{n+1} = y + h (b0 k0 + b5 k5 + b6 (k6 + k7) + b8 (k8 + k9) + b10 k10) (int_rungekutta8.cu:264-274)
+            constexpr double b0 = 41.0 / 840.0, b5 = 34.0 / 105.0, b6 = 9.0 / 35.0, b8 = 9.0 / 280.0,
+                             b10 = 41.0 / 840.0;
+            *at(a.out[q]) = yy + h * (b0 * y10v[0] + b5 * y10v[1] + b6 * (y10v[2] + y10v[3]) +
+                                     b8 * (y10v[4] + y10v[5]) + b10 * kk);
+            *at(a.out[3 + q]) = vv + h * (b0 * y10a[0] + b5 * y10a[1] + b6 * (y10a[2] + y10a[3]) +
+                                         b8 * (y10a[4] + y10a[5]) + b10 * kRa);
+            if (a.adaptive) {
+                double p, w;
+                rk8_comb_q<11, R>(yy, vv, h, kv, ka, kk, kRa, p, w);
+                *at(a.npos[q]) = p;
+                *at(kv_w(a, 11, q)) = w;
+            }
+        } else if constexpr (R == 11) {
+            double p, w;
+            rk8_comb_q<12, R>(yy, vv, h, kv, ka, kk, kRa, p, w);
+            *at(a.npos[q]) = p;
+            *at(kv_w(a, 12, q)) = w;
+        } else if constexpr (R == 12) {
+            // |f0 + f10 - f11 - f12| (int_rungekutta8.cu:250-260)
+            return fmax(fabs(e0v + e10v - e11v - kk), fabs(e0a + e10a - e11a - kRa));
+        }
+        return 0.0;
+    }
+};
+
 // RKF7(8) stage R over a single disk.
 template <int R>
 __device__ __forceinline__ void stage_rk8_one(const StageArgs& a)
@@ -1591,25 +1636,8 @@ __device__ __forceinline__ void stage_rk8_one(const StageArgs& a)
     const DiskCtl c = a.ctl[0];
     if constexpr (R == 0)
         if (!(c.flags & F_NEED_K0)) return;
-    const double yy = a.pos[q][i], vv = a.vel[q][i];
-    const double kk = kv_of(a, R, q)[i];
-    constexpr int NR = (R >= 1 && R <= 9) ? R + 1 : (R == 10 ? 11 : (R == 11 ? 12 : 1));
-    double kv[9], ka[9];
-    if constexpr (R >= 1 && R <= 11) rk8_load_row<NR, R>(a, i, q, kv, ka);
-    double y10v[6], y10a[6];
-    if constexpr (R == 10) {
-        const int cols[6] = {0, 5, 6, 7, 8, 9};
-#pragma unroll
-        for (int u = 0; u < 6; ++u) {
-            y10v[u] = kv_of(a, cols[u], q)[i];
-            y10a[u] = ka_of(a, cols[u], q)[i];
-        }
-    }
-    double e0v = 0, e10v = 0, e11v = 0, e0a = 0, e10a = 0, e11a = 0;
-    if constexpr (R == 12) {
-        e0v = kv_of(a, 0, q)[i]; e10v = kv_of(a, 10, q)[i]; e11v = kv_of(a, 11, q)[i];
-        e0a = ka_of(a, 0, q)[i]; e10a = ka_of(a, 10, q)[i]; e11a = ka_of(a, 11, q)[i];
-    }
+    Rk8Rows<R> rows;
+    rows.load(a, i, q);
     double ps, b;
     one_disk_sums(a, i, q, ps, b);
     const bool valid = in && (c.flags & (R == 0 ? F_NEED_K0 : F_ACTIVE)) != 0;
@@ -1618,41 +1646,47 @@ __device__ __forceinline__ void stage_rk8_one(const StageArgs& a)
     const double* vR[3] = {kv_of(a, R, 0), kv_of(a, R, 1), kv_of(a, R, 2)};
     const double kRa = stage_accel(a, i, q, di, t, b, ps, a.fpos, vR);
     double* const trash = a.trash + (size_t)q * kBodyBlock + threadIdx.x;
-    auto at = [&](double* p) { return valid ? p + i : trash; };
-    *at(ka_w(a, R, q)) = kRa;
-    if constexpr (R >= 1 && R <= 9) {
-        double p, w;
-        rk8_comb_q<NR, R>(yy, vv, h, kv, ka, kk, kRa, p, w);
-        *at(a.npos[q]) = p;
-        *at(kv_w(a, NR, q)) = w;
-    } else if constexpr (R == 10) {
-        // y_{n+1} = y + h (b0 k0 + b5 k5 + b6 (k6 + k7) + b8 (k8 + k9) + b10 k10) (int_rungekutta8.cu:264-274)
-        constexpr double b0 = 41.0 / 840.0, b5 = 34.0 / 105.0, b6 = 9.0 / 35.0, b8 = 9.0 / 280.0,
-                         b10 = 41.0 / 840.0;
-        *at(a.out[q]) = yy + h * (b0 * y10v[0] + b5 * y10v[1] + b6 * (y10v[2] + y10v[3]) +
-                                 b8 * (y10v[4] + y10v[5]) + b10 * kk);
-        *at(a.out[3 + q]) = vv + h * (b0 * y10a[0] + b5 * y10a[1] + b6 * (y10a[2] + y10a[3]) +
-                                     b8 * (y10a[4] + y10a[5]) + b10 * kRa);
-        if (a.adaptive) {
-            double p, w;
-            rk8_comb_q<11, R>(yy, vv, h, kv, ka, kk, kRa, p, w);
-            *at(a.npos[q]) = p;
-            *at(kv_w(a, 11, q)) = w;
-        }
-    } else if constexpr (R == 11) {
-        double p, w;
-        rk8_comb_q<12, R>(yy, vv, h, kv, ka, kk, kRa, p, w);
-        *at(a.npos[q]) = p;
-        *at(kv_w(a, 12, q)) = w;
-    } else if constexpr (R == 12) {
-        const uint32_t li = i - di.off;
-        double e = 0.0;
-        // |f0 + f10 - f11 - f12| (int_rungekutta8.cu:250-260)
-        if (valid && (a.err_all || li < di.err_hi))
-            e = fmax(fabs(e0v + e10v - e11v - kk), fabs(e0a + e10a - e11a - kRa));
-        error_store_wave(a, valid, e);
+    const double e = rows.finish(a, q, h, kRa, [&](double* p) { return valid ? p + i : trash; });
+    if constexpr (R == 12) {
+        const bool counted = valid && (a.err_all || i - di.off < di.err_hi);
+        error_store_wave(a, valid, counted ? e : 0.0, blockIdx.y * gridDim.x + blockIdx.x);
     }
 }
+
+// RKF7(8) stage R of a single disk in the FP64 pair kernel's summing lanes: the
+// operations of stage_rk8_one.  Gas-free only: the drag's powers take 190-256
+// registers and a serial chain that the pair waves would wait for (301 bodies in
+// gas: 14.5 us a stage, 13.6 with the stage kernel's three waves per 64 bodies).
+template <int R>
+struct Rk8Sum {
+    const StageArgs& a;
+    static constexpr bool kWave = R == 12;   // the error's maximum is the wave's
+    struct Lane {
+        Rk8Rows<R> rows;
+        double h;
+        int id;
+    };
+    __device__ __forceinline__ void load(uint32_t i, int q, Lane& s) const
+    {
+        s.id = a.id[i];
+        s.rows.load(a, i, q);
+        s.h = a.ctl[0].h;
+    }
+    __device__ __forceinline__ void finish(bool owner, uint32_t i, int q, uint32_t, Lane& s, double sum) const
+    {
+        double e = 0.0;
+        if (owner) {
+            const double kRa = s.id > 0 ? sum : 0.0;
+            e = s.rows.finish(a, q, s.h, kRa, [&](double* p) { return p + i; });
+            if (!(a.err_all || i - a.info0.off < a.info0.err_hi)) e = 0.0;
+        }
+        // one error slot per summing wave, 3 kS / 4 of them in a block
+        if constexpr (R == 12) {
+            const uint32_t waves = blockDim.x / 64u - kRowSumTermWaves;
+            error_store_wave(a, owner, e, blockIdx.x * waves + threadIdx.x / 64u - kRowSumTermWaves);
+        }
+    }
+};
 
 // RKF7(8) stage kernel for stage R: finishes k_R (partials, FP64 prefix,
 // drag) and forms what the next stage needs from body i's own k values.
@@ -1760,21 +1794,31 @@ __global__ __launch_bounds__(kBodyBlock) void k_stage_rk8(StageArgs a)
 // the stage kernel's (stage_rk4_one); returns early where the stage does not
 // apply.  With gas the drag code would take the registers the pair pass needs.
 template <int R>
-__device__ __forceinline__ void rk4_lane_load(const StageArgs& a, uint32_t i, int q, Rk4Lane& s)
-{
-    static_assert(R >= 0 && R <= 3, "fused stages are the fixed-step ones");
-    s.c = a.ctl[0];
-    s.id = a.id[i];
-    s.yy = a.pos[q][i];
-    s.vv = a.vel[q][i];
-    s.kk = kv_of(a, R, q)[i];
-    if constexpr (R == 3) {
-        s.k0v = kv_of(a, 0, q)[i]; s.k1v = kv_of(a, 1, q)[i]; s.k2v = kv_of(a, 2, q)[i];
-        s.k0a = ka_of(a, 0, q)[i]; s.k1a = ka_of(a, 1, q)[i]; s.k2a = ka_of(a, 2, q)[i];
+struct Rk4Sum {
+    const StageArgs& a;
+    static constexpr bool kWave = false;
+    struct Lane {
+        DiskCtl c;
+        double yy, vv, kk, k0v, k1v, k2v, k0a, k1a, k2a;
+        int id;
+    };
+    __device__ __forceinline__ void load(uint32_t i, int q, Lane& s) const
+    {
+        static_assert(R >= 0 && R <= 3, "fused stages are the fixed-step ones");
+        s.c = a.ctl[0];
+        s.id = a.id[i];
+        s.yy = a.pos[q][i];
+        s.vv = a.vel[q][i];
+        s.kk = kv_of(a, R, q)[i];
+        if constexpr (R == 3) {
+            s.k0v = kv_of(a, 0, q)[i]; s.k1v = kv_of(a, 1, q)[i]; s.k2v = kv_of(a, 2, q)[i];
+            s.k0a = ka_of(a, 0, q)[i]; s.k1a = ka_of(a, 1, q)[i]; s.k2a = ka_of(a, 2, q)[i];
+        }
     }
-}
+    __device__ __forceinline__ void finish(bool, uint32_t i, int q, uint32_t, const Lane& s, double ps) const;
+};
 template <int R>
-__device__ __forceinline__ void rk4_lane_finish(const StageArgs& a, uint32_t i, int q, const Rk4Lane& s, double ps)
+__device__ __forceinline__ void Rk4Sum<R>::finish(bool, uint32_t i, int q, uint32_t, const Lane& s, double ps) const
 {
     const DiskCtl& c = s.c;
     if (!(c.flags & (R == 0 ? F_NEED_K0 : F_ACTIVE))) return;
@@ -1871,7 +1915,7 @@ __device__ __forceinline__ void stage_rk4_one(const StageArgs& a)
         const uint32_t li = i - di.off;
         double e = 0.0;
         if (valid && (a.err_all || li < di.err_hi)) e = fmax(fabs(k3v - kk), fabs(k3a - kRa));   // |f4 - f5|
-        error_store_wave(a, valid, e);
+        error_store_wave(a, valid, e, blockIdx.y * gridDim.x + blockIdx.x);
     }
 }
 
@@ -2087,22 +2131,125 @@ hipError_t launch_decide(hipStream_t s, const unsigned long long* errw, uint32_t
     return hipGetLastError();
 }
 
-// pp_disk::calc_dydx(1, ...) for one disk: acceleration at time t from the
-// partials, written to acc[q].
-__global__ __launch_bounds__(kBodyBlock) void k_operator(StageArgs a, double t, uint32_t disk, double* ax,
-                                                         double* ay, double* az, const double* vx, const double* vy,
-                                                         const double* vz)
+// pp_disk::calc_dydx(1, ...) for one disk (a.info0): accelerations at time t from
+// the partials, written as var4 records (w = 0).  a.fpos and vel: the caller's
+// positions and velocities.  The slots are read as in the single-disk stages
+// (9001 bodies of all classes: 20 us with dependent loads of the disk's info).
+__global__ __launch_bounds__(kBodyBlock) void k_operator(StageArgs a, double t, const double* vx, const double* vy,
+                                                         const double* vz, double* dy)
 {
-    const DiskInfo di = a.info[disk];
-    const uint32_t li = blockIdx.x * kBodyBlock + threadIdx.x;
+    const DiskInfo& di = a.info0;
+    const uint32_t l0 = blockIdx.x * kBodyBlock + threadIdx.x;
+    const uint32_t li = min(l0, di.n - 1u);
     const int q = blockIdx.y;
-    if (li >= di.n) return;
     const uint32_t i = di.off + li;
     const double* vel[3] = {vx, vy, vz};
-    const double b = prefix_accel(a, i, q, di, a.fpos);
-    const double s = stage_accel(a, i, q, di, t, b, partial_sum(a, i, q, nchunk_of(di, i)), a.fpos, vel);
-    (q == 0 ? ax : (q == 1 ? ay : az))[i] = s;
+    double ps, b;
+    one_disk_sums(a, i, q, ps, b);
+    const double s = stage_accel(a, i, q, di, t, b, ps, a.fpos, vel);
+    if (l0 >= di.n) return;
+    dy[4 * (size_t)li + q] = s;
+    if (q == 0) dy[4 * (size_t)li + 3] = 0.0;
 }
+
+// k_operator's work in the FP64 pair kernel's summing lanes.
+template <bool kGas>
+struct OperatorSum {
+    const StageArgs& a;
+    double t;
+    const double *vx, *vy, *vz;
+    double* dy;
+    static constexpr bool kWave = false;
+    struct Lane {
+        double f;
+        int id;
+        bool drag;
+    };
+    __device__ __forceinline__ void load(uint32_t i, int q, Lane& s) const
+    {
+        const double* vel[3] = {vx, vy, vz};
+        s.id = a.id[i];
+        if constexpr (kGas) s.drag = drag_on(a, i, q, a.info0, t, a.fpos, vel, s.f);
+    }
+    __device__ __forceinline__ void finish(bool, uint32_t i, int q, uint32_t, const Lane& s, double sum) const
+    {
+        const uint32_t li = i - a.info0.off;
+        double acc = s.id > 0 ? sum : 0.0;
+        if constexpr (kGas)
+            if (s.drag) acc += s.f;
+        dy[4 * (size_t)li + q] = acc;
+        if (q == 0) dy[4 * (size_t)li + 3] = 0.0;
+    }
+};
+
+// The FP64 pair pass of a single disk's stage (or of the operator) with what
+// follows it done by the summing lanes.
+#define EXACT_ARGS                                                                                               \
+    const WorkItem *__restrict__ items, uint32_t n_items, const double *__restrict__ x,                          \
+        const double *__restrict__ y, const double *__restrict__ z, const double *__restrict__ m_ex,             \
+        const uint32_t *__restrict__ mass_odd, const DiskCtl *__restrict__ ctl, uint32_t need, StageArgs sa
+template <uint32_t kS, int R>
+__global__ __launch_bounds__(exact_block(kS)) void k_force_exact_rk4(EXACT_ARGS)
+{
+    force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, Rk4Sum<R>{sa});
+}
+template <uint32_t kS, int R>
+__global__ __launch_bounds__(exact_block(kS)) void k_force_exact_rk8(EXACT_ARGS)
+{
+    force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, Rk8Sum<R>{sa});
+}
+template <uint32_t kS, bool kGas>
+__global__ __launch_bounds__(exact_block(kS)) void k_force_exact_operator(EXACT_ARGS, double t, const double* vx,
+                                                                          const double* vy, const double* vz,
+                                                                          double* dy)
+{
+    force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, OperatorSum<kGas>{sa, t, vx, vy, vz, dy});
+}
+#undef EXACT_ARGS
+
+#define EXACT_FUSED(KERNEL, S, ...)                                                                                 \
+    hipLaunchKernelGGL(KERNEL, dim3(l.grid), dim3(exact_block(S)), 0, st, l.items, l.n_items, a.fpos[0], a.fpos[1], \
+                       a.fpos[2], l.m_ex, l.mass_odd, a.ctl, need, __VA_ARGS__)
+hipError_t launch_force_exact_stage(hipStream_t st, const ExactLists& l, int method, int r, uint32_t need,
+                                    const StageArgs& a)
+{
+    if (l.n_items == 0) return hipSuccess;
+    if (l.sinks != 4 && l.sinks != 8) return hipErrorInvalidValue;
+    if (a.gas.on != kGasNone) return hipErrorInvalidValue;
+#define EXACT_STAGE(M, R)                                                              \
+    case R:                                                                            \
+        if (l.sinks == 4) EXACT_FUSED((k_force_exact_##M<4, R>), 4, a);                \
+        else EXACT_FUSED((k_force_exact_##M<8, R>), 8, a);                             \
+        break;
+    if (method == 4) {
+        switch (r) {
+            EXACT_STAGE(rk8, 0) EXACT_STAGE(rk8, 1) EXACT_STAGE(rk8, 2) EXACT_STAGE(rk8, 3) EXACT_STAGE(rk8, 4)
+            EXACT_STAGE(rk8, 5) EXACT_STAGE(rk8, 6) EXACT_STAGE(rk8, 7) EXACT_STAGE(rk8, 8) EXACT_STAGE(rk8, 9)
+            EXACT_STAGE(rk8, 10) EXACT_STAGE(rk8, 11) EXACT_STAGE(rk8, 12)
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        switch (r) {
+            EXACT_STAGE(rk4, 0) EXACT_STAGE(rk4, 1) EXACT_STAGE(rk4, 2) EXACT_STAGE(rk4, 3)
+        default: return hipErrorInvalidValue;
+        }
+    }
+#undef EXACT_STAGE
+    return hipGetLastError();
+}
+
+hipError_t launch_force_exact_operator(hipStream_t st, const ExactLists& l, uint32_t need, const StageArgs& a,
+                                       double t, const double* const vel[3], double* dy)
+{
+    if (l.n_items == 0) return hipSuccess;
+    const bool gas = a.gas.on != kGasNone;
+    if (l.sinks != 4 && (gas || l.sinks != 8)) return hipErrorInvalidValue;
+    if (gas) EXACT_FUSED((k_force_exact_operator<4, true>), 4, a, t, vel[0], vel[1], vel[2], dy);
+    else if (l.sinks == 4) EXACT_FUSED((k_force_exact_operator<4, false>), 4, a, t, vel[0], vel[1], vel[2], dy);
+    else EXACT_FUSED((k_force_exact_operator<8, false>), 8, a, t, vel[0], vel[1], vel[2], dy);
+    return hipGetLastError();
+}
+#undef EXACT_FUSED
 
 #define STAGE_CASE(M, R)                                                                   \
     case R:                                                                                \
@@ -2166,25 +2313,25 @@ hipError_t launch_commit(hipStream_t st, const StageArgs& a, int advance, DiskCt
     return hipGetLastError();
 }
 
-hipError_t launch_operator(hipStream_t st, const StageArgs& a, double t, uint32_t disk, double* ax, double* ay,
-                           double* az, const double* vx, const double* vy, const double* vz)
+hipError_t launch_operator(hipStream_t st, const StageArgs& a, double t, const double* const vel[3], double* dy)
 {
-    if (a.n_all == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_operator, body_grid(a.n_all), dim3(kBodyBlock), 0, st, a, t, disk, ax, ay, az, vx, vy, vz);
+    if (a.info0.n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_operator, body_grid(a.info0.n), dim3(kBodyBlock), 0, st, a, t, vel[0], vel[1], vel[2], dy);
     return hipGetLastError();
 }
 
-// calc_dydx on device arrays: the caller's var4 records (x, y, z, w; 32 B)
-// split into the engine's component arrays, and the accelerations joined back
-// into var4 records with w = 0.  Scalar loads and stores: a caller's record
-// array need only be 8-byte aligned.
-__global__ __launch_bounds__(kBodyBlock) void k_var4_split(uint32_t n, const double* __restrict__ r,
-                                                           const double* __restrict__ v, double* __restrict__ px,
-                                                           double* __restrict__ py, double* __restrict__ pz,
-                                                           double* __restrict__ vx, double* __restrict__ vy,
-                                                           double* __restrict__ vz)
+// calc_dydx on device arrays: the caller's var4 records (x, y, z, w; 32 B) split
+// into the engine's component arrays, and the disk's control set, as one
+// launch.  Scalar loads: a caller's record array need only be 8-byte aligned.
+__global__ __launch_bounds__(kBodyBlock) void k_operator_begin(uint32_t n, const double* __restrict__ r,
+                                                               const double* __restrict__ v, double* __restrict__ px,
+                                                               double* __restrict__ py, double* __restrict__ pz,
+                                                               double* __restrict__ vx, double* __restrict__ vy,
+                                                               double* __restrict__ vz, DiskCtl* __restrict__ ctl,
+                                                               uint32_t n_disk, uint32_t disk)
 {
     const uint32_t q = blockIdx.x * kBodyBlock + threadIdx.x;
+    if (q < n_disk) ctl[q].flags = q == disk ? F_NEED_K0 : 0u;
     if (q >= n) return;
     px[q] = r[4 * (size_t)q + 0];
     py[q] = r[4 * (size_t)q + 1];
@@ -2194,32 +2341,13 @@ __global__ __launch_bounds__(kBodyBlock) void k_var4_split(uint32_t n, const dou
     vz[q] = v[4 * (size_t)q + 2];
 }
 
-__global__ __launch_bounds__(kBodyBlock) void k_var4_join(uint32_t n, const double* __restrict__ ax,
-                                                          const double* __restrict__ ay,
-                                                          const double* __restrict__ az, double* __restrict__ dy)
-{
-    const uint32_t q = blockIdx.x * kBodyBlock + threadIdx.x;
-    if (q >= n) return;
-    dy[4 * (size_t)q + 0] = ax[q];
-    dy[4 * (size_t)q + 1] = ay[q];
-    dy[4 * (size_t)q + 2] = az[q];
-    dy[4 * (size_t)q + 3] = 0.0;
-}
-
-hipError_t launch_var4_split(hipStream_t st, uint32_t n, const double* r, const double* v, double* const p[3],
-                             double* const vel[3])
+hipError_t launch_operator_begin(hipStream_t st, uint32_t n, const double* r, const double* v, double* const p[3],
+                                 double* const vel[3], DiskCtl* ctl, uint32_t n_disk, uint32_t disk)
 {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_var4_split, dim3((n + kBodyBlock - 1) / kBodyBlock), dim3(kBodyBlock), 0, st, n, r, v, p[0],
-                       p[1], p[2], vel[0], vel[1], vel[2]);
-    return hipGetLastError();
-}
-
-hipError_t launch_var4_join(hipStream_t st, uint32_t n, const double* const a[3], double* dy)
-{
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_var4_join, dim3((n + kBodyBlock - 1) / kBodyBlock), dim3(kBodyBlock), 0, st, n, a[0], a[1],
-                       a[2], dy);
+    const uint32_t threads = std::max(n, n_disk);
+    hipLaunchKernelGGL(k_operator_begin, dim3((threads + kBodyBlock - 1) / kBodyBlock), dim3(kBodyBlock), 0, st, n, r,
+                       v, p[0], p[1], p[2], vel[0], vel[1], vel[2], ctl, n_disk, disk);
     return hipGetLastError();
 }
 
