@@ -159,7 +159,8 @@ struct rd_disk {
     uint32_t n_items_force = 0, grid_force = 0;
     WorkItem* items_sym = nullptr;   // mixed precision, symmetric SI x SI pairs
     uint32_t n_items_sym = 0, grid_sym = 0, sym_R = 1;
-    bool sym_self = false;           // diagonal tiles with reactions (launch_force_sym)
+    bool sym_self = false;           // diagonal tiles with reactions
+    bool sym_split = false;          // items_sym cut finer (k_force_split)
     // collision grid: bucket heads, per-body list links and cells, largest radius
     uint32_t* coll_head = nullptr;
     uint32_t* coll_next = nullptr;
@@ -656,6 +657,36 @@ int build_lists(rd_disk* d)
     for (auto& q : sym_items) d->sym_self |= (q.second.flags & kItemSelf) != 0;
     std::vector<WorkItem> symv;
     for (auto& q : sym_items) symv.push_back(q.second);
+    // few tiles: cut finer, one block per item
+    double tiles = (double)symv.size();
+    if (d->precision == RD_PREC_MIXED)
+        for (const WorkItem& w : items)
+            tiles += (double)(w.sink_hi - w.sink_lo) * (w.src_hi - w.src_lo) / ((double)kSymBlockBodies * kSymBlockBodies);
+    d->sym_split = !symv.empty() && d->sym_R == 1 && tiles <= kSymSplitTiles;
+    if (d->sym_split) {
+        std::vector<WorkItem> cut;
+        for (const WorkItem& w : symv) {
+            const bool diag = w.sink_lo == w.src_lo;
+            // reactions on a diagonal tile of full rows only, as the whole tile's sweep
+            const uint32_t self = w.sink_hi - w.sink_lo > kSymBlockBodies - 64 ? w.flags & kItemSelf : 0u;
+            for (uint32_t i = w.sink_lo; i < w.sink_hi; i += 64) {
+                WorkItem q = w;
+                q.sink_lo = i;
+                q.sink_hi = std::min(w.sink_hi, i + 64);
+                q.flags = diag ? kItemDiagRow | self : kItemRow;
+                cut.push_back(q);
+            }
+            if (diag) continue;
+            for (uint32_t j = w.src_lo; j < w.src_hi; j += 64) {
+                WorkItem q = w;
+                q.src_lo = j;
+                q.src_hi = std::min(w.src_hi, j + 64);
+                q.flags = kItemReact;
+                cut.push_back(q);
+            }
+        }
+        symv.swap(cut);
+    }
     dev_free(d->items_force);
     dev_free(d->items_sym);
     dev_free(d->items_feat);
@@ -675,7 +706,7 @@ int build_lists(rd_disk* d)
     // the term-parallel FP64 kernel's items are single-pass: a block each, up to 8 per CU
     const uint32_t grid_cap = d->precision == RD_PREC_FP64 && d->exact_sinks != 1 ? 8u * (uint32_t)d->n_cu : maxgrid;
     d->grid_force = std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_force, grid_cap));
-    d->grid_sym = std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_sym, maxgrid));
+    d->grid_sym = d->sym_split ? d->n_items_sym : std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_sym, maxgrid));
     const size_t need = max_chunks * 3 * (size_t)d->n_all;
     if (need > d->part_len) {
         dev_free(d->part);
@@ -746,7 +777,7 @@ hipError_t enqueue_force(rd_disk* d, const double* fx, const double* fy, const d
                                   fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all);
     // mixed precision: FP32 slot totals, in float units of the same buffer
     float* part32 = reinterpret_cast<float*>(d->part);
-    const MixedLists l{d->items_sym,   d->n_items_sym,   d->grid_sym,   d->sym_R,                    d->sym_self,
+    const MixedLists l{d->items_sym,   d->n_items_sym,   d->grid_sym,   d->sym_R, d->sym_self, d->sym_split,
                        d->items_force, d->n_items_force, d->grid_force, (int)d->tuning.sinks_per_lane};
     return launch_force_mixed(d->stream, l, fx, fy, fz, d->m32, d->ctl, need, part32, d->n_all);
 }

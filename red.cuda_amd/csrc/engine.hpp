@@ -93,13 +93,21 @@ struct WorkItem {
     uint32_t src_lo, src_hi;
     uint32_t slot;       // partial-sum slot of the sinks
     uint32_t src_slot;   // symmetric kernel: partial-sum slot of the sources
-    uint32_t flags;      // kItemSelf, kItemNarrow
+    uint32_t flags;      // kItemSelf, kItemNarrow, kItemRow, ...
 };
 // diagonal item whose full-block diagonal tiles take each pair once with its
 // reaction (a disk of at most kSymSelfMaxBlocks blocks)
 constexpr uint32_t kItemSelf = 1u;
 // one-sided item of 64 sinks, one per lane, whatever the launch's sinks per lane
 constexpr uint32_t kItemNarrow = 2u;
+// the symmetric kernel's tiles cut finer (k_force_split)
+constexpr uint32_t kItemRow = 4u, kItemReact = 8u, kItemDiagRow = 16u;
+// A launch of at most this many tiles, its one-sided pairs counted as 65536 a
+// tile, cuts them finer (same bits, so the rule may look at the whole batch).
+// Driver loop, us a step whole -> cut: 1001 bodies (10 tiles) 350 -> 241, 3301 (91)
+// 364 -> 290, 4601 (171) 371 -> 352, 5101 (210) 375 -> 381; 9001 bodies of all classes
+// (78 + 580) 494 -> 526.
+constexpr uint32_t kSymSplitTiles = 180;
 // One-sided items of a disk: chunks are halved (down to one 256-source tile),
 // then the sinks taken one per lane, until the disk has this many items -- two
 // per CU.  A decision of the disk alone: results never depend on the batch.
@@ -189,7 +197,7 @@ hipError_t launch_force_exact_operator(hipStream_t s, const ExactLists& l, uint3
 struct MixedLists {
     const WorkItem* sym;
     uint32_t n_sym, grid_sym, R;
-    bool self;
+    bool self, split;   // split: the items are k_force_split's
     const WorkItem* one;
     uint32_t n_one, grid_one;
     int S;

@@ -1118,6 +1118,222 @@ __global__ __launch_bounds__(kBlock) void k_force_both(const WorkItem* __restric
                             need, part, n_all);
 }
 
+// The symmetric kernel's tiles cut finer, same bits.  A tile is 64 steps of 4
+// rows in each of 4 waves, about 24 instructions a row and step: 10 us on a CU
+// whatever the launch holds, so a disk of few tiles (kSymSplitTiles) waits for one
+// while most CUs are idle.  Its sums come apart without changing an operation:
+//   kItemRow: the sink sums of one row (64 sinks) over the block's four quarters,
+//     one quarter a wave, as sym_sweep's rows;
+//   kItemReact: the reactions of block I on one quarter of block J.  They are
+//     FP32 over 16 steps, then FP64 over the four groups of steps in order:
+//     one group a wave;
+//   kItemDiagRow: a row of a diagonal tile, its sink sums and, with kItemSelf,
+//     its reactions as a quarter (sym_sweep_self's step ranges), which share a slot.
+// Each side computes the pair's distance for itself (17 of the 24 instructions),
+// 8 items of 1.8 us of issue in place of one of 10: worth it while CUs are idle.
+// Star + 1000 protoplanets: 17 -> 9.2 us; 3001 bodies of all classes, one-sided
+// items included: 17.3 -> 9.2.
+constexpr size_t kSplitLds = kSymTile * (sizeof(double2) + sizeof(SrcZM)) + (size_t)4 * 3 * 64 * sizeof(double);
+
+// Offset source - sink in FP32 and the inverse cube of its length, sym_sweep's operations.
+__device__ __forceinline__ void sym_pair(const double2& a, const SrcZM& b, double xi, double yi, double zi, float& dx,
+                                         float& dy, float& dz, float& ri3)
+{
+    dx = (float)(a.x - xi);
+    dy = (float)(a.y - yi);
+    dz = (float)(b.z - zi);
+    float r2 = __builtin_fmaf(dz, dz, kEps2);
+    r2 = __builtin_fmaf(dy, dy, r2);
+    r2 = __builtin_fmaf(dx, dx, r2);
+    const float ri = __builtin_amdgcn_rsqf(r2);
+    ri3 = (ri * ri) * ri;
+}
+
+// Sink sums of one row over steps [u0, u1) of a quarter (kb: tile entry at step 0).
+__device__ __forceinline__ void split_row(const double2* txy, const SrcZM* tzm, uint32_t kb, uint32_t u0, uint32_t u1,
+                                          double xi, double yi, double zi, float& fx, float& fy, float& fz)
+{
+#pragma unroll 4
+    for (uint32_t u = u0; u < u1; ++u) {
+        const double2 a = txy[kb - u];
+        const SrcZM b = tzm[kb - u];
+        float dx, dy, dz, ri3;
+        sym_pair(a, b, xi, yi, zi, dx, dy, dz, ri3);
+        const float scj = b.m * ri3;
+        fx = __builtin_fmaf(scj, dx, fx);
+        fy = __builtin_fmaf(scj, dy, fy);
+        fz = __builtin_fmaf(scj, dz, fz);
+    }
+}
+
+// Reactions of rows [0, n(u)) on a quarter over the 16 steps from u0.
+template <int kS, typename N>
+__device__ __forceinline__ void split_react(const double2* txy, const SrcZM* tzm, uint32_t kb, uint32_t u0,
+                                            const double* xi, const double* yi, const double* zi, const float* mi, N n,
+                                            float& ax, float& ay, float& az)
+{
+#pragma unroll 2
+    for (uint32_t u = u0; u < u0 + 16; ++u) {
+        const double2 a = txy[kb - u];
+        const SrcZM b = tzm[kb - u];
+        float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+#pragma unroll
+        for (int s = 0; s < kS; ++s) {
+            if (!n(s, u)) continue;
+            float dx, dy, dz, ri3;
+            sym_pair(a, b, xi[s], yi[s], zi[s], dx, dy, dz, ri3);
+            const float sci = mi[s] * ri3;
+            sx = __builtin_fmaf(sci, dx, sx);
+            sy = __builtin_fmaf(sci, dy, sy);
+            sz = __builtin_fmaf(sci, dz, sz);
+        }
+        ax = rot_sub(ax, sx);
+        ay = rot_sub(ay, sy);
+        az = rot_sub(az, sz);
+    }
+}
+
+__device__ __forceinline__ void force_split_item(const WorkItem& w, unsigned char* lds, const double* __restrict__ x,
+                                                 const double* __restrict__ y, const double* __restrict__ z,
+                                                 const float* __restrict__ m32, float* __restrict__ part,
+                                                 uint32_t n_all)
+{
+    double2* txy = reinterpret_cast<double2*>(lds);
+    SrcZM* tzm = reinterpret_cast<SrcZM*>(txy + kSymTile);
+    double(*red)[3][64] = reinterpret_cast<double(*)[3][64]>(tzm + kSymTile);   // [4][3][64]
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t n_src = w.src_hi - w.src_lo;
+    // the source block, each quarter twice (kSymTile)
+    if (tid < ((n_src + 63u) & ~63u)) {
+        double2 a = make_double2(0.0, 0.0);
+        SrcZM b{0.0, 0.0f, 0.0f};
+        if (tid < n_src) {
+            const uint32_t j = w.src_lo + tid;
+            a = make_double2(x[j], y[j]);
+            b.z = z[j];
+            b.m = m32[j];
+        }
+        const uint32_t e = (tid & ~63u) * 2u + lane;
+        txy[e] = a;
+        txy[e + 64u] = a;
+        tzm[e] = b;
+        tzm[e + 64u] = b;
+    }
+    const uint32_t kq = 64u + lane;   // tile entry at step 0 of quarter 0
+    auto store = [&](uint32_t slot, uint32_t i, double sx, double sy, double sz) {
+        part[(size_t)(slot * 3 + 0) * n_all + i] = (float)sx;
+        part[(size_t)(slot * 3 + 1) * n_all + i] = (float)sy;
+        part[(size_t)(slot * 3 + 2) * n_all + i] = (float)sz;
+    };
+    // a group's FP32 reactions, by source: lane l holds that on source l - u0 - 15
+    auto put_group = [&](float ax, float ay, float az) {
+        const uint32_t j = (lane - 16u * wave - 15u) & 63u;
+        red[wave][0][j] = (double)ax;
+        red[wave][1][j] = (double)ay;
+        red[wave][2][j] = (double)az;
+    };
+    auto sum_groups = [&](uint32_t c) { return (((0.0 + red[0][c][lane]) + red[1][c][lane]) + red[2][c][lane]) + red[3][c][lane]; };
+    if (w.flags & kItemReact) {
+        double xi[kSymS], yi[kSymS], zi[kSymS];
+        float mi[kSymS], ax = 0.0f, ay = 0.0f, az = 0.0f;
+#pragma unroll
+        for (uint32_t s = 0; s < kSymS; ++s) {   // a whole block: sinks lie below the last one
+            const uint32_t i = w.sink_lo + lane + 64u * s;
+            xi[s] = x[i];
+            yi[s] = y[i];
+            zi[s] = z[i];
+            mi[s] = m32[i];
+        }
+        __syncthreads();
+        split_react<(int)kSymS>(txy, tzm, kq, 16u * wave, xi, yi, zi, mi, [](int, uint32_t) { return true; }, ax, ay,
+                                az);
+        put_group(ax, ay, az);
+        __syncthreads();
+        if (wave == 0 && lane < n_src)
+            store(w.src_slot, w.src_lo + lane, sum_groups(0), sum_groups(1), sum_groups(2));
+        return;
+    }
+    const bool diag = w.flags & kItemDiagRow, self = w.flags & kItemSelf;
+    const uint32_t i = w.sink_lo + lane;
+    const uint32_t ic = min(i, w.sink_hi - 1u);   // lanes past the end repeat the last sink, unstored
+    const double xi = x[ic], yi = y[ic], zi = z[ic];
+    const uint32_t row = (w.sink_lo - w.src_lo) / 64u;   // of a diagonal tile
+    uint32_t u0 = 0, u1 = 64;
+    if (diag && self) switch ((wave - row) & 3u) {   // sym_sweep_self's slots 2, 0, 1 and none
+        case 0: u0 = 1; u1 = 33; break;
+        case 1: break;
+        case 2: u0 = wave < 2u ? 1u : 0u; u1 = u0 + 32u; break;
+        default: u1 = 0;
+        }
+    // a quarter without a source adds nothing
+    if (64u * wave >= n_src) u1 = 0;
+    double rx = 0.0, ry = 0.0, rz = 0.0;
+    if (diag && self) {
+        // rows (W + 3), (W + 2) and W (mod 4) of the block on quarter W = row
+        double xs[3], ys[3], zs[3];
+        float ms[3], ax = 0.0f, ay = 0.0f, az = 0.0f;
+#pragma unroll
+        for (uint32_t s = 0; s < 3; ++s) {
+            const uint32_t q = w.src_lo + lane + 64u * ((row + (s == 2 ? 0u : 3u - s)) & 3u);
+            const bool valid = q < w.src_hi;
+            xs[s] = valid ? x[q] : 0.0;
+            ys[s] = valid ? y[q] : 0.0;
+            zs[s] = valid ? z[q] : 0.0;
+            ms[s] = valid ? m32[q] : 0.0f;
+        }
+        __syncthreads();
+        const uint32_t lo1 = row < 2u ? 1u : 0u;
+        split_react<3>(txy, tzm, 128u * row + kq, 16u * wave, xs, ys, zs, ms,
+                       [lo1](int s, uint32_t u) { return s == 0 || (s == 1 ? u - lo1 < 32u : u - 1u < 31u); }, ax, ay,
+                       az);
+        put_group(ax, ay, az);
+        __syncthreads();
+        if (wave == 0) {
+            rx = sum_groups(0);
+            ry = sum_groups(1);
+            rz = sum_groups(2);
+        }
+    }
+    __syncthreads();
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+    split_row(txy, tzm, 128u * wave + kq, u0, u1, xi, yi, zi, fx, fy, fz);
+    red[wave][0][lane] = 0.0 + (double)fx;
+    red[wave][1][lane] = 0.0 + (double)fy;
+    red[wave][2][lane] = 0.0 + (double)fz;
+    __syncthreads();
+    if (wave == 0 && i < w.sink_hi) {
+        auto total = [&](uint32_t c) { return ((red[0][c][lane] + red[1][c][lane]) + red[2][c][lane]) + red[3][c][lane]; };
+        // a diagonal tile's sums go on top of its reactions
+        if (diag) store(w.slot, i, rx + total(0), ry + total(1), rz + total(2));
+        else store(w.slot, i, total(0), total(1), total(2));
+    }
+}
+
+// Split items (blocks [0, grid_split)) and one-sided ones in one launch.
+template <int S>
+__global__ __launch_bounds__(kBlock) void k_force_split(const WorkItem* __restrict__ items_split, uint32_t n_split,
+                                                        uint32_t grid_split, const WorkItem* __restrict__ items,
+                                                        uint32_t n_items, const double* __restrict__ x,
+                                                        const double* __restrict__ y, const double* __restrict__ z,
+                                                        const float* __restrict__ m32,
+                                                        const DiskCtl* __restrict__ ctl, uint32_t need,
+                                                        float* __restrict__ part, uint32_t n_all)
+{
+    extern __shared__ __align__(16) unsigned char split_lds[];
+    if (blockIdx.x >= grid_split) {
+        force_mixed_body<S>(blockIdx.x - grid_split, gridDim.x - grid_split, split_lds, items, n_items, x, y, z, m32,
+                            ctl, need, part, n_all);
+        return;
+    }
+    for (uint32_t it = blockIdx.x; it < n_split; it += grid_split) {
+        const WorkItem w = items_split[it];
+        if (!(ctl[w.disk].flags & need)) continue;
+        force_split_item(w, split_lds, x, y, z, m32, part, n_all);
+        __syncthreads();
+    }
+}
+
 hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
@@ -1144,7 +1360,16 @@ hipError_t launch_force_mixed(hipStream_t st, const MixedLists& l, const double*
 {
     if (l.n_sym && (l.R < 1 || l.R > kSymMaxR)) return hipErrorInvalidValue;
     if (l.S != 1 && l.S != 2 && l.S != 4) return hipErrorInvalidValue;
-    if (l.n_sym && l.n_one) {
+    if (l.n_sym && l.split) {
+        const size_t lds = std::max(kSplitLds, l.n_one ? mixed_lds_bytes(l.S) : 0);
+#define FORCE_SPLIT(S)                                                                                              \
+    hipLaunchKernelGGL(k_force_split<S>, dim3(l.grid_sym + (l.n_one ? l.grid_one : 0)), dim3(kBlock), lds, st, l.sym, \
+                       l.n_sym, l.grid_sym, l.one, l.n_one, x, y, z, m32, ctl, need, part, n_all)
+        if (l.S == 1) FORCE_SPLIT(1);
+        else if (l.S == 2) FORCE_SPLIT(2);
+        else FORCE_SPLIT(4);
+#undef FORCE_SPLIT
+    } else if (l.n_sym && l.n_one) {
         const size_t lds = std::max(sym_lds_bytes(l.R), mixed_lds_bytes(l.S));
 #define FORCE_BOTH(SELF, S)                                                                                         \
     hipLaunchKernelGGL((k_force_both<SELF, S>), dim3(l.grid_sym + l.grid_one), dim3(kBlock), lds, st, l.sym, l.n_sym, \
