@@ -144,7 +144,6 @@ struct rd_disk {
     unsigned long long* err = nullptr;
     double* scratch = nullptr;
     size_t scratch_len = 0;
-    double* red_out = nullptr;     // 12 doubles for integrals
     double* trash = nullptr;       // [3][kBodyBlock], written by single-disk stages that do not apply
     unsigned long long* errw = nullptr;     // single disk: per-wave error bits of the last stage
     unsigned long long* h_errw = nullptr;   // pinned copy of errw
@@ -186,12 +185,14 @@ struct rd_disk {
     std::vector<rd_integrator*> integrators;
 
     // pinned host mirrors
+    void* pinned = nullptr;        // holds the host arrays below
     DiskCtl* h_ctl = nullptr;
     unsigned long long* h_err = nullptr;
     uint32_t* h_feat = nullptr;    // [3 * n_disk]
     double* h_esum = nullptr;      // [n_disk]
     float* h_fx = nullptr;         // [n_disk][12]
     float* h_fy = nullptr;         // [n_disk]
+    double* h_red = nullptr;       // 12 doubles of an integral
     double* h_stage = nullptr;     // [2][3][stage_bodies] records (download_bodies)
     uint32_t stage_bodies = 0;
 
@@ -281,7 +282,7 @@ void free_buffers(rd_disk* d)
 {
     double** dp[] = {&d->x, &d->y, &d->z, &d->vx, &d->vy, &d->vz, &d->xo, &d->yo, &d->zo, &d->vxo, &d->vyo,
                      &d->vzo, &d->K, &d->part, &d->mass, &d->radius, &d->density, &d->cd, &d->m_ex, &d->scratch,
-                     &d->red_out, &d->eterm, &d->trash};
+                     &d->eterm, &d->trash};
     for (auto p : dp) dev_free(*p);
     for (int b = 0; b < 2; ++b)
         for (int c = 0; c < 3; ++c) dev_free(d->P[b][c]);
@@ -313,11 +314,11 @@ void free_buffers(rd_disk* d)
     dev_free(d->fx);
     dev_free(d->fy);
     dev_free(d->grid);
+    if (d->pinned) (void)hipHostFree(d->pinned);
+    d->pinned = nullptr;
     for (void** h : {(void**)&d->h_ctl, (void**)&d->h_err, (void**)&d->h_feat, (void**)&d->h_esum, (void**)&d->h_fx,
-                     (void**)&d->h_fy, (void**)&d->h_errw, (void**)&d->h_stage}) {
-        if (*h) (void)hipHostFree(*h);
+                     (void**)&d->h_fy, (void**)&d->h_errw, (void**)&d->h_red, (void**)&d->h_stage})
         *h = nullptr;
-    }
     d->part_len = 0;
     d->scratch_len = 0;
 }
@@ -349,7 +350,6 @@ int alloc_buffers(rd_disk* d)
     if (int rc = dev_alloc(&d->info, d->n_disk)) return rc;
     if (int rc = dev_alloc(&d->ctl, d->n_disk)) return rc;
     if (int rc = dev_alloc(&d->err, 2 * (size_t)d->n_disk)) return rc;   // max bits, then non-finite flags
-    if (int rc = dev_alloc(&d->red_out, 16)) return rc;
     if (int rc = dev_alloc(&d->trash, 3 * (size_t)kBodyBlock)) return rc;
     if (int rc = dev_alloc(&d->errw, n_errw(d))) return rc;
     if (int rc = dev_alloc(&d->feat, 3 * (size_t)d->n_disk)) return rc;
@@ -365,18 +365,31 @@ int alloc_buffers(rd_disk* d)
     if (int rc = dev_alloc(&d->coll_next, n)) return rc;
     if (int rc = dev_alloc(&d->coll_cell, 3 * n)) return rc;
     if (int rc = dev_alloc(&d->coll_rmax, 1)) return rc;
-    HIP_TRY(hipHostMalloc((void**)&d->h_ctl, sizeof(DiskCtl) * std::max<uint32_t>(1, d->n_disk)));
-    HIP_TRY(hipHostMalloc((void**)&d->h_err, 2 * sizeof(unsigned long long) * std::max<uint32_t>(1, d->n_disk)));
-    HIP_TRY(hipHostMalloc((void**)&d->h_errw, sizeof(unsigned long long) * n_errw(d)));
-    HIP_TRY(hipHostMalloc((void**)&d->h_feat, 3 * sizeof(uint32_t) * std::max<uint32_t>(1, d->n_disk)));
-    HIP_TRY(hipHostMalloc((void**)&d->h_esum, sizeof(double) * std::max<uint32_t>(1, d->n_disk)));
-    HIP_TRY(hipHostMalloc((void**)&d->h_fx, RD_MLP_IN * sizeof(float) * std::max<uint32_t>(1, d->n_disk)));
-    HIP_TRY(hipHostMalloc((void**)&d->h_fy, sizeof(float) * std::max<uint32_t>(1, d->n_disk)));
     // staging for records: the largest disk's, at most 2 x 3 MiB in all
     uint32_t n_max = 1;
     for (auto& h : d->hd) n_max = std::max(n_max, h.n);
     d->stage_bodies = std::min<uint32_t>(n_max, 32768);
-    HIP_TRY(hipHostMalloc((void**)&d->h_stage, (size_t)2 * 3 * d->stage_bodies * sizeof(rd_var4)));
+    // all pinned host memory in one allocation (one costs about 0.1 ms, and a small
+    // disk's creation was mostly eight of them)
+    const size_t nd1 = std::max<uint32_t>(1, d->n_disk);
+    const std::pair<void**, size_t> host[] = {{(void**)&d->h_ctl, nd1 * sizeof(DiskCtl)},
+                                              {(void**)&d->h_err, 2 * nd1 * sizeof(unsigned long long)},
+                                              {(void**)&d->h_errw, n_errw(d) * sizeof(unsigned long long)},
+                                              {(void**)&d->h_feat, 3 * nd1 * sizeof(uint32_t)},
+                                              {(void**)&d->h_esum, nd1 * sizeof(double)},
+                                              {(void**)&d->h_fx, nd1 * RD_MLP_IN * sizeof(float)},
+                                              {(void**)&d->h_fy, nd1 * sizeof(float)},
+                                              {(void**)&d->h_red, 12 * sizeof(double)},
+                                              {(void**)&d->h_stage, (size_t)2 * 3 * d->stage_bodies * sizeof(rd_var4)}};
+    auto padded = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
+    size_t total = 0;
+    for (auto& h : host) total += padded(h.second);
+    HIP_TRY(hipHostMalloc(&d->pinned, total));
+    char* at = (char*)d->pinned;
+    for (auto& h : host) {
+        *h.first = at;
+        at += padded(h.second);
+    }
     HIP_TRY(hipMemsetAsync(d->K, 0, (size_t)kMaxStage * 6 * n * sizeof(double), d->stream));
     HIP_TRY(hipMemsetAsync(d->ctl, 0, sizeof(DiskCtl) * d->n_disk, d->stream));
     d->generation++;
@@ -2447,16 +2460,15 @@ namespace {
 
 // The integrals of disk k from the kernels of launch_integral on `scr` (len
 // doubles of partial sums) with the 12 reduced values in `red`.
-int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, double* red, rd_integral* out)
+int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, rd_integral* out)
 {
     const HostDisk& h = d->hd[k];
     // the masses' range flag belongs to the work lists' sources
     if (int rc = ensure_lists(d)) return rc;
     HIP_TRY(launch_integral(d->stream, h.off, h.off + h.n, d->x, d->y, d->z, d->vx, d->vy, d->vz, d->mass, d->id,
-                            d->mass_odd, scr, len, red, red + 11));
-    double o[12];
-    HIP_TRY(hipMemcpyAsync(o, red, sizeof(o), hipMemcpyDeviceToHost, d->stream));
+                            d->mass_odd, scr, len, d->h_red, d->h_red + 11));
     HIP_TRY(hipStreamSynchronize(d->stream));
+    const double* const o = d->h_red;
     const double M0 = o[0];
     out->R = rd_var4{o[1] / M0, o[2] / M0, o[3] / M0, 0.0};
     out->V = rd_var4{o[4] / M0, o[5] / M0, o[6] / M0, 0.0};
@@ -2467,12 +2479,12 @@ int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, double* red, 
 
 // Scratch of rd_calc_integral_noalloc: a file-scope device array, so the call
 // allocates nothing.  Every GPU the library runs on holds its own copy (4 MiB
-// of partial sums plus 16 doubles of results) until the process ends; calls on
+// of partial sums) until the process ends; calls on
 // one GPU share it, so calls that overlap on one GPU race.  Every value a call
 // reads was written by the same call: nothing needs clearing.
 constexpr uint32_t kNoAllocBodies = 65536;
 constexpr size_t kNoAllocScratch = (size_t)1 << 19;
-static __device__ __align__(256) double scratch[kNoAllocScratch + 16];
+static __device__ __align__(256) double scratch[kNoAllocScratch];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -2510,7 +2522,7 @@ int rd_calc_integral(rd_disk* d, uint32_t k, rd_integral* out)
         if (int rc = dev_alloc(&d->scratch, need)) return rc;
         d->scratch_len = need;
     }
-    return integral_with(d, k, d->scratch, d->scratch_len, d->red_out, out);
+    return integral_with(d, k, d->scratch, d->scratch_len, out);
 }
 
 int rd_calc_integral_noalloc(rd_disk* d, uint32_t k, rd_integral* out)
@@ -2524,7 +2536,7 @@ int rd_calc_integral_noalloc(rd_disk* d, uint32_t k, rd_integral* out)
                                    std::to_string(kNoAllocBodies) + " bodies)");
     double* scr = nullptr;
     if (int rc = scratch_on(d->device, &scr)) return rc;
-    return integral_with(d, k, scr, kNoAllocScratch, scr + kNoAllocScratch, out);
+    return integral_with(d, k, scr, kNoAllocScratch, out);
 }
 
 // run_simulation's loop (src/red.cuda/main.cu:470-625) per disk, all disks in

@@ -183,31 +183,23 @@ __device__ __forceinline__ void exact_scale_fast(const double (&r2)[kT], double 
     EXACT_EACH sc[q] = __builtin_fma(e[q], g[q], h[q]);
 #undef EXACT_EACH
 }
-// m / sqrt(r2), the same sequences and range (r2 as above; |m| in [2^-600, 2^600]
-// or 0).
+// m / sqrt(r2) for r2 in the same range, as m times the inverse root: v_rsq_f64 (2^-24)
+// and one step of third order, y + y e (1/2 + 3/8 e) with e = 1 - r2 y^2 (error below
+// 2^-68 before rounding).  Its roundings weigh what those of a root and a
+// division do: the step's about 0.3 units in the last place (root mean square),
+// the product's another 0.3.
 template <uint32_t kT>
-__device__ __forceinline__ void exact_ratio_fast(const double (&r2)[kT], const double (&m)[kT], double (&v)[kT])
+__device__ __forceinline__ void ratio_fast(const double (&r2)[kT], const double (&m)[kT], double (&v)[kT])
 {
-    double g[kT], h[kT], e[kT];
+    double y[kT], e[kT], p[kT];
 #define EXACT_EACH _Pragma("unroll") for (uint32_t q = 0; q < kT; ++q)
-    EXACT_EACH h[q] = __builtin_amdgcn_rsq(r2[q]);
-    EXACT_EACH g[q] = r2[q] * h[q];
-    EXACT_EACH h[q] = h[q] * 0.5;
-    EXACT_EACH e[q] = __builtin_fma(-h[q], g[q], 0.5);
-    EXACT_EACH g[q] = __builtin_fma(g[q], e[q], g[q]);
-    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);
-    EXACT_EACH e[q] = __builtin_fma(-g[q], g[q], r2[q]);
-    EXACT_EACH g[q] = __builtin_fma(e[q], h[q], g[q]);
-    EXACT_EACH e[q] = __builtin_fma(-g[q], g[q], r2[q]);
-    EXACT_EACH g[q] = __builtin_fma(e[q], h[q], g[q]);   // sqrt(r2)
-    EXACT_EACH h[q] = __builtin_amdgcn_rcp(g[q]);
-    EXACT_EACH e[q] = __builtin_fma(-g[q], h[q], 1.0);
-    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);
-    EXACT_EACH e[q] = __builtin_fma(-g[q], h[q], 1.0);
-    EXACT_EACH h[q] = __builtin_fma(h[q], e[q], h[q]);   // 1 / sqrt(r2)
-    EXACT_EACH v[q] = m[q] * h[q];
-    EXACT_EACH e[q] = __builtin_fma(-g[q], v[q], m[q]);
-    EXACT_EACH v[q] = __builtin_fma(e[q], h[q], v[q]);
+    EXACT_EACH y[q] = __builtin_amdgcn_rsq(r2[q]);
+    EXACT_EACH p[q] = r2[q] * y[q];
+    EXACT_EACH e[q] = __builtin_fma(-p[q], y[q], 1.0);
+    EXACT_EACH p[q] = __builtin_fma(e[q], 0.375, 0.5);
+    EXACT_EACH e[q] = y[q] * e[q];
+    EXACT_EACH y[q] = __builtin_fma(e[q], p[q], y[q]);
+    EXACT_EACH v[q] = m[q] * y[q];
 #undef EXACT_EACH
 }
 
@@ -2884,68 +2876,11 @@ __device__ KSum block_sum(KSum v)
 
 constexpr uint32_t kIntSrc = 128;   // sources per block of the potential pass
 
-// Potential: sum of m_i m_j / r_ij over the pairs i < j of active bodies (the
-// reference sums the ordered pairs and halves them; both orders of a pair give
-// the same value).  A block takes 256 sinks, one per thread, against kIntSrc
-// sources on or above the diagonal and leaves one partial sum.  VALU-bound:
-// about 33 FP64 instructions per pair with the short root and division
-// sequences (exact_ratio_fast; the library's outside their range).  16385
-// bodies, under the profiler: 226 us, where every ordered pair with the
-// library's root and division took 827.
-__global__ __launch_bounds__(kBlock) void k_potential(uint32_t lo, uint32_t hi, const double* __restrict__ x,
-                                                      const double* __restrict__ y, const double* __restrict__ z,
-                                                      const double* __restrict__ mass,
-                                                      const int32_t* __restrict__ id,
-                                                      const uint32_t* __restrict__ mass_odd, KSum* __restrict__ out)
-{
-    __shared__ double4 tile[kIntSrc];
-    const uint32_t i0 = lo + blockIdx.x * kBlock, j0 = lo + blockIdx.y * kIntSrc;
-    const uint32_t j1 = min(hi, j0 + kIntSrc);
-    KSum s{0.0, 0.0};
-    if (j1 > i0 + 1) {   // else no pair i < j
-        const uint32_t i = i0 + threadIdx.x;
-        const bool valid = i < hi && id[i] > 0;
-        const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
-        const double mi = valid ? mass[i] : 0.0;
-        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
-        if (threadIdx.x < kIntSrc) {
-            const uint32_t j = j0 + threadIdx.x;
-            // w: the mass, -0 for an inactive body
-            if (j < j1) tile[threadIdx.x] = make_double4(x[j], y[j], z[j], id[j] > 0 ? mass[j] + 0.0 : -0.0);
-        }
-        __syncthreads();
-        // the sources past the sink, two at a time
-        const uint32_t k0 = i + 1 > j0 ? min(i + 1 - j0, j1 - j0) : 0u;
-        const uint32_t k_first = __builtin_amdgcn_readfirstlane(k0);   // the wave's smallest
-        for (uint32_t k = k_first & ~1u; k < j1 - j0; k += 2) {
-            double r2[2], m[2], d[2];
-#pragma unroll
-            for (uint32_t u = 0; u < 2; ++u) {
-                const double4 q = tile[min(k + u, j1 - j0 - 1)];
-                r2[u] = SQR(q.x - xi) + SQR(q.y - yi) + SQR(q.z - zi);
-                m[u] = mi * q.w;
-                const bool on = valid && k + u >= k0 && k + u < j1 - j0 && !(q.w == 0.0 && signbit(q.w));
-                d[u] = on ? 1.0 : 0.0;
-            }
-            double v[2];
-            exact_ratio_fast<2>(r2, m, v);
-#pragma unroll
-            for (uint32_t u = 0; u < 2; ++u) {
-                if (!exact_r2_in_range(r2[u], r2_span)) v[u] = d[u] != 0.0 ? m[u] / sqrt(r2[u]) : 0.0;
-                s.add(d[u] != 0.0 ? v[u] : 0.0);
-            }
-        }
-    }
-    s = block_sum(s);
-    if (threadIdx.x == 0) out[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
-}
-
 // Per-body terms of M, R, V, C and T: a partial sum of each per block of kBlock
 // bodies, out[k * gridDim.x + block].
-__global__ __launch_bounds__(kBlock) void k_body_terms(uint32_t lo, uint32_t hi, const double* x, const double* y,
-                                                       const double* z, const double* vx, const double* vy,
-                                                       const double* vz, const double* mass, const int32_t* id,
-                                                       KSum* out)
+__device__ void body_terms(uint32_t lo, uint32_t hi, const double* x, const double* y, const double* z,
+                           const double* vx, const double* vy, const double* vz, const double* mass,
+                           const int32_t* id, KSum* out)
 {
     const uint32_t i = lo + blockIdx.x * kBlock + threadIdx.x;
     const uint32_t ic = min(i, hi - 1);
@@ -2964,8 +2899,78 @@ __global__ __launch_bounds__(kBlock) void k_body_terms(uint32_t lo, uint32_t hi,
     }
 }
 
+// Potential: sum of m_i m_j / r_ij over the pairs i < j of active bodies (the
+// reference sums the ordered pairs and halves them; both orders of a pair give
+// the same value).  A block takes 256 sinks, one per thread, against kIntSrc
+// sources on or above the diagonal and leaves one partial sum; the first row of
+// blocks takes the body terms (8 us as a launch of their own).  VALU-bound:
+// about 27 FP64 instructions per pair, 7 of them the compensated sum (ratio_fast;
+// the library's root and division outside its range).  16385 bodies, under the
+// profiler: 152 us (226 with a correctly rounded root and division per pair).
+__global__ __launch_bounds__(kBlock) void k_integral(uint32_t lo, uint32_t hi, const double* __restrict__ x,
+                                                     const double* __restrict__ y, const double* __restrict__ z,
+                                                     const double* vx, const double* vy, const double* vz,
+                                                     const double* __restrict__ mass, const int32_t* __restrict__ id,
+                                                     const uint32_t* __restrict__ mass_odd, KSum* body,
+                                                     KSum* __restrict__ out)
+{
+    if (blockIdx.y == 0) {
+        body_terms(lo, hi, x, y, z, vx, vy, vz, mass, id, body);
+        return;
+    }
+    __shared__ double4 tile[kIntSrc];
+    const uint32_t by = blockIdx.y - 1u;
+    const uint32_t i0 = lo + blockIdx.x * kBlock, j0 = lo + by * kIntSrc;
+    const uint32_t j1 = min(hi, j0 + kIntSrc);
+    KSum s{0.0, 0.0};
+    if (j1 > i0 + 1) {   // else no pair i < j
+        const uint32_t i = i0 + threadIdx.x;
+        const bool valid = i < hi && id[i] > 0;
+        const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
+        const double mi = valid ? mass[i] : 0.0;
+        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
+        if (threadIdx.x < kIntSrc) {
+            const uint32_t j = j0 + threadIdx.x;
+            // w: the mass, -0 for an inactive body or none
+            tile[threadIdx.x] = j < j1 ? make_double4(x[j], y[j], z[j], id[j] > 0 ? mass[j] + 0.0 : -0.0)
+                                       : make_double4(0.0, 0.0, 0.0, -0.0);
+        }
+        __syncthreads();
+        // the sources past the sink, two at a time; pairs that do not count have
+        // mass 0 on one side
+        const uint32_t k0 = i + 1 > j0 ? min(i + 1 - j0, j1 - j0) : 0u;
+        const uint32_t k_first = __builtin_amdgcn_readfirstlane(k0);   // the wave's smallest
+        for (uint32_t k = k_first & ~1u; k < j1 - j0; k += 2) {
+            double r2[2], m[2], v[2];
+            bool out = false;
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                const double4 q = tile[k + u];
+                r2[u] = SQR(q.x - xi) + SQR(q.y - yi) + SQR(q.z - zi);
+                m[u] = k + u >= k0 ? mi * q.w : 0.0;
+                out |= !exact_r2_in_range(r2[u], r2_span);
+            }
+            ratio_fast<2>(r2, m, v);
+            if (out) {
+#pragma unroll
+                for (uint32_t u = 0; u < 2; ++u) {
+                    const double w = tile[k + u].w;
+                    const bool on = valid && k + u >= k0 && !(w == 0.0 && signbit(w));
+                    if (!exact_r2_in_range(r2[u], r2_span)) v[u] = on ? m[u] / sqrt(r2[u]) : 0.0;
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) s.add(v[u]);
+        }
+    }
+    s = block_sum(s);
+    if (threadIdx.x == 0) out[(size_t)by * gridDim.x + blockIdx.x] = s;
+}
+
 // The totals: block k < 11 sums the n_body partials of body term k, block 11
-// the n_pair partials of the potential, in a fixed order.
+// the n_pair partials of the potential, in a fixed order.  Eight partials are fetched at
+// a time (one at a time, a thread's 33 of 16385 bodies took 12.7 us of waiting).
+// out and out_u are the host's (pinned).
 __global__ __launch_bounds__(kBlock) void k_integral_total(const KSum* __restrict__ body, uint32_t n_body,
                                                            const KSum* __restrict__ pair, uint32_t n_pair,
                                                            double* __restrict__ out, double* __restrict__ out_u)
@@ -2974,7 +2979,14 @@ __global__ __launch_bounds__(kBlock) void k_integral_total(const KSum* __restric
     const KSum* row = k < 11 ? body + (size_t)k * n_body : pair;
     const uint32_t len = k < 11 ? n_body : n_pair;
     KSum s{0.0, 0.0};
-    for (uint32_t q = threadIdx.x; q < len; q += kBlock) s.add(row[q]);
+    for (uint32_t q = threadIdx.x; q < len; q += 8 * kBlock) {
+        KSum v[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) v[u] = row[min(q + u * kBlock, len - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            if (q + u * kBlock < len) s.add(v[u]);
+    }
     s = block_sum(s);
     if (threadIdx.x == 0) *(k < 11 ? out + k : out_u) = s.s + s.c;
 }
@@ -2996,8 +3008,8 @@ hipError_t launch_integral(hipStream_t st, uint32_t lo, uint32_t hi, const doubl
     const uint32_t nb = (n + kBlock - 1) / kBlock, nc = (n + kIntSrc - 1) / kIntSrc;
     KSum* body = reinterpret_cast<KSum*>(scratch);
     KSum* pair = body + (size_t)11 * nb;
-    hipLaunchKernelGGL(k_body_terms, dim3(nb), dim3(kBlock), 0, st, lo, hi, x, y, z, vx, vy, vz, mass, id, body);
-    hipLaunchKernelGGL(k_potential, dim3(nb, nc), dim3(kBlock), 0, st, lo, hi, x, y, z, mass, id, mass_odd, pair);
+    hipLaunchKernelGGL(k_integral, dim3(nb, nc + 1), dim3(kBlock), 0, st, lo, hi, x, y, z, vx, vy, vz, mass, id,
+                       mass_odd, body, pair);
     hipLaunchKernelGGL(k_integral_total, dim3(12), dim3(kBlock), 0, st, body, nb, pair, nb * nc, out, out_u);
     return hipGetLastError();
 }
