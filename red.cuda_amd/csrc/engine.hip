@@ -886,9 +886,14 @@ hipError_t enqueue_attempt(rd_integrator* it, int commit_advance)
                 // summing lanes cover every body, and no pair term of that launch reads y_n
                 if (r == last_stage(it)) a.commit = commit_advance;
             }
-            if ((e = launch_force_exact_stage(d->stream, exact_lists(d), it->method, r,
-                                              r == 0 ? F_K0_FORCE : F_ACTIVE, a)) != hipSuccess)
-                return e;
+            if (d->exact_sinks == 8 && exact_wide_stage(it->method, r)) {
+                if ((e = enqueue_force(d, a.fpos[0], a.fpos[1], a.fpos[2], F_ACTIVE)) != hipSuccess) return e;
+                e = launch_stage(d->stream, it->method, r, a);
+            } else {
+                e = launch_force_exact_stage(d->stream, exact_lists(d), it->method, r,
+                                             r == 0 ? F_K0_FORCE : F_ACTIVE, a);
+            }
+            if (e != hipSuccess) return e;
             if (r == 0 && it->method == RD_RKF78 && (e = launch_comb1(d->stream, it->method, a)) != hipSuccess)
                 return e;
         }

@@ -177,7 +177,8 @@ hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, const WorkItem* ite
                               uint32_t n_all);
 // The FP64 pair pass on 4- or 8-sink items with what follows the sums done by the
 // kernel's summing lanes (no stage kernel, no partial-sum slot): stage r of a single
-// gas-free disk's RKF7(8) (method 4, 0-12) or fixed-step RK4 (0-3), or the operator on
+// gas-free disk's RKF7(8) (method 4, 0-12; on 8-sink items not the wide stages) or
+// fixed-step RK4 (0-3), or the operator on
 // disk a.info0 (launch_operator's work; with gas, 4-sink items only).
 struct ExactLists {
     const WorkItem* items;
@@ -185,6 +186,10 @@ struct ExactLists {
     const double* m_ex;
     const uint32_t* mass_odd;
 };
+// RKF7(8) stages that combine the most k rows: their rows do not fit the registers of
+// the ten waves of an 8-sink block beside the pair terms (stage 10 of 1501 bodies: 20.8
+// us spilled, 13.9 + 4.7 as pair pass and stage kernel; stage 8 17.0)
+constexpr bool exact_wide_stage(int method, int r) { return method == 4 && r >= 9 && r <= 11; }
 hipError_t launch_force_exact_stage(hipStream_t s, const ExactLists& l, int method, int r, uint32_t need,
                                     const StageArgs& a);
 hipError_t launch_force_exact_operator(hipStream_t s, const ExactLists& l, uint32_t need, const StageArgs& a,

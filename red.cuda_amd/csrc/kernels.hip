@@ -2438,11 +2438,17 @@ hipError_t launch_force_exact_stage(hipStream_t st, const ExactLists& l, int met
         if (l.sinks == 4) EXACT_FUSED((k_force_exact_##M<4, R>), 4, a);                \
         else EXACT_FUSED((k_force_exact_##M<8, R>), 8, a);                             \
         break;
+    // the stages of most k rows (exact_wide_stage): 4-sink items only
+#define EXACT_WIDE(R)                                                                  \
+    case R:                                                                            \
+        if (l.sinks != 4) return hipErrorInvalidValue;                                 \
+        EXACT_FUSED((k_force_exact_rk8<4, R>), 4, a);                                  \
+        break;
     if (method == 4) {
         switch (r) {
             EXACT_STAGE(rk8, 0) EXACT_STAGE(rk8, 1) EXACT_STAGE(rk8, 2) EXACT_STAGE(rk8, 3) EXACT_STAGE(rk8, 4)
-            EXACT_STAGE(rk8, 5) EXACT_STAGE(rk8, 6) EXACT_STAGE(rk8, 7) EXACT_STAGE(rk8, 8) EXACT_STAGE(rk8, 9)
-            EXACT_STAGE(rk8, 10) EXACT_STAGE(rk8, 11) EXACT_STAGE(rk8, 12)
+            EXACT_STAGE(rk8, 5) EXACT_STAGE(rk8, 6) EXACT_STAGE(rk8, 7) EXACT_STAGE(rk8, 8) EXACT_STAGE(rk8, 12)
+            EXACT_WIDE(9) EXACT_WIDE(10) EXACT_WIDE(11)
         default: return hipErrorInvalidValue;
         }
     } else {
@@ -2452,6 +2458,7 @@ hipError_t launch_force_exact_stage(hipStream_t st, const ExactLists& l, int met
         }
     }
 #undef EXACT_STAGE
+#undef EXACT_WIDE
     return hipGetLastError();
 }
 
