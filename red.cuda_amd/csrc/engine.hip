@@ -856,6 +856,9 @@ hipError_t enqueue_k0_ahead(rd_integrator* it)
 int enqueue_operator(rd_disk* d, uint32_t k, double t, const double* r, const double* v, double* dy)
 {
     const HostDisk& h = d->hd[k];
+    // a disk whose bodies were all removed: no record to write, and the other
+    // disks' flags, which only launch_operator_begin clears, may hold F_NEED_K0
+    if (h.n == 0) return RD_OK;
     double* const p[3] = {d->P[0][0] + h.off, d->P[0][1] + h.off, d->P[0][2] + h.off};
     double* const vel[3] = {kv_ptr(d, 1, 0) + h.off, kv_ptr(d, 1, 1) + h.off, kv_ptr(d, 1, 2) + h.off};
     HIP_TRY(launch_operator_begin(d->stream, h.n, r, v, p, vel, d->ctl, d->n_disk, k));
