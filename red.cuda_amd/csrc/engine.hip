@@ -323,9 +323,8 @@ void free_buffers(rd_disk* d)
     d->scratch_len = 0;
 }
 
-// Waves of a per-body launch (3 components): the single-disk error slots.
-// error words: one per wave of the last stage kernel, or per summing wave of the
-// fused one (at most 6 in a block, a block per CU)
+// Error words of a single disk: one per wave of the last stage kernel, or per
+// summing wave of the fused one (at most 6 in a block, a block per CU).
 size_t n_errw(const rd_disk* d)
 {
     return std::max(3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock) + 1, 6 * (size_t)d->n_cu);
@@ -835,9 +834,11 @@ bool fused_operator(const rd_disk* d)
 }
 
 // error words that the last stage of an adaptive attempt writes for a single disk
+// (none for a disk without bodies, whose stages launch nothing)
 size_t error_words(const rd_integrator* it)
 {
     const rd_disk* d = it->d;
+    if (d->n_all == 0) return 0;
     if (fused_stages(it)) return (size_t)d->grid_force * (3 * d->exact_sinks / 4);
     return 3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock);
 }

@@ -59,3 +59,19 @@ def test_operator_on_an_empty_disk_of_a_batch(prec, k):
             rr, vv = before[q]
             rc, ody = O.ODisk(*parts[q]).calc_dydx(1, 0, 0.0, rr, vv)
             assert rc == 0 and bits_equal(d.calc_dydx(1, 0, 0.0, rr, vv, k=q), ody)
+
+
+@pytest.mark.parametrize("steps", [False, True])
+@pytest.mark.parametrize("method", [R.RD_RKF78, R.RD_RK4])
+def test_adaptive_steps_of_an_empty_disk(method, steps):
+    """No body, no error: every attempt is accepted and the step doubles (the
+    reference's rule for an error of zero)."""
+    d = R.Disk(*_far(3, 8), threshold=THR)
+    _eject_all(d, 0)
+    it = R.Integrator(d, method, 1e-3, adaptive=True, tol=1e-10)
+    it.set_guard(max_attempts=4)
+    if steps:
+        it.steps(2)
+    else:
+        assert it.step() == 1e-3 and it.step() == 2e-3
+    assert it.dt_next() == 4e-3
