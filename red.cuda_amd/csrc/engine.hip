@@ -313,7 +313,6 @@ void free_buffers(rd_disk* d)
     dev_free(d->esum);
     dev_free(d->fx);
     dev_free(d->fy);
-    dev_free(d->grid);
     if (d->pinned) (void)hipHostFree(d->pinned);
     d->pinned = nullptr;
     for (void** h : {(void**)&d->h_ctl, (void**)&d->h_err, (void**)&d->h_feat, (void**)&d->h_esum, (void**)&d->h_fx,
@@ -1093,6 +1092,7 @@ int rd_disk_destroy(rd_disk* d)
     d->integrators.clear();
     (void)hipStreamSynchronize(d->stream);
     free_buffers(d);
+    dev_free(d->grid);   // not with the buffers: rd_rebuild_vectors keeps the gas
     if (d->ev_err) (void)hipEventDestroy(d->ev_err);
     (void)hipStreamDestroy(d->stream);
     delete d;
