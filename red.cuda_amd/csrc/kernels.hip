@@ -206,13 +206,11 @@ __device__ __forceinline__ void ratio_fast(const double (&r2)[kT], const double 
 // An inactive source's mass is -0 (k_set_sources; an active one's never is), and
 // so is padding's.  Its terms are then zeros of either sign, which leave the
 // running sum unchanged: it starts at +0 and round-to-nearest never makes it -0.
-// The scale of a pair outside the short sequences' range: 0 for the sink itself
-// and for an inactive or padding source.
-__device__ __forceinline__ double exact_scale_any(double r2, double m, bool self)
-{
-    if (self || (m == 0.0 && signbit(m))) return 0.0;
-    return m / (sqrt(r2) * r2);
-}
+// A pair outside the short sequences' range is skipped if it is the sink itself
+// or such a source, whose position need not be finite then (0 times it would not
+// be zero), and takes the library's root and division otherwise.
+__device__ __forceinline__ bool exact_skip(double m, bool self) { return self || (m == 0.0 && signbit(m)); }
+__device__ __forceinline__ double exact_scale_any(double r2, double m) { return m / (sqrt(r2) * r2); }
 
 // What becomes of a body's complete sum, in the summing lane that holds component
 // q of body i.  load() is called by the lane that owns the sum, before the
@@ -412,9 +410,11 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
                     exact_scale_fast<kT>(r2, m, sc);
                     if (out) {
 #pragma unroll
-                        for (uint32_t q = 0; q < kT; ++q)
-                            if (!exact_r2_in_range(r2[q], r2_span))
-                                sc[q] = exact_scale_any(r2[q], m, j == w.sink_lo + g0 + kGroups * q);
+                        for (uint32_t q = 0; q < kT; ++q) {
+                            if (exact_r2_in_range(r2[q], r2_span)) continue;
+                            if (exact_skip(m, j == w.sink_lo + g0 + kGroups * q)) sc[q] = dx[q] = dy[q] = dz[q] = 0.0;
+                            else sc[q] = exact_scale_any(r2[q], m);
+                        }
                     }
 #pragma unroll
                     for (uint32_t q = 0; q < kT; ++q) {
@@ -496,7 +496,10 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
                 double one_sc[1];
                 exact_scale_fast<1>({r2}, sj.w, one_sc);
                 double sc = one_sc[0];
-                if (!exact_r2_in_range(r2, r2_span)) sc = exact_scale_any(r2, sj.w, t0 + k == i);
+                if (!exact_r2_in_range(r2, r2_span)) {
+                    if (exact_skip(sj.w, t0 + k == i)) continue;
+                    sc = exact_scale_any(r2, sj.w);
+                }
                 ax += sc * dx;
                 ay += sc * dy;
                 az += sc * dz;
