@@ -152,10 +152,18 @@ __device__ __forceinline__ void row_add8(double& sum, double v)
 // third of a pair term's instructions.  The range of r2 is tested on its high
 // word (one subtract, one compare); the masses' when they are set
 // (k_set_sources): *mass_odd is nonzero if some source is outside, and every
-// pair then takes the library's root and division.
+// pair then takes the branch of the rare ones (span 0: no r2 is in range), which
+// looks at its own mass (16385 bodies, one mass outside: 519 us, 470 without, 851
+// with the library's for every pair).  A span for each source would cost every
+// launch: registers where it is a lane's, 3% at 5000 bodies as a scalar.  The
+// kernel with one sink per lane looks at its tiles' masses as it loads them.
 __device__ __forceinline__ bool exact_r2_in_range(double r2, uint32_t span)
 {
     return (uint32_t)__double2hiint(r2) - kExactR2Lo < span;
+}
+__device__ __forceinline__ bool exact_mass_odd(double m)
+{
+    return !(m == 0.0 || (fabs(m) >= 0x1p-300 && fabs(m) <= 0x1p300));   // NaN too
 }
 template <uint32_t kT>
 __device__ __forceinline__ void exact_scale_fast(const double (&r2)[kT], double m, double (&sc)[kT])
@@ -409,11 +417,14 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
                     }
                     exact_scale_fast<kT>(r2, m, sc);
                     if (out) {
+                        const uint32_t own_span = exact_mass_odd(m) ? 0u : kExactR2Span;
 #pragma unroll
                         for (uint32_t q = 0; q < kT; ++q) {
-                            if (exact_r2_in_range(r2[q], r2_span)) continue;
-                            if (exact_skip(m, j == w.sink_lo + g0 + kGroups * q)) sc[q] = dx[q] = dy[q] = dz[q] = 0.0;
-                            else sc[q] = exact_scale_any(r2[q], m);
+                            if (exact_r2_in_range(r2[q], own_span)) continue;
+                            if (exact_skip(m, j == w.sink_lo + g0 + kGroups * q))
+                                sc[q] = dx[q] = dy[q] = dz[q] = 0.0;
+                            else
+                                sc[q] = exact_scale_any(r2[q], m);
                         }
                     }
 #pragma unroll
@@ -467,7 +478,6 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
                                                              const double* __restrict__ y,
                                                              const double* __restrict__ z,
                                                              const double* __restrict__ m_ex,
-                                                             const uint32_t* __restrict__ mass_odd,
                                                              const DiskCtl* __restrict__ ctl, uint32_t need,
                                                              double* __restrict__ part, uint32_t n_all)
 {
@@ -476,7 +486,6 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
         const WorkItem w = items[it];
         if (!(ctl[w.disk].flags & need)) continue;
-        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
         const uint32_t i = w.sink_lo + tid;
         const bool valid = i < w.sink_hi;
         const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
@@ -484,21 +493,23 @@ __global__ __launch_bounds__(kBlock) void k_force_exact_lane(const WorkItem* __r
         for (uint32_t t0 = w.src_lo; t0 < w.src_hi; t0 += kTile) {
             __syncthreads();
             const uint32_t j = t0 + tid;
-            if (j < w.src_hi) tile[tid] = make_double4(x[j], y[j], z[j], m_ex[j]);
-            __syncthreads();
+            const double m = j < w.src_hi ? m_ex[j] : -0.0;
+            if (j < w.src_hi) tile[tid] = make_double4(x[j], y[j], z[j], m);
+            // the rare pairs' branch for every pair of a tile with a mass outside
+            const uint32_t r2_span = __syncthreads_or(exact_mass_odd(m)) ? 0u : kExactR2Span;
             const uint32_t nt = min((uint32_t)kTile, w.src_hi - t0);
             for (uint32_t k = 0; k < nt; ++k) {
                 const double4 sj = tile[k];
-                const double dx = sj.x - xi;
-                const double dy = sj.y - yi;
-                const double dz = sj.z - zi;
+                double dx = sj.x - xi;
+                double dy = sj.y - yi;
+                double dz = sj.z - zi;
                 const double r2 = SQR(dx) + SQR(dy) + SQR(dz);
                 double one_sc[1];
                 exact_scale_fast<1>({r2}, sj.w, one_sc);
                 double sc = one_sc[0];
                 if (!exact_r2_in_range(r2, r2_span)) {
-                    if (exact_skip(sj.w, t0 + k == i)) continue;
-                    sc = exact_scale_any(r2, sj.w);
+                    if (exact_skip(sj.w, t0 + k == i)) sc = dx = dy = dz = 0.0;
+                    else if (!exact_r2_in_range(r2, kExactR2Span) || exact_mass_odd(sj.w)) sc = exact_scale_any(r2, sj.w);
                 }
                 ax += sc * dx;
                 ay += sc * dy;
@@ -1339,7 +1350,10 @@ hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* it
     hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(BLOCK), 0, st, items, n_items, x, y, z, m_ex, mass_odd, ctl, need, \
                        __VA_ARGS__)
     switch (sinks) {
-    case 1: EXACT_LAUNCH(k_force_exact_lane, kBlock, part, n_all); break;
+    case 1:
+        hipLaunchKernelGGL(k_force_exact_lane, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m_ex, ctl,
+                           need, part, n_all);
+        break;
     case 4: EXACT_LAUNCH(k_force_exact<4>, exact_block(4), part, n_all); break;
     case 8: EXACT_LAUNCH(k_force_exact<8>, exact_block(8), part, n_all); break;
     case 12: EXACT_LAUNCH(k_force_exact<12>, exact_block(12), part, n_all); break;
@@ -2595,7 +2609,7 @@ __global__ __launch_bounds__(kBlock) void k_set_sources(uint32_t n_all, const do
     const bool act = id[i] > 0;
     const double m = mass[i] + 0.0;
     m_ex[i] = act ? m : -0.0;
-    if (act && !(m == 0.0 || (fabs(m) >= 0x1p-300 && fabs(m) <= 0x1p300))) *mass_odd = 1u;   // NaN too
+    if (act && exact_mass_odd(m)) *mass_odd = 1u;
     m32[i] = (act && (i - di.off) >= di.n_fp64) ? (float)mass[i] : 0.0f;
 }
 
