@@ -191,23 +191,29 @@ __device__ __forceinline__ void exact_scale_fast(const double (&r2)[kT], double 
     EXACT_EACH sc[q] = __builtin_fma(e[q], g[q], h[q]);
 #undef EXACT_EACH
 }
-// m / sqrt(r2) for r2 in the same range, as m times the inverse root: v_rsq_f64 (2^-24)
-// and one step of third order, y + y e (1/2 + 3/8 e) with e = 1 - r2 y^2 (error below
-// 2^-68 before rounding).  Its roundings weigh what those of a root and a
-// division do: the step's about 0.3 units in the last place (root mean square),
-// the product's another 0.3.
+// m / sqrt(r2) for r2 in the same range and |m| in [2^-600, 2^600] or 0, as m times
+// the inverse root: y = v_rsq_f64 (2^-24) and one step of third order, a factor
+// 1 + c with c = e (1/2 + 3/8 e), e = 1 - r2 y^2 (error below 2^-68).  The
+// roundings of r2 y and m y, which a correctly rounded root and division do not
+// have, are kept (l) and added, so all that is left is the last one: at most
+// 0.5001 units in the last place, 0.29 root mean square; root and division, each
+// rounded, come to 0.42.
 template <uint32_t kT>
 __device__ __forceinline__ void ratio_fast(const double (&r2)[kT], const double (&m)[kT], double (&v)[kT])
 {
-    double y[kT], e[kT], p[kT];
+    double y[kT], e[kT], p[kT], l[kT];
 #define EXACT_EACH _Pragma("unroll") for (uint32_t q = 0; q < kT; ++q)
     EXACT_EACH y[q] = __builtin_amdgcn_rsq(r2[q]);
     EXACT_EACH p[q] = r2[q] * y[q];
+    EXACT_EACH l[q] = __builtin_fma(r2[q], y[q], -p[q]);
     EXACT_EACH e[q] = __builtin_fma(-p[q], y[q], 1.0);
-    EXACT_EACH p[q] = __builtin_fma(e[q], 0.375, 0.5);
-    EXACT_EACH e[q] = y[q] * e[q];
-    EXACT_EACH y[q] = __builtin_fma(e[q], p[q], y[q]);
+    EXACT_EACH e[q] = __builtin_fma(-l[q], y[q], e[q]);
     EXACT_EACH v[q] = m[q] * y[q];
+    EXACT_EACH l[q] = __builtin_fma(m[q], y[q], -v[q]);
+    EXACT_EACH p[q] = __builtin_fma(e[q], 0.375, 0.5);
+    EXACT_EACH e[q] = e[q] * p[q];
+    EXACT_EACH l[q] = __builtin_fma(v[q], e[q], l[q]);
+    EXACT_EACH v[q] = v[q] + l[q];
 #undef EXACT_EACH
 }
 
@@ -2928,9 +2934,9 @@ __device__ void body_terms(uint32_t lo, uint32_t hi, const double* x, const doub
 // the same value).  A block takes 256 sinks, one per thread, against kIntSrc
 // sources on or above the diagonal and leaves one partial sum; the first row of
 // blocks takes the body terms (8 us as a launch of their own).  VALU-bound:
-// about 27 FP64 instructions per pair, 7 of them the compensated sum (ratio_fast;
-// the library's root and division outside its range).  16385 bodies, under the
-// profiler: 152 us (226 with a correctly rounded root and division per pair).
+// about 31 FP64 instructions per pair, 7 of them the compensated sum (ratio_fast;
+// the library's root and division outside its range).  One energy of 16385
+// bodies: 165 us, 203 with a correctly rounded root and division per pair.
 __global__ __launch_bounds__(kBlock) void k_integral(uint32_t lo, uint32_t hi, const double* __restrict__ x,
                                                      const double* __restrict__ y, const double* __restrict__ z,
                                                      const double* vx, const double* vy, const double* vz,
