@@ -2468,14 +2468,12 @@ int rd_rebuild_vectors(rd_disk* d, uint32_t k)
 namespace {
 
 // The integrals of disk k from the kernels of launch_integral on `scr` (len
-// doubles of partial sums) with the 12 reduced values in `red`.
+// doubles of partial sums).  Needs no work lists: it must not allocate.
 int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, rd_integral* out)
 {
     const HostDisk& h = d->hd[k];
-    // the masses' range flag belongs to the work lists' sources
-    if (int rc = ensure_lists(d)) return rc;
-    HIP_TRY(launch_integral(d->stream, h.off, h.off + h.n, d->x, d->y, d->z, d->vx, d->vy, d->vz, d->mass, d->id,
-                            d->mass_odd, scr, len, d->h_red, d->h_red + 11));
+    HIP_TRY(launch_integral(d->stream, h.off, h.off + h.n, d->x, d->y, d->z, d->vx, d->vy, d->vz, d->mass, d->id, scr,
+                            len, d->h_red, d->h_red + 11));
     HIP_TRY(hipStreamSynchronize(d->stream));
     const double* const o = d->h_red;
     const double M0 = o[0];
@@ -2488,9 +2486,9 @@ int integral_with(rd_disk* d, uint32_t k, double* scr, size_t len, rd_integral* 
 
 // Scratch of rd_calc_integral_noalloc: a file-scope device array, so the call
 // allocates nothing.  Every GPU the library runs on holds its own copy (4 MiB
-// of partial sums) until the process ends; calls on
-// one GPU share it, so calls that overlap on one GPU race.  Every value a call
-// reads was written by the same call: nothing needs clearing.
+// of partial sums) until the process ends; calls on one GPU share it, so calls
+// that overlap on one GPU race.  Every value a call reads was written by the
+// same call: nothing needs clearing.
 constexpr uint32_t kNoAllocBodies = 65536;
 constexpr size_t kNoAllocScratch = (size_t)1 << 19;
 static __device__ __align__(256) double scratch[kNoAllocScratch];

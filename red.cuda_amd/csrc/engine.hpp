@@ -234,8 +234,8 @@ hipError_t launch_ejection(hipStream_t s, uint32_t n_all, const double* x, const
                            double ed2, double hcd2, uint32_t* out, uint32_t* counter, uint32_t cap);
 hipError_t launch_integral(hipStream_t s, uint32_t lo, uint32_t hi, const double* x, const double* y,
                            const double* z, const double* vx, const double* vy, const double* vz,
-                           const double* mass, const int32_t* id, const uint32_t* mass_odd, double* scratch,
-                           size_t scratch_len, double* out /* 11 doubles: M, Rx,Ry,Rz, Vx,Vy,Vz, Cx,Cy,Cz, T */,
+                           const double* mass, const int32_t* id, double* scratch, size_t scratch_len,
+                           double* out /* 11 doubles: M, Rx,Ry,Rz, Vx,Vy,Vz, Cx,Cy,Cz, T */,
                            double* out_u /* sum of m_i m_j / r_ij over i < j */);   // both may be pinned host memory
 // doubles of partial sums launch_integral needs for n bodies
 size_t integral_scratch(uint32_t n);

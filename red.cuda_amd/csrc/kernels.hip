@@ -2941,8 +2941,7 @@ __global__ __launch_bounds__(kBlock) void k_integral(uint32_t lo, uint32_t hi, c
                                                      const double* __restrict__ y, const double* __restrict__ z,
                                                      const double* vx, const double* vy, const double* vz,
                                                      const double* __restrict__ mass, const int32_t* __restrict__ id,
-                                                     const uint32_t* __restrict__ mass_odd, KSum* body,
-                                                     KSum* __restrict__ out)
+                                                     KSum* body, KSum* __restrict__ out)
 {
     if (blockIdx.y == 0) {
         body_terms(lo, hi, x, y, z, vx, vy, vz, mass, id, body);
@@ -2958,14 +2957,17 @@ __global__ __launch_bounds__(kBlock) void k_integral(uint32_t lo, uint32_t hi, c
         const bool valid = i < hi && id[i] > 0;
         const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
         const double mi = valid ? mass[i] : 0.0;
-        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
+        bool odd = exact_mass_odd(mi);
         if (threadIdx.x < kIntSrc) {
             const uint32_t j = j0 + threadIdx.x;
             // w: the mass, -0 for an inactive body or none
-            tile[threadIdx.x] = j < j1 ? make_double4(x[j], y[j], z[j], id[j] > 0 ? mass[j] + 0.0 : -0.0)
-                                       : make_double4(0.0, 0.0, 0.0, -0.0);
+            const double4 q = j < j1 ? make_double4(x[j], y[j], z[j], id[j] > 0 ? mass[j] + 0.0 : -0.0)
+                                     : make_double4(0.0, 0.0, 0.0, -0.0);
+            odd |= exact_mass_odd(q.w);
+            tile[threadIdx.x] = q;
         }
-        __syncthreads();
+        // the library's root and division for every pair of a block with a mass outside
+        const uint32_t r2_span = __syncthreads_or(odd) ? 0u : kExactR2Span;
         // the sources past the sink, two at a time; pairs that do not count have
         // mass 0 on one side
         const uint32_t k0 = i + 1 > j0 ? min(i + 1 - j0, j1 - j0) : 0u;
@@ -3029,8 +3031,8 @@ size_t integral_scratch(uint32_t n)
 
 hipError_t launch_integral(hipStream_t st, uint32_t lo, uint32_t hi, const double* x, const double* y,
                            const double* z, const double* vx, const double* vy, const double* vz,
-                           const double* mass, const int32_t* id, const uint32_t* mass_odd, double* scratch,
-                           size_t scratch_len, double* out, double* out_u)
+                           const double* mass, const int32_t* id, double* scratch, size_t scratch_len, double* out,
+                           double* out_u)
 {
     const uint32_t n = hi - lo;
     if (n == 0) return hipSuccess;
@@ -3039,7 +3041,7 @@ hipError_t launch_integral(hipStream_t st, uint32_t lo, uint32_t hi, const doubl
     KSum* body = reinterpret_cast<KSum*>(scratch);
     KSum* pair = body + (size_t)11 * nb;
     hipLaunchKernelGGL(k_integral, dim3(nb, nc + 1), dim3(kBlock), 0, st, lo, hi, x, y, z, vx, vy, vz, mass, id,
-                       mass_odd, body, pair);
+                       body, pair);
     hipLaunchKernelGGL(k_integral_total, dim3(12), dim3(kBlock), 0, st, body, nb, pair, nb * nc, out, out_u);
     return hipGetLastError();
 }
