@@ -567,21 +567,43 @@ int build_lists(rd_disk* d)
             const uint32_t lo = std::max(b[2], di.n_fp64);
             return sym && cls == 0 ? std::max(lo, b[1]) : lo;
         };
-        uint32_t C = C_max, S_one = S;
+        // chunks of the symmetric kernel: R blocks each.  kSymChunks..2 kSymChunks - 1
+        // once the disk is that large: enough items to fill the device, few
+        // partial-sum slots; at least sym_chunk_min blocks (many small disks fill the
+        // device by themselves)
+        const uint32_t nblk = sym ? (h.n_si() + kSymBlockBodies - 1) / kSymBlockBodies : 0;
+        const uint32_t rmin = std::max<uint32_t>(1, d->tuning.sym_chunk_min);
+        const uint32_t R = std::min<uint32_t>(kSymMaxR, std::max<uint32_t>(rmin, nblk / kSymChunks));
+        const uint32_t n_sym_chunk = (nblk + R - 1) / R;
+        uint32_t C[3] = {C_max, C_max, C_max}, S_one = S;
         if (d->precision == RD_PREC_MIXED) {
-            auto n_one = [&](uint32_t chunk, uint32_t s) {
+            auto n_src = [&](int cls) {   // one-sided sources of a class with sinks
+                uint32_t b[4];
+                class_bounds(h, cls, b);
+                const uint32_t lo = one_sided_src(cls, b);
+                return b[1] > b[0] && b[3] > lo ? b[3] - lo : 0u;
+            };
+            auto n_one = [&]() {
                 size_t n = 0;
                 for (int cls = 0; cls < 3; ++cls) {
                     uint32_t b[4];
                     class_bounds(h, cls, b);
-                    const uint32_t lo = one_sided_src(cls, b);
-                    if (b[1] > b[0] && b[3] > lo)
-                        n += (size_t)((b[1] - b[0] + 64 * s - 1) / (64 * s)) * ((b[3] - lo + chunk - 1) / chunk);
+                    n += (size_t)((b[1] - b[0] + 64 * S - 1) / (64 * S)) * ((n_src(cls) + C[cls] - 1) / C[cls]);
                 }
                 return n;
             };
-            while (C > (uint32_t)kTile && n_one(C, S) < kOneSidedItems) C = (C / 2 + kTile - 1) / kTile * kTile;
-            if (n_one(C, S) < kOneSidedItems) S_one = 1;
+            while (n_one() < kOneSidedItems) {
+                bool cut = false;
+                for (int cls = 0; cls < 3; ++cls) {
+                    const uint32_t half = (C[cls] / 2 + kTile - 1) / kTile * kTile;
+                    const uint32_t slots = (cls == 0 ? n_sym_chunk : 0) + (n_src(cls) + half - 1) / half;
+                    if (C[cls] == (uint32_t)kTile || n_src(cls) == 0 || slots > kSlotBatch) continue;
+                    C[cls] = half;
+                    cut = true;
+                }
+                if (!cut) break;
+            }
+            if (n_one() < kOneSidedItems) S_one = 1;
         }
         for (int cls = 0; cls < 3; ++cls) {
             uint32_t b[4];
@@ -602,13 +624,7 @@ int build_lists(rd_disk* d)
                 uint32_t base = 0;
                 const uint32_t lo = one_sided_src(cls, b);
                 if (sym && cls == 0) {
-                    const uint32_t nblk = (b[1] + kSymBlockBodies - 1) / kSymBlockBodies;
-                    // kSymChunks..2 kSymChunks - 1 chunks once the disk is that large:
-                    // enough items to fill the device, few partial-sum slots; at least
-                    // sym_chunk_min blocks (many small disks fill the device by themselves)
-                    const uint32_t rmin = std::max<uint32_t>(1, d->tuning.sym_chunk_min);
-                    const uint32_t R = std::min<uint32_t>(kSymMaxR, std::max<uint32_t>(rmin, nblk / kSymChunks));
-                    const uint32_t nc = (nblk + R - 1) / R, span = R * kSymBlockBodies;
+                    const uint32_t nc = n_sym_chunk, span = R * kSymBlockBodies;
                     d->sym_R = std::max(d->sym_R, R);
                     // a decision of the disk alone: results never depend on the batch
                     const uint32_t self = nblk <= kSymSelfMaxBlocks ? kItemSelf : 0u;
@@ -624,7 +640,7 @@ int build_lists(rd_disk* d)
                 }
                 const uint32_t hi = b[3];
                 const uint32_t nsrc = hi > lo ? hi - lo : 0;
-                const uint32_t nch = (nsrc + C - 1) / C;
+                const uint32_t nch = (nsrc + C[cls] - 1) / C[cls];
                 di.nchunk[cls] = base + nch;
                 max_chunks = std::max<size_t>(max_chunks, base + nch);
                 const uint32_t G = 64u * S_one;
@@ -632,8 +648,8 @@ int build_lists(rd_disk* d)
                 for (uint32_t s = b[0]; s < b[1]; s += G)
                     for (uint32_t c = 0; c < nch; ++c)
                         items.push_back(WorkItem{k, h.off + s, h.off + std::min(b[1], s + G),
-                                                 h.off + lo + c * C, h.off + std::min(hi, lo + (c + 1) * C), base + c,
-                                                 0, narrow});
+                                                 h.off + lo + c * C[cls],
+                                                 h.off + std::min(hi, lo + (c + 1) * C[cls]), base + c, 0, narrow});
             }
         }
     }

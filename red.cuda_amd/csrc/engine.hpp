@@ -108,9 +108,15 @@ constexpr uint32_t kItemRow = 4u, kItemReact = 8u, kItemDiagRow = 16u;
 // 364 -> 290, 4601 (171) 371 -> 352, 5101 (210) 375 -> 381; 9001 bodies of all classes
 // (78 + 580) 494 -> 526.
 constexpr uint32_t kSymSplitTiles = 180;
+// FP32 partial-sum slots that a single-disk stage reads at once: a 65-chunk disk
+// (16385 bodies) in one batch.
+constexpr uint32_t kSlotBatch = 72;
 // One-sided items of a disk: chunks are halved (down to one 256-source tile),
 // then the sinks taken one per lane, until the disk has this many items -- two
-// per CU.  A decision of the disk alone: results never depend on the batch.
+// per CU.  A class whose slots would pass kSlotBatch keeps its chunk: every body
+// of the disk reads as many slots as the class with the most (star + 130000
+// planetesimals, 508 slots for the star: 176 us a pair pass and stage; 78 with
+// 127).  A decision of the disk alone: results never depend on the batch.
 constexpr uint32_t kOneSidedItems = 512;
 
 // Gas disk, device copy: the analytic model (analytic_gas_disk_params_t

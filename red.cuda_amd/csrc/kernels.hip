@@ -1606,8 +1606,7 @@ __device__ double partial_sum_upto_t(const T* __restrict__ p, size_t st, uint32_
 __device__ double partial_sum_upto(const StageArgs& a, uint32_t i, int q, uint32_t nc, uint32_t ncmax)
 {
     const size_t off = (size_t)q * a.n_all + i, st = (size_t)3 * a.n_all;
-    // one batch of 72 FP32 slots covers a 65-chunk disk (16385 bodies) at once
-    if (a.mixed) return partial_sum_upto_t<float, 72>(reinterpret_cast<const float*>(a.part) + off, st, nc, ncmax);
+    if (a.mixed) return partial_sum_upto_t<float, kSlotBatch>(reinterpret_cast<const float*>(a.part) + off, st, nc, ncmax);
     return partial_sum_upto_t<double, 16>(a.part + off, st, nc, ncmax);
 }
 
