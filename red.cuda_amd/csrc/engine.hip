@@ -596,7 +596,7 @@ int build_lists(rd_disk* d)
                 bool cut = false;
                 for (int cls = 0; cls < 3; ++cls) {
                     const uint32_t half = (C[cls] / 2 + kTile - 1) / kTile * kTile;
-                    const uint32_t slots = (cls == 0 ? n_sym_chunk : 0) + (n_src(cls) + half - 1) / half;
+                    const uint32_t slots = (cls == 0 ? n_sym_chunk : 0) + 2 * ((n_src(cls) + half - 1) / half);
                     if (C[cls] == (uint32_t)kTile || n_src(cls) == 0 || slots > kSlotBatch) continue;
                     C[cls] = half;
                     cut = true;
@@ -641,15 +641,18 @@ int build_lists(rd_disk* d)
                 const uint32_t hi = b[3];
                 const uint32_t nsrc = hi > lo ? hi - lo : 0;
                 const uint32_t nch = (nsrc + C[cls] - 1) / C[cls];
-                di.nchunk[cls] = base + nch;
-                max_chunks = std::max<size_t>(max_chunks, base + nch);
+                // a cut chunk's sum in two slots, so that cutting rounds no oftener
+                const uint32_t per = C[cls] < C_max ? 2u : 1u;
+                di.nchunk[cls] = base + per * nch;
+                max_chunks = std::max<size_t>(max_chunks, di.nchunk[cls]);
                 const uint32_t G = 64u * S_one;
-                const uint32_t narrow = S_one == 1 ? kItemNarrow : 0u;
+                const uint32_t flags = (S_one == 1 ? kItemNarrow : 0u) | (per == 2 ? kItemTwoSlots : 0u);
                 for (uint32_t s = b[0]; s < b[1]; s += G)
                     for (uint32_t c = 0; c < nch; ++c)
                         items.push_back(WorkItem{k, h.off + s, h.off + std::min(b[1], s + G),
                                                  h.off + lo + c * C[cls],
-                                                 h.off + std::min(hi, lo + (c + 1) * C[cls]), base + c, 0, narrow});
+                                                 h.off + std::min(hi, lo + (c + 1) * C[cls]), base + per * c, 0,
+                                                 flags});
             }
         }
     }

@@ -100,6 +100,10 @@ struct WorkItem {
 constexpr uint32_t kItemSelf = 1u;
 // one-sided item of 64 sinks, one per lane, whatever the launch's sinks per lane
 constexpr uint32_t kItemNarrow = 2u;
+// one-sided item whose sums go to two slots each, the sum rounded to FP32 and what
+// that rounding left: the chunk was cut (kOneSidedItems), and the FP64 sum over the
+// whole chunk would otherwise be rounded once for each piece
+constexpr uint32_t kItemTwoSlots = 32u;
 // the symmetric kernel's tiles cut finer (k_force_split)
 constexpr uint32_t kItemRow = 4u, kItemReact = 8u, kItemDiagRow = 16u;
 // A launch of at most this many tiles, its one-sided pairs counted as 65536 a

@@ -637,9 +637,15 @@ __device__ __forceinline__ void force_mixed_item(const WorkItem& w, unsigned cha
                 const double sx = ((ax[s] + red[s][0][lane]) + red[S + s][0][lane]) + red[2 * S + s][0][lane];
                 const double sy = ((ay[s] + red[s][1][lane]) + red[S + s][1][lane]) + red[2 * S + s][1][lane];
                 const double sz = ((az[s] + red[s][2][lane]) + red[S + s][2][lane]) + red[2 * S + s][2][lane];
-                part[(size_t)(w.slot * 3 + 0) * n_all + i] = (float)sx;
-                part[(size_t)(w.slot * 3 + 1) * n_all + i] = (float)sy;
-                part[(size_t)(w.slot * 3 + 2) * n_all + i] = (float)sz;
+                const double sum[3] = {sx, sy, sz};
+#pragma unroll
+                for (uint32_t c = 0; c < 3; ++c) {
+                    const float hi = (float)sum[c];
+                    part[(size_t)(w.slot * 3 + c) * n_all + i] = hi;
+                    if (w.flags & kItemTwoSlots)   // (nothing is left of a sum that is not finite)
+                        part[(size_t)(w.slot * 3 + 3 + c) * n_all + i] =
+                            fabsf(hi) <= FLT_MAX ? (float)(sum[c] - (double)hi) : 0.0f;
+                }
             }
         }
     }
@@ -1554,7 +1560,8 @@ __device__ inline double* ka_w(const StageArgs& a, int r, int q) { return a.K + 
 // Sum of the pair partials of body i, component q, in slot order, in FP64.
 // The FP64 pair kernel leaves one FP64 slot; the mixed-precision kernels leave
 // one FP32 slot per source chunk (the chunk's total, formed in FP64 and
-// rounded once), at the same index in float units.  Loads go out in batches
+// rounded once; two for a chunk cut finer, kItemTwoSlots), at the same index in
+// float units.  Loads go out in batches
 // of 128 bytes per lane (16 doubles or 32 floats); a slot index past the last
 // is clamped to it, so every load is unconditional and in bounds and only the
 // sum skips it (a guarded load would become a branch and a wait per slot).
