@@ -733,7 +733,8 @@ int build_lists(rd_disk* d)
     if (!items.empty())
         HIP_TRY(hipMemcpy(d->items_force, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
     const uint32_t maxgrid = std::max<uint32_t>(1, d->tuning.blocks_per_cu) * (uint32_t)d->n_cu;
-    // the term-parallel FP64 kernel's items are single-pass: a block each, up to 8 per CU
+    // the term-parallel FP64 kernel: a block for each item, up to 8 per CU (beyond, a
+    // block takes several items in turn)
     const uint32_t grid_cap = d->precision == RD_PREC_FP64 && d->exact_sinks != 1 ? 8u * (uint32_t)d->n_cu : maxgrid;
     d->grid_force = std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_force, grid_cap));
     d->grid_sym = d->sym_split ? d->n_items_sym : std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_sym, maxgrid));
@@ -804,7 +805,7 @@ hipError_t enqueue_force(rd_disk* d, const double* fx, const double* fy, const d
 {
     if (d->precision == RD_PREC_FP64)
         return launch_force_exact(d->stream, d->exact_sinks, d->items_force, d->n_items_force, d->grid_force, fx, fy,
-                                  fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all);
+                                  fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all, (uint32_t)d->n_cu);
     // mixed precision: FP32 slot totals, in float units of the same buffer
     float* part32 = reinterpret_cast<float*>(d->part);
     const MixedLists l{d->items_sym,   d->n_items_sym,   d->grid_sym,   d->sym_R, d->sym_self, d->sym_split,

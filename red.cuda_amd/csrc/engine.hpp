@@ -184,7 +184,7 @@ struct BodyArrays {
 hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
-                              uint32_t n_all);
+                              uint32_t n_all, uint32_t n_cu);
 // The FP64 pair pass on 4- or 8-sink items with what follows the sums done by the
 // kernel's summing lanes (no stage kernel, no partial-sum slot): stage r of a single
 // gas-free disk's RKF7(8) (method 4, 0-12; on 8-sink items not the wide stages) or

@@ -253,7 +253,8 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
                                                  const double* __restrict__ x, const double* __restrict__ y,
                                                  const double* __restrict__ z, const double* __restrict__ m_ex,
                                                  const uint32_t* __restrict__ mass_odd,
-                                                 const DiskCtl* __restrict__ ctl, uint32_t need, const Fin& fin)
+                                                 const DiskCtl* __restrict__ ctl, uint32_t need, const Fin& fin,
+                                                 bool turns = false)
 {
     constexpr uint32_t kTile = exact_tile(kS);
     constexpr uint32_t kTermers = 64 * exact_term_waves(kS);
@@ -302,9 +303,8 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
     // blocks that share a CU take turns there, by tile: the oldest block would
     // otherwise run at full speed, end first and leave the CU to ever fewer
     // (16385 bodies: blocks ended between 259 and 538 us).
-    // Only while all blocks of the launch are resident: beyond, those that end
-    // early make room for the next.
-    const bool shared_cu = gridDim.x > 256u && gridDim.x <= (kS == 18 ? 1280u : 1536u);
+    // Only while all blocks of the launch are resident (turns, launch_force_exact):
+    // beyond, those that end early make room for the next.
     if (!termer && kS != 8) __builtin_amdgcn_s_setprio(3);
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
         const WorkItem w = items[it];
@@ -399,7 +399,7 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
         // the sums of the tile before, from term[b ^ 1]
         auto tile = [&](uint32_t t, uint32_t b, double4& sj) {
             if (termer) {
-                if (!kRowSum && shared_cu) switch ((t + my_turn) & 3u) {
+                if (!kRowSum && turns) switch ((t + my_turn) & 3u) {
                     case 0: __builtin_amdgcn_s_setprio(0); break;
                     case 1: __builtin_amdgcn_s_setprio(1); break;
                     default: __builtin_amdgcn_s_setprio(2);
@@ -470,9 +470,9 @@ void k_force_exact(const WorkItem* __restrict__ items, uint32_t n_items,
                                                              const double* __restrict__ m_ex,
                                                              const uint32_t* __restrict__ mass_odd,
                                                              const DiskCtl* __restrict__ ctl, uint32_t need,
-                                                             double* __restrict__ part, uint32_t n_all)
+                                                             double* __restrict__ part, uint32_t n_all, bool turns)
 {
-    force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, StoreSum{part, n_all});
+    force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, StoreSum{part, n_all}, turns);
 }
 
 // The same sum with one sink per lane, each lane adding its terms in j order
@@ -1355,9 +1355,11 @@ __global__ __launch_bounds__(kBlock) void k_force_split(const WorkItem* __restri
 hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
-                              uint32_t n_all)
+                              uint32_t n_all, uint32_t n_cu)
 {
     if (n_items == 0) return hipSuccess;
+    // several blocks on a CU, all of them resident (6 of 12 sinks, 5 of 18)
+    const bool turns = grid > n_cu && grid <= (sinks == 18 ? 5u : 6u) * n_cu;
 #define EXACT_LAUNCH(KERNEL, BLOCK, ...)                                                                        \
     hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(BLOCK), 0, st, items, n_items, x, y, z, m_ex, mass_odd, ctl, need, \
                        __VA_ARGS__)
@@ -1366,10 +1368,10 @@ hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* it
         hipLaunchKernelGGL(k_force_exact_lane, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m_ex, ctl,
                            need, part, n_all);
         break;
-    case 4: EXACT_LAUNCH(k_force_exact<4>, exact_block(4), part, n_all); break;
-    case 8: EXACT_LAUNCH(k_force_exact<8>, exact_block(8), part, n_all); break;
-    case 12: EXACT_LAUNCH(k_force_exact<12>, exact_block(12), part, n_all); break;
-    case 18: EXACT_LAUNCH(k_force_exact<18>, exact_block(18), part, n_all); break;
+    case 4: EXACT_LAUNCH(k_force_exact<4>, exact_block(4), part, n_all, turns); break;
+    case 8: EXACT_LAUNCH(k_force_exact<8>, exact_block(8), part, n_all, turns); break;
+    case 12: EXACT_LAUNCH(k_force_exact<12>, exact_block(12), part, n_all, turns); break;
+    case 18: EXACT_LAUNCH(k_force_exact<18>, exact_block(18), part, n_all, turns); break;
     default: return hipErrorInvalidValue;
     }
 #undef EXACT_LAUNCH
