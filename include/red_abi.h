@@ -109,10 +109,13 @@ typedef struct rd_gas_grid {
     const double* vtheta;     /* n_rad * n_sec */
 } rd_gas_grid;
 
-/* Launch shapes of the pair kernels (chosen by rd_autotune or by hand). */
+/* Launch shapes of the pair kernels (chosen by rd_autotune or by hand).
+ * sinks_per_lane and chunk are upper limits: a disk whose one-sided items would
+ * be too few for the GPU takes one sink per lane and smaller chunks. */
 typedef struct rd_tuning {
-    uint32_t sinks_per_lane;   /* mixed kernel: 1, 2 or 4 sinks per lane          */
-    uint32_t chunk;            /* mixed kernel: sources per work item (mult. of 256) */
+    uint32_t sinks_per_lane;   /* mixed kernel: at most 1, 2 or 4 sinks per lane  */
+    uint32_t chunk;            /* mixed kernel: sources per work item at most     */
+                               /* (multiple of 256)                               */
     uint32_t blocks_per_cu;    /* persistent grid size = blocks_per_cu * CUs      */
     uint32_t use_graph;        /* capture one RK attempt in a hipGraph            */
     uint32_t pair_mode;        /* mixed kernel, SI x SI pairs: RD_PAIRS_*         */

@@ -17,7 +17,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -160,6 +162,7 @@ struct rd_disk {
     uint32_t n_items_sym = 0, grid_sym = 0, sym_R = 1;
     bool sym_self = false;           // diagonal tiles with reactions
     bool sym_split = false;          // items_sym cut finer (k_force_split)
+    uint32_t one_S = 1;              // mixed precision: sinks per lane of the widest one-sided item
     // collision grid: bucket heads, per-body list links and cells, largest radius
     uint32_t* coll_head = nullptr;
     uint32_t* coll_next = nullptr;
@@ -513,7 +516,8 @@ void class_bounds(const HostDisk& h, int cls, uint32_t b[4])
     else { b[0] = mas; b[1] = mas + ni; b[2] = 0; b[3] = mas; }
 }
 
-int build_lists(rd_disk* d)
+// shapes, if given: the bytes of the lists and launch shapes (rd_autotune compares them).
+int build_lists(rd_disk* d, std::string* shapes = nullptr)
 {
     d->lists_valid = false;   // until this build completes: a failure part-way forces a rebuild
     fill_info(d);
@@ -683,6 +687,10 @@ int build_lists(rd_disk* d)
     }
     // largest items first; ties keep the disk order
     std::stable_sort(sym_items.begin(), sym_items.end(), [](auto& a, auto& b) { return a.first > b.first; });
+    d->one_S = 1;
+    if (d->precision == RD_PREC_MIXED)
+        for (auto& w : items)
+            if (!(w.flags & kItemNarrow)) d->one_S = S;
     d->sym_self = false;
     for (auto& q : sym_items) d->sym_self |= (q.second.flags & kItemSelf) != 0;
     std::vector<WorkItem> symv;
@@ -738,6 +746,12 @@ int build_lists(rd_disk* d)
     const uint32_t grid_cap = d->precision == RD_PREC_FP64 && d->exact_sinks != 1 ? 8u * (uint32_t)d->n_cu : maxgrid;
     d->grid_force = std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_force, grid_cap));
     d->grid_sym = d->sym_split ? d->n_items_sym : std::max<uint32_t>(1, std::min<uint32_t>(d->n_items_sym, maxgrid));
+    if (shapes) {
+        const uint32_t shape[] = {d->n_items_force, d->grid_force, d->n_items_sym, d->grid_sym, d->sym_R, d->one_S};
+        shapes->assign((const char*)shape, sizeof(shape));
+        shapes->append((const char*)items.data(), items.size() * sizeof(WorkItem));
+        shapes->append((const char*)symv.data(), symv.size() * sizeof(WorkItem));
+    }
     const size_t need = max_chunks * 3 * (size_t)d->n_all;
     if (need > d->part_len) {
         dev_free(d->part);
@@ -809,7 +823,7 @@ hipError_t enqueue_force(rd_disk* d, const double* fx, const double* fy, const d
     // mixed precision: FP32 slot totals, in float units of the same buffer
     float* part32 = reinterpret_cast<float*>(d->part);
     const MixedLists l{d->items_sym,   d->n_items_sym,   d->grid_sym,   d->sym_R, d->sym_self, d->sym_split,
-                       d->items_force, d->n_items_force, d->grid_force, (int)d->tuning.sinks_per_lane};
+                       d->items_force, d->n_items_force, d->grid_force, (int)d->one_S};
     return launch_force_mixed(d->stream, l, fx, fy, fz, d->m32, d->ctl, need, part32, d->n_all);
 }
 
@@ -1467,9 +1481,14 @@ int rd_autotune(rd_disk* d, rd_tuning* best)
         one_sided_rest |= h.n_massive() > h.n_si() || h.n > h.n_massive();
         small_disks |= (h.n_si() + kSymBlockBodies - 1) / kSymBlockBodies < 2 * kSymChunks && h.n_si() > kSymBlockBodies;
     }
+    // small disks cut chunks and sinks themselves (kOneSidedItems): many settings are
+    // one and the same launch, timed once
+    std::set<size_t> timed;
     auto trial = [&](const rd_tuning& t) -> int {
         d->tuning = t;
-        if (int rc = build_lists(d)) { d->tuning = keep; build_lists(d); return rc; }
+        std::string shapes;
+        if (int rc = build_lists(d, &shapes)) { d->tuning = keep; build_lists(d); return rc; }
+        if (!timed.insert(std::hash<std::string>{}(shapes)).second) return RD_OK;
         double ms = 0.0;
         if (int rc = time_force_stage(d, 3, &ms)) { d->tuning = keep; build_lists(d); return rc; }
         if (ms < best_ms) { best_ms = ms; win = t; }
