@@ -153,7 +153,7 @@ __device__ __forceinline__ void row_add8(double& sum, double v)
 // word (one subtract, one compare); the masses' when they are set
 // (k_set_sources): *mass_odd is nonzero if some source is outside, and every
 // pair then takes the branch of the rare ones (span 0: no r2 is in range), which
-// looks at its own mass (16385 bodies, one mass outside: 519 us, 470 without, 851
+// looks at its own mass (16385 bodies, one mass outside: 530 us, 470 without, 855
 // with the library's for every pair).  A span for each source would cost every
 // launch: registers where it is a lane's, 3% at 5000 bodies as a scalar.  The
 // kernel with one sink per lane looks at its tiles' masses as it loads them.
@@ -422,11 +422,11 @@ __device__ __forceinline__ void force_exact_body(const WorkItem* __restrict__ it
                         out |= !exact_r2_in_range(r2[q], r2_span);
                     }
                     exact_scale_fast<kT>(r2, m, sc);
-                    if (out) {
-                        const uint32_t own_span = exact_mass_odd(m) ? 0u : kExactR2Span;
+                    if (__builtin_expect(out, 0)) {
+                        const bool odd = r2_span == 0u && exact_mass_odd(m);
 #pragma unroll
                         for (uint32_t q = 0; q < kT; ++q) {
-                            if (exact_r2_in_range(r2[q], own_span)) continue;
+                            if (!odd && exact_r2_in_range(r2[q], kExactR2Span)) continue;
                             if (exact_skip(m, j == w.sink_lo + g0 + kGroups * q))
                                 sc[q] = dx[q] = dy[q] = dz[q] = 0.0;
                             else
