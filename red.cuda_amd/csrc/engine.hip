@@ -852,7 +852,7 @@ ExactLists exact_lists(const rd_disk* d)
 // do what follows it.  One gas-free disk's RKF7(8) or fixed-step RK4 runs each stage
 // so (launch_force_exact_stage): the same operations in the same order as pair
 // pass + stage kernel, one launch per stage instead of two (RKF7(8), 1501
-// bodies: 267 -> 253 us a step; 701 bodies: 163 -> 134)
+// bodies: 267 -> 248 us a step; 701 bodies: 163 -> 134)
 bool fused_stages(const rd_integrator* it)
 {
     const rd_disk* d = it->d;

@@ -74,12 +74,12 @@ __host__ __device__ constexpr double rk4_c(int r) { return (r == 1 || r == 2) ? 
 // Pair kernels
 // ---------------------------------------------------------------------------
 // Reference formula (pp_disk.cu:374-416): sources j ascending, skip i == j
-// and inactive j (m_ex < 0), a += (m_j / (d * d^2)) * d_vec, every operation
+// and inactive j (m_ex = -0), a += (m_j / (d * d^2)) * d_vec, every operation
 // rounded separately (the reference builds -fmad=false).
 //
 // The sum per (sink, component) is a chain of FP64 adds in j order, so it
-// cannot be split; the pair terms feeding it can.  A block takes kS sinks (4, 8
-// or 18, build_lists).  Its term waves compute, for each tile of kTile sources, the
+// cannot be split; the pair terms feeding it can.  A block takes kS sinks (4, 8,
+// 12 or 18, build_lists).  Its term waves compute, for each tile of kTile sources, the
 // kS x kTile terms (m_j / (d * d^2)) * dx (sqrt and divide are the costly part)
 // into LDS; the summing waves add a tile's terms in j order to their running
 // sums.  The term buffer is doubled: tile t - 1 is added while tile t is
@@ -98,7 +98,7 @@ __host__ __device__ constexpr double rk4_c(int r) { return (r == 1 || r == 2) ? 
 //     16 consecutive terms at once; each is broadcast to the row and added by
 //     v_fmac_f64 with row_newbcast (term * 1 + sum: the add's rounding), every
 //     lane of the row holding the same sum.  One LDS read per 16 terms.
-//   18 sinks (throughput-bound: a broadcast add per term would cost more
+//   12 or 18 sinks (throughput-bound: a broadcast add per term would cost more
 //     than the term's share of a wave): one summing wave, a lane per (sink,
 //     component), reading two terms at a time.  Three term waves: a block of
 //     four waves puts one on each SIMD, and since consecutive blocks of a CU
@@ -110,7 +110,7 @@ __host__ __device__ constexpr double rk4_c(int r) { return (r == 1 || r == 2) ? 
 // A term thread takes one source of the tile against kT sinks.  Its source
 // comes from memory straight into registers, kAhead tiles early (every wave reads
 // the same few KB: L1 hits), so no source passes through LDS, whose traffic the
-// 18-sink shape would run into next.  The kT terms are
+// larger shapes would run into next.  The kT terms are
 // computed phase by phase (their chains of dependent FP64 operations, ~450
 // cycles each, interleave) with a single branch at the end for the rare pair
 // outside the short sequences' range.
