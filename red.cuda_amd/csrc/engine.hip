@@ -172,6 +172,7 @@ struct rd_disk {
     WorkItem* items_feat = nullptr;
     uint32_t n_items_feat = 0;
     uint32_t exact_sinks = 18;     // FP64 pair kernel: sinks per item, 1 for one per lane (see build_lists)
+    bool exact_few = false;        // ... its items for few sources (kExactFewBodies)
     bool lists_valid = false;
     double pairs_per_eval = 0.0;
 
@@ -544,8 +545,14 @@ int build_lists(rd_disk* d, std::string* shapes = nullptr)
                 }
             return n;
         };
+        uint32_t n_max = 0;
+        for (auto& h : d->hd) n_max = std::max(n_max, h.n);
+        d->exact_few = false;
         if (n_groups((uint32_t)kBlock) >= 4 * (size_t)d->n_cu) {
             d->exact_sinks = 1;
+        } else if (d->n_disk > 1 && n_max <= kExactFewBodies) {
+            d->exact_few = true;
+            d->exact_sinks = n_groups(16) < (size_t)d->n_cu ? 4 : 16;
         } else {
             size_t best = ~(size_t)0;   // sinks of the fullest CU
             for (uint32_t q : kExactSinks) {
@@ -558,6 +565,7 @@ int build_lists(rd_disk* d, std::string* shapes = nullptr)
                     d->exact_sinks = q;
                 }
             }
+            d->exact_few = d->exact_sinks == 4 && n_max <= kExactFewAlone;
         }
     }
     const uint32_t exact_group = d->exact_sinks == 1 ? (uint32_t)kBlock : d->exact_sinks;
@@ -820,8 +828,9 @@ StageArgs make_args(rd_disk* d, int r, int adaptive, int err_all)
 hipError_t enqueue_force(rd_disk* d, const double* fx, const double* fy, const double* fz, uint32_t need)
 {
     if (d->precision == RD_PREC_FP64)
-        return launch_force_exact(d->stream, d->exact_sinks, d->items_force, d->n_items_force, d->grid_force, fx, fy,
-                                  fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all, (uint32_t)d->n_cu);
+        return launch_force_exact(d->stream, d->exact_sinks, d->exact_few, d->items_force, d->n_items_force,
+                                  d->grid_force, fx, fy, fz, d->m_ex, d->mass_odd, d->ctl, need, d->part, d->n_all,
+                                  (uint32_t)d->n_cu);
     // mixed precision: FP32 slot totals, in float units of the same buffer
     float* part32 = reinterpret_cast<float*>(d->part);
     const MixedLists l{d->items_sym,   d->n_items_sym,   d->grid_sym,   d->sym_R, d->sym_self, d->sym_split,

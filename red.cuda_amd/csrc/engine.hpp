@@ -33,6 +33,12 @@ constexpr int kTile = 256;           // sources staged in LDS per tile
 // blocks a CU on (16384 bodies: 470 us, 545 with 12), and past six blocks of 12,
 // all that a CU holds at once (20000 bodies: 725 us, 799 with 12).
 constexpr uint32_t kExactSinks[] = {4, 8, 12, 18};
+// A batch whose largest disk has at most this many bodies takes items for few sources
+// (k_force_exact_few), of 16 sinks, or of 4 where those would leave CUs idle (300 disks
+// of 201 bodies: 34.2 us, 36.1 with items of 18; 900 of 251: 138 and 129); so does a
+// single disk's launch of 4-sink items, up to one 64-source tile (31 bodies 2.9 us and
+// 3.1, 101 bodies 3.6 and 3.4).
+constexpr uint32_t kExactFewBodies = 224, kExactFewAlone = 64;
 // high words of the r^2 the FP64 kernels' short root and division sequences
 // take: from 2^-200, up to 2^200
 constexpr uint32_t kExactR2Lo = (1023u - 200u) << 20;
@@ -179,9 +185,10 @@ struct BodyArrays {
 };
 
 // Launchers (kernels.hip).
-// sinks: sinks per item, 4, 8, 12 or 18 (term-parallel), or 1 for one sink per lane
-// (256-sink items)
-hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
+// sinks: sinks per item, 4, 8, 12 or 18 (term-parallel; 4 or 16 with few), or 1 for
+// one sink per lane (256-sink items)
+hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, bool few, const WorkItem* items, uint32_t n_items,
+                              uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
                               uint32_t n_all, uint32_t n_cu);

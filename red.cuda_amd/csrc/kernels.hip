@@ -475,6 +475,106 @@ void k_force_exact(const WorkItem* __restrict__ items, uint32_t n_items,
     force_exact_body<kS>(items, n_items, x, y, z, m_ex, mass_odd, ctl, need, StoreSum{part, n_all}, turns);
 }
 
+// The same sums for few sources (kExactFewBodies): a few tiles, too short for the shapes
+// above, whose time is then mostly the fetch of their unrolled code and the way to
+// the first term.  Sources pass through LDS; four term waves, a thread one
+// sink and kT sources of a tile, so a wave without a sink does nothing; one
+// summing wave, a lane per (sink, component), adds a tile's terms one by one.
+// 16 sinks and 32-source tiles, or 4 and 64.  600 disks of 20 bodies: 4.3 us (12-sink
+// items above: 6.0); 100 of 101 bodies: 6.2 (8.1); 21 of 51: 3.1 (4.0).
+template <uint32_t kS>
+__global__ __launch_bounds__(kBlock + 64) void k_force_exact_few(const WorkItem* __restrict__ items, uint32_t n_items,
+                                                                 const double* __restrict__ x,
+                                                                 const double* __restrict__ y,
+                                                                 const double* __restrict__ z,
+                                                                 const double* __restrict__ m_ex,
+                                                                 const uint32_t* __restrict__ mass_odd,
+                                                                 const DiskCtl* __restrict__ ctl, uint32_t need,
+                                                                 double* __restrict__ part, uint32_t n_all)
+{
+    constexpr uint32_t kLanes = kBlock / kS;                // term threads sharing one sink
+    constexpr uint32_t kTile = kS >= 16 ? 32u : kLanes;
+    constexpr uint32_t kT = kTile / kLanes;                 // terms per thread per tile
+    static_assert(kS * kTile == kT * kBlock && kT >= 1 && 3 * kS <= 64 && kTile <= kBlock, "tile shape");
+    __shared__ double4 src[2][kTile];
+    __shared__ double term[2][3][kS][kTile + 1];   // +1: summing lanes read with an odd stride
+    const uint32_t tid = threadIdx.x;
+    const bool termer = tid < (uint32_t)kBlock;     // waves 0-3
+    const uint32_t g = tid / kLanes;                // term threads: their sink,
+    const uint32_t k0 = tid % kLanes;               //               their sources k0 + kLanes q, q < kT
+    const uint32_t sl = tid - (uint32_t)kBlock;     // wave 4: summing lane (sl < 3 kS),
+    const uint32_t sc_c = sl / kS % 3u;             //         its component
+    const uint32_t sc_g = sl % kS;                  //         and sink
+    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
+        const WorkItem w = items[it];
+        if (!(ctl[w.disk].flags & need)) continue;
+        const uint32_t i = w.sink_lo + g;
+        const bool valid = termer && i < w.sink_hi;
+        const double xi = valid ? x[i] : 0.0, yi = valid ? y[i] : 0.0, zi = valid ? z[i] : 0.0;
+        const uint32_t si = w.sink_lo + sc_g;       // sink of a summing lane
+        const bool summer = !termer && sl < 3 * kS && si < w.sink_hi;
+        const uint32_t n_tiles = (w.src_hi - w.src_lo + kTile - 1) / kTile;
+        const uint32_t r2_span = *mass_odd ? 0u : kExactR2Span;
+        auto load_src = [&](uint32_t j) {
+            return j < w.src_hi ? make_double4(x[j], y[j], z[j], m_ex[j]) : make_double4(0.0, 0.0, 0.0, -0.0);
+        };
+        double acc = 0.0;
+        // tile 0 into LDS, tile 1 into registers; the loop stages tile t + 1 and
+        // loads tile t + 2 while tile t's terms are computed
+        double4 nxt = make_double4(0.0, 0.0, 0.0, -0.0);
+        if (tid < kTile) {
+            src[0][tid] = load_src(w.src_lo + tid);
+            nxt = load_src(w.src_lo + kTile + tid);
+        }
+        __syncthreads();
+        for (uint32_t t = 0; t <= n_tiles; ++t) {
+            const uint32_t b = t & 1u;
+            if (termer) {
+                if (t < n_tiles) {
+                    if (valid) {
+#pragma unroll
+                        for (uint32_t q = 0; q < kT; ++q) {
+                            const uint32_t k = k0 + kLanes * q;
+                            const double4 sj = src[b][k];
+                            double dx = sj.x - xi, dy = sj.y - yi, dz = sj.z - zi;
+                            const double r2 = SQR(dx) + SQR(dy) + SQR(dz);
+                            const bool self = w.src_lo + t * kTile + k == i;
+                            double sc;
+                            if constexpr (kS >= 16) {
+                                double one[1];
+                                exact_scale_fast<1>({r2}, sj.w, one);
+                                sc = one[0];
+                                if (!exact_r2_in_range(r2, r2_span)) {
+                                    const bool odd = r2_span == 0u && exact_mass_odd(sj.w);
+                                    if (exact_skip(sj.w, self)) sc = dx = dy = dz = 0.0;
+                                    else if (odd || !exact_r2_in_range(r2, kExactR2Span)) sc = exact_scale_any(r2, sj.w);
+                                }
+                            } else {
+                                // latency-bound: the branch would cost more than the shorter sequence saves
+                                sc = exact_scale_any(r2, sj.w);
+                                if (exact_skip(sj.w, self)) sc = dx = dy = dz = 0.0;
+                            }
+                            term[b][0][g][k] = sc * dx;
+                            term[b][1][g][k] = sc * dy;
+                            term[b][2][g][k] = sc * dz;
+                        }
+                    }
+                    if (tid < kTile) {
+                        src[b ^ 1u][tid] = nxt;
+                        nxt = load_src(w.src_lo + (t + 2) * kTile + tid);
+                    }
+                }
+            } else if (t > 0 && summer) {
+                const double* tr = &term[b ^ 1u][sc_c][sc_g][0];
+#pragma unroll
+                for (uint32_t k = 0; k < kTile; ++k) acc += tr[k];
+            }
+            __syncthreads();
+        }
+        if (summer) part[(size_t)(w.slot * 3 + sc_c) * n_all + si] = acc;
+    }
+}
+
 // The same sum with one sink per lane, each lane adding its terms in j order
 // as it computes them (the reference kernel's structure): cheaper per pair,
 // but only one lane per sink, so it is used when 256-sink work items alone
@@ -1352,7 +1452,8 @@ __global__ __launch_bounds__(kBlock) void k_force_split(const WorkItem* __restri
     }
 }
 
-hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* items, uint32_t n_items, uint32_t grid,
+hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, bool few, const WorkItem* items, uint32_t n_items,
+                              uint32_t grid,
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
                               uint32_t n_all, uint32_t n_cu)
@@ -1363,6 +1464,12 @@ hipError_t launch_force_exact(hipStream_t st, uint32_t sinks, const WorkItem* it
 #define EXACT_LAUNCH(KERNEL, BLOCK, ...)                                                                        \
     hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(BLOCK), 0, st, items, n_items, x, y, z, m_ex, mass_odd, ctl, need, \
                        __VA_ARGS__)
+    if (few) {
+        if (sinks == 4) EXACT_LAUNCH(k_force_exact_few<4>, kBlock + 64, part, n_all);
+        else if (sinks == 16) EXACT_LAUNCH(k_force_exact_few<16>, kBlock + 64, part, n_all);
+        else return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
     switch (sinks) {
     case 1:
         hipLaunchKernelGGL(k_force_exact_lane, dim3(grid), dim3(kBlock), 0, st, items, n_items, x, y, z, m_ex, ctl,

@@ -13,16 +13,17 @@ from test_gpu_device_dydx import DevArray
 pytestmark = pytest.mark.gpu
 
 
-def test_blocks_of_several_items():
-    """600 disks of 65 bodies: 2400 items of 18 sinks (8 blocks a CU: 2048 on 256
-    CUs), fewer than the 1024 groups of 256 that take one sink per lane.  One
-    fixed RK4 step advances all of them, so every item of every launch works."""
-    parts = [R.make_disk(64, 1200 + k) for k in range(600)]
+# 7500 items of 18 sinks and 3000 of 16 (8 blocks a CU: 2048 on 256 CUs), fewer than
+# the 1024 groups of 256 that take one sink per lane
+@pytest.mark.parametrize("n_disk,n", [(500, 257), (600, 65)])
+def test_blocks_of_several_items(n_disk, n):
+    """One fixed RK4 step advances all disks, so every item of every launch works."""
+    parts = [R.make_disk(n - 1, 1200 + k) for k in range(n_disk)]
     d = R.Disk(*[np.concatenate([q[i] for q in parts]) for i in range(4)], np.stack([q[4] for q in parts]),
                batch=True)
     h = 0.1 * R.K_GAUSS
     R.Integrator(d, R.RD_RK4, h, adaptive=False).steps(1)
-    for k in list(range(0, 600, 37)) + [511, 512, 513, 598, 599]:
+    for k in list(range(0, n_disk, 37)) + [n_disk - 2, n_disk - 1]:
         o = O.ODisk(*parts[k])
         O.OInteg(o, 2, h, adaptive=False).step()
         _, rr, vv, _, _ = d.state(k)
