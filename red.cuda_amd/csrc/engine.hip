@@ -856,17 +856,20 @@ ExactLists exact_lists(const rd_disk* d)
     return {d->items_force, d->n_items_force, d->grid_force, d->exact_sinks, d->m_ex, d->mass_odd};
 }
 
-// FP64 items of 4 or 8 sinks are at most one block per CU: launches, not pairs,
-// set the time, and the summing lanes, which hold every body's complete sum, can
-// do what follows it.  One gas-free disk's RKF7(8) or fixed-step RK4 runs each stage
-// so (launch_force_exact_stage): the same operations in the same order as pair
-// pass + stage kernel, one launch per stage instead of two (RKF7(8), 1501
-// bodies: 267 -> 248 us a step; 701 bodies: 163 -> 134)
+// With one block of an FP64 item per CU, or two of 12 sinks, the summing lanes, which
+// hold every body's complete sum, can do what follows it.  One gas-free disk's
+// RKF7(8) or fixed-step RK4 runs each stage so (launch_force_exact_stage): the same
+// operations in the same order as pair pass + stage kernel, one launch per stage
+// instead of two (RKF7(8), 701 bodies: 163 -> 134 us a step, 1501 267 -> 248, 2500
+// 519 -> 483; RK4, 2500 bodies: 159 -> 144).  With more blocks on a CU the
+// registers of the rows would cost it blocks.
 bool fused_stages(const rd_integrator* it)
 {
     const rd_disk* d = it->d;
-    return d->precision == RD_PREC_FP64 && (d->exact_sinks == 4 || d->exact_sinks == 8) && d->n_disk == 1 &&
-           d->gas.on == kGasNone && (it->method == RD_RKF78 || (it->method == RD_RK4 && !it->adaptive));
+    const size_t most = d->exact_sinks == 12 ? 2 : (d->exact_sinks == 1 ? 0 : 1);   // blocks a CU
+    const bool items = d->n_items_force <= most * (size_t)d->n_cu;
+    return d->precision == RD_PREC_FP64 && items && d->n_disk == 1 && d->gas.on == kGasNone &&
+           (it->method == RD_RKF78 || (it->method == RD_RK4 && !it->adaptive));
 }
 
 // The operator too, and with gas on 4-sink items (drag takes more registers than the
@@ -883,7 +886,7 @@ size_t error_words(const rd_integrator* it)
 {
     const rd_disk* d = it->d;
     if (d->n_all == 0) return 0;
-    if (fused_stages(it)) return (size_t)d->grid_force * (3 * d->exact_sinks / 4);
+    if (fused_stages(it)) return (size_t)d->grid_force * (d->exact_sinks >= 12 ? 1 : 3 * d->exact_sinks / 4);
     return 3 * (((size_t)d->n_all + kBodyBlock - 1) / kBodyBlock);
 }
 

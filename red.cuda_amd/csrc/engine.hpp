@@ -192,11 +192,11 @@ hipError_t launch_force_exact(hipStream_t s, uint32_t sinks, bool few, const Wor
                               const double* x, const double* y, const double* z, const double* m_ex,
                               const uint32_t* mass_odd, const DiskCtl* ctl, uint32_t need, double* part,
                               uint32_t n_all, uint32_t n_cu);
-// The FP64 pair pass on 4- or 8-sink items with what follows the sums done by the
-// kernel's summing lanes (no stage kernel, no partial-sum slot): stage r of a single
-// gas-free disk's RKF7(8) (method 4, 0-12; on 8-sink items not the wide stages) or
-// fixed-step RK4 (0-3), or the operator on
-// disk a.info0 (launch_operator's work; with gas, 4-sink items only).
+// The FP64 pair pass with what follows the sums done by the kernel's summing lanes
+// (no stage kernel, no partial-sum slot): stage r of a single gas-free disk's RKF7(8)
+// (method 4, 0-12; on 8-sink items not the wide stages) or fixed-step RK4 (0-3), or
+// the operator on disk a.info0 (launch_operator's work; 4- and 8-sink items, with gas
+// 4-sink items only).
 struct ExactLists {
     const WorkItem* items;
     uint32_t n_items, grid, sinks;

@@ -2035,10 +2035,12 @@ struct Rk8Sum {
             e = s.rows.finish(a, q, s.h, kRa, [&](double* p) { return p + i; });
             if (!(a.err_all || i - a.info0.off < a.info0.err_hi)) e = 0.0;
         }
-        // one error slot per summing wave, 3 kS / 4 of them in a block
+        // one error slot per summing wave: 3 kS / 4 of them in a block, one on 12- and
+        // 18-sink items (any of the block's four waves)
         if constexpr (R == 12) {
             const uint32_t waves = blockDim.x / 64u - kRowSumTermWaves;
-            error_store_wave(a, owner, e, blockIdx.x * waves + threadIdx.x / 64u - kRowSumTermWaves);
+            error_store_wave(a, owner, e,
+                             waves == 0 ? blockIdx.x : blockIdx.x * waves + threadIdx.x / 64u - kRowSumTermWaves);
         }
     }
 };
@@ -2569,18 +2571,22 @@ hipError_t launch_force_exact_stage(hipStream_t st, const ExactLists& l, int met
                                     const StageArgs& a)
 {
     if (l.n_items == 0) return hipSuccess;
-    if (l.sinks != 4 && l.sinks != 8) return hipErrorInvalidValue;
+    if (l.sinks != 4 && l.sinks != 8 && l.sinks != 12 && l.sinks != 18) return hipErrorInvalidValue;
     if (a.gas.on != kGasNone) return hipErrorInvalidValue;
 #define EXACT_STAGE(M, R)                                                              \
     case R:                                                                            \
         if (l.sinks == 4) EXACT_FUSED((k_force_exact_##M<4, R>), 4, a);                \
-        else EXACT_FUSED((k_force_exact_##M<8, R>), 8, a);                             \
+        else if (l.sinks == 8) EXACT_FUSED((k_force_exact_##M<8, R>), 8, a);           \
+        else if (l.sinks == 12) EXACT_FUSED((k_force_exact_##M<12, R>), 12, a);        \
+        else EXACT_FUSED((k_force_exact_##M<18, R>), 18, a);                           \
         break;
-    // the stages of most k rows (exact_wide_stage): 4-sink items only
+    // the stages of most k rows (exact_wide_stage): not on 8-sink items
 #define EXACT_WIDE(R)                                                                  \
     case R:                                                                            \
-        if (l.sinks != 4) return hipErrorInvalidValue;                                 \
-        EXACT_FUSED((k_force_exact_rk8<4, R>), 4, a);                                  \
+        if (l.sinks == 8) return hipErrorInvalidValue;                                 \
+        if (l.sinks == 4) EXACT_FUSED((k_force_exact_rk8<4, R>), 4, a);                \
+        else if (l.sinks == 12) EXACT_FUSED((k_force_exact_rk8<12, R>), 12, a);        \
+        else EXACT_FUSED((k_force_exact_rk8<18, R>), 18, a);                           \
         break;
     if (method == 4) {
         switch (r) {
