@@ -533,7 +533,8 @@ int build_lists(rd_disk* d, std::string* shapes = nullptr)
     const uint32_t S = d->tuning.sinks_per_lane;
     const uint32_t C_max = std::max<uint32_t>(kTile, d->tuning.chunk / kTile * kTile);
     // FP64: one sink per lane when 256-sink items give >= 4 blocks per CU, else
-    // the term-parallel kernel on items of kExactSinks (same bits in every case)
+    // the term-parallel kernel on items of kExactSinks, or for few sources
+    // (kExactFewBodies); same bits in every case
     if (d->precision == RD_PREC_FP64) {
         auto n_groups = [&](uint32_t group) {
             size_t n = 0;

@@ -243,7 +243,7 @@ struct StoreSum {
     }
 };
 
-// Fin: what follows the sum.  The fused ones (single disk, 4- or 8-sink items) run
+// Fin: what follows the sum.  The fused ones (a single disk whose blocks fit) run
 // the stage for the body in the lane that holds its sum, the value the stage
 // kernel would read back from the slot: it reads only that body's state and k
 // rows and writes the other position buffer, which no pair term of this launch
